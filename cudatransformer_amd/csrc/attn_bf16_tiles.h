@@ -55,11 +55,11 @@ struct F16Fmt {
 // touch each bank once.
 template <int D>
 struct Tile {
-    static_assert(D == 32 || D == 64 || D == 128, "bf16 MFMA kernels support d in {32, 64, 128}");
+    static_assert(D == 32 || D == 64 || D == 128 || D == 256, "tile width");
     static constexpr int CH = D / 8;         // 16-byte chunks per row
     static constexpr int ROW_BYTES = 2 * D;  // bytes per row
     __device__ static constexpr int swz(int r) {
-        return D == 128 ? 4 * (r & 3) + ((r >> 2) & 3)
+        return D >= 128 ? 4 * (r & 3) + ((r >> 2) & 3)
              : D == 64  ? 4 * ((r >> 1) & 1) + ((r >> 2) & 3)
                         : (r >> 2) & 3;
     }

@@ -40,6 +40,16 @@ hipError_t launch_generic_bwd(int dtype, const void *q, const void *k, const voi
                               void *dk, void *dv, void *delta, const AttnShape &s,
                               hipStream_t stream);
 
+// ---- wide heads on MFMA (attn_wide.hip): 128 < d <= 256, d a multiple of 8, fp32 / bf16 / fp16,
+// 16-byte aligned tensors, from a shortest T on.  The backward runs its own preprocess into `delta` and needs no other
+// scratch; no atomics. ----
+bool wide_supported(int dtype, const AttnShape &s, bool backward);
+hipError_t launch_wide_fwd(int dtype, const void *q, const void *k, const void *v, void *o, float *lse,
+                           const AttnShape &s, hipStream_t stream);
+hipError_t launch_wide_bwd(int dtype, const void *q, const void *k, const void *v, const void *o, const void *dout,
+                           const float *lse, float *delta, void *dq, void *dk, void *dv, const AttnShape &s,
+                           hipStream_t stream);
+
 // ---- shared backward preprocess: delta[row] = sum_c dO[row][c] * O[row][c] ----
 hipError_t launch_bwd_preprocess(int dtype, const void *o, const void *dout, void *delta,
                                  const AttnShape &s, hipStream_t stream);

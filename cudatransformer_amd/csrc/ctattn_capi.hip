@@ -99,6 +99,10 @@ bool use_mfma_bwd(int dtype, int64_t d) {
 bool use_f64_mfma(int dtype, int64_t d) {
     return dtype == CTATTN_F64 && g_policy.load() != CTATTN_POLICY_GENERIC && ctattn::f64_mfma_supported(d);
 }
+// Head dims above 128 on MFMA (attn_wide.hip); the others there take the generic kernels.
+bool use_wide(int dtype, const ctattn::AttnShape &s, bool backward) {
+    return g_policy.load() != CTATTN_POLICY_GENERIC && ctattn::wide_supported(dtype, s, backward);
+}
 // The MFMA kernels move 16 bytes per load (float4 / double2 / direct-to-LDS dwordx4); row
 // strides are multiples of 16 bytes for d in {32, 64, 128}, so 16-byte-aligned base pointers
 // suffice.  Element-aligned views that are not (a tensor offset into its storage) take the
@@ -298,6 +302,7 @@ int ctattn_fwd(int dtype, const void *q, const void *k, const void *v, void *o, 
     const bool al = aligned16({q, k, v, o, lse});
     hipError_t e = use_mfma_fwd(dtype, d) && al ? ctattn::launch_mfma_fwd(dtype, q, k, v, o, static_cast<float *>(lse), s, st)
                    : use_f64_mfma(dtype, d) && al ? ctattn::launch_f64_fwd(q, k, v, o, lse, s, st)
+                   : use_wide(dtype, s, false) && al ? ctattn::launch_wide_fwd(dtype, q, k, v, o, static_cast<float *>(lse), s, st)
                                                   : ctattn::launch_generic_fwd(dtype, q, k, v, o, lse, s, st);
     return finish("ctattn_fwd", e, st);
 }
@@ -403,6 +408,9 @@ int ctattn_bwd(int dtype, const void *q, const void *k, const void *v, const voi
                                     deterministic_policy(), s, st);
     } else if (use_f64_mfma(dtype, d) && al) {
         e = ctattn::launch_f64_bwd(q, k, v, o, dout, lse, workspace, dq, dk, dv, s, st);
+    } else if (use_wide(dtype, s, true) && al) {
+        e = ctattn::launch_wide_bwd(dtype, q, k, v, o, dout, static_cast<const float *>(lse),
+                                    static_cast<float *>(workspace), dq, dk, dv, s, st);
     } else {
         e = ctattn::launch_generic_bwd(dtype, q, k, v, o, dout, lse, dq, dk, dv, workspace, s, st);
     }

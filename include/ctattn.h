@@ -29,10 +29,12 @@
  *     padded columns of the outputs are dropped): the backward keeps the copies in its
  *     workspace, the forward takes them from a stream-ordered memory pool the library owns
  *     per device (hipMallocFromPoolAsync / hipFreeAsync on `stream`).  d above 128 runs on
- *     the generic kernels.  Tensors must be element-aligned; the MFMA kernels at d in
- *     {32, 64, 128} also need 16-byte-aligned q, k, v, o, lse (and dout, dq, dk, dv,
- *     workspace in the backward); calls whose pointers are not take the generic kernels
- *     (same results, slower).
+ *     MFMA too in fp32, bf16 and fp16 where d is a multiple of 8 (T >= 8; fp32 T >= 32, its
+ *     backward T >= 96), with P and dS at fp32 precision, and on the generic kernels
+ *     otherwise.  Tensors must be element-aligned; the MFMA kernels at d in {32, 64, 128} and
+ *     above 128 also need 16-byte-aligned q, k, v, o, lse (and dout, dq, dk, dv, workspace in
+ *     the backward); calls whose pointers are not take the generic kernels (same results,
+ *     slower).
  */
 #ifndef CTATTN_H
 #define CTATTN_H

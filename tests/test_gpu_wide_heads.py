@@ -1,0 +1,95 @@
+"""Head dims above 128 (a multiple of 8) on the MFMA kernels of attn_wide.hip, against the generic
+kernels (POLICY_GENERIC) on the same inputs and forward state.
+
+Both sides compute in fp32 (the 16-bit MFMAs take P and dS as two 16-bit terms), so before the
+one rounding to storage they differ by fp32 summation error e < 1e-5 of the result's norm.  At
+fp32 that is the tolerance.  At 16 bits with unit roundoff u a value changes by one step (2u) only
+when e crosses a rounding boundary, a share e / 2u of the values: a norm of sqrt(e / 2u) 2u =
+sqrt(2 u e), 2e-4 for bf16 (u = 2^-9) and 1e-4 for fp16 (u = 2^-11); twice that is allowed.
+"""
+import pytest
+import torch
+
+import cudatransformer_amd as ct
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+TOL = {"f32": 1e-5, "bf16": 4e-4, "f16": 2e-4}
+
+
+def inputs(shape, name, seed, std=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [(std * torch.randn(shape, generator=g, device="cuda")).to(DT[name]) for _ in range(4)]
+
+
+def both(x, causal):
+    """(MFMA, generic) outputs, the backward of both from the generic forward's O and LSE."""
+    q, k, v, do = x
+    out = []
+    prev = ct.set_policy(ct.POLICY_GENERIC)
+    try:
+        og, lg = ct.flash_attn_fwd(q, k, v, causal)
+        gen = dict(zip(("o", "lse", "dq", "dk", "dv"), (og, lg, *ct.flash_attn_bwd(q, k, v, og, do, lg, causal))))
+    finally:
+        ct.set_policy(prev)
+    o, lse = ct.flash_attn_fwd(q, k, v, causal)
+    out = dict(zip(("o", "lse", "dq", "dk", "dv"), (o, lse, *ct.flash_attn_bwd(q, k, v, og, do, lg, causal))))
+    torch.cuda.synchronize()
+    return out, gen
+
+
+def check(got, want, name):
+    floor = want["dv"].double().norm()  # dQ and dK of a row with one key vanish
+    for key in want:
+        w, g = want[key].double(), got[key].double()
+        tol = 1e-5 if key == "lse" else TOL[name]
+        err = (g - w).norm() / torch.maximum(w.norm(), floor if key in ("dq", "dk") else w.norm())
+        assert err <= tol, (key, float(err))
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 8, 256), (2, 1, 31, 160), (1, 2, 33, 192), (1, 3, 64, 256), (1, 1, 97, 136),
+                                   (2, 2, 200, 200), (1, 3, 161, 160), (2, 1, 129, 192), (1, 2, 333, 256)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_matches_generic(name, causal, shape):
+    print(f"wide heads {name} causal={causal} {shape}", flush=True)
+    x = inputs(shape, name, seed=sum(shape))
+    got, want = both(x, causal)
+    check(got, want, name)
+    again, _ = both(x, causal)
+    assert all(torch.equal(got[k], again[k]) for k in got)  # no atomics
+
+
+@pytest.mark.parametrize("std", [2e-4, 30.0])
+def test_wide_f16_range(std):
+    """dS far below and above 1: the fp16 split keeps its precision over fp16's inputs."""
+    print(f"wide heads f16 gradient scale {std}", flush=True)
+    x = inputs((1, 2, 130, 256), "f16", seed=7)
+    x[3] = (x[3].float() * std).half()
+    got, want = both(x, True)
+    # dV and dK of a small dO are fp16 subnormals on both sides: compare what is above them.
+    for key in ("dq", "dk", "dv"):
+        w, g = want[key].double(), got[key].double()
+        err = ((g - w).abs() - 2.0 ** -24).clamp_min(0).norm() / w.norm()
+        assert err <= TOL["f16"], (key, float(err))
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_nonfinite_inputs(name, causal):
+    """An infinity and a NaN reach exactly the outputs they reach in the generic kernels: under a
+    causal mask not the rows before theirs, though those share a tile with it."""
+    print(f"wide heads non-finite {name} causal={causal}", flush=True)
+    x = inputs((1, 2, 110, 256), name, seed=3)
+    x[2][0, 0, 40, 5] = float("inf")
+    x[1][0, 1, 50, 7] = float("nan")
+    x[3][0, 0, 20, 9] = float("inf")
+    got, want = both(x, causal)
+    for key in want:
+        g, w = got[key].double(), want[key].double()
+        assert torch.equal(torch.isnan(g), torch.isnan(w)), key
+        assert torch.equal(torch.isinf(g), torch.isinf(w)), key
+        ok = torch.isfinite(w)
+        err = (g[ok] - w[ok]).norm() / w[ok].norm().clamp_min(1e-30)
+        assert err <= max(TOL[name], 1e-5), (key, float(err))
