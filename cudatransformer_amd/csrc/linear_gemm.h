@@ -58,16 +58,21 @@ struct LinGemm {
 LinGemm lin_plain(int dtype, bool a_kc, bool b_kc, int64_t M, int64_t N, int64_t K, const void *a, int64_t lda,
                   const void *b, int64_t ldb, void *c, int64_t ldc, const void *bias, bool beta);
 
-// Whether the product is in these kernels' domain: fp32 / bf16 / fp16; K a multiple of the
-// 64-byte K chunk (16 fp32 or 32 16-bit elements) and, for head-split operands, chunks and
-// 4- (fp32) or 8-element (16-bit) column groups inside one head; 16-byte aligned operands and
-// pitches; M/N-contiguous extents a multiple of 4 (fp32) or 8 (16-bit); 32-bit lane offsets.
+// Whether the product is in these kernels' domain: fp32 / bf16 / fp16 and
+//   * the direct-load kernels: K a multiple of the 64-byte K chunk (16 fp32 or 32 16-bit elements)
+//     and, for head-split operands, chunks and 4- (fp32) or 8-element (16-bit) column groups inside
+//     one head; 16-byte aligned operands and pitches; M/N-contiguous extents a multiple of 4 (fp32)
+//     or 8 (16-bit); 32-bit lane offsets; or else
+//   * the ragged kernels: any K, pitch, extent and element-aligned pointer, head-split views with d
+//     a multiple of 4 (fp32) or 8 (16-bit).
 bool lin_gemm_supported(const LinGemm &g);
 
 // Bytes of split-K partials the product's launch plan uses when workspace is allowed (0: the
 // plan does not split K across workgroups, or the shape is not supported).  Depends on the
-// dtype, layout, views and sizes only: the pointers may be null.
+// dtype, layout, views and sizes only: the pointers may be null.  _min: of the direct-load
+// kernels only (a ragged product runs unsplit on less).
 int64_t lin_gemm_workspace_bytes(const LinGemm &g);
+int64_t lin_gemm_workspace_min(const LinGemm &g);
 
 // Launches the product.  ws / ws_bytes: workspace for split-K partials (may be null / 0: the
 // plan then keeps K inside the workgroup).  Deterministic: fixed summation order, no atomics.

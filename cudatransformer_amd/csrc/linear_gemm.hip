@@ -81,6 +81,11 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+// Element-aligned vectors in global memory (one access each: the hardware takes any alignment).
+typedef u16x4 u16x4u __attribute__((aligned(2)));
+typedef floatx4 floatx4u __attribute__((aligned(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4u __attribute__((aligned(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -118,9 +123,9 @@ struct F32Fmt {
     static constexpr int KWE = 16;  // elements per 64-byte K chunk
     static constexpr bool WIDE = true;
     __device__ static float load(const char *p) { return *reinterpret_cast<const float *>(p); }
-    __device__ static floatx4 load4(const char *p) { return *reinterpret_cast<const floatx4 *>(p); }
+    __device__ static floatx4 load4(const char *p) { return *reinterpret_cast<const floatx4u *>(p); }
     __device__ static void store(char *p, float x) { *reinterpret_cast<float *>(p) = x; }
-    __device__ static void store4(char *p, floatx4 x) { *reinterpret_cast<floatx4 *>(p) = x; }
+    __device__ static void store4(char *p, floatx4 x) { *reinterpret_cast<floatx4u *>(p) = x; }
     // The value a store and a load back give (the storage type's rounding).
     __device__ static float round(float x) { return x; }
     // Sum of the 16-byte MFMA operand (4 fp32 values).
@@ -148,12 +153,12 @@ struct H16Fmt {
     __device__ static float load(const char *p) { return widen(*reinterpret_cast<const uint16_t *>(p)); }
     __device__ static float round(float x) { return widen(narrow(x)); }
     __device__ static floatx4 load4(const char *p) {
-        const u16x4 u = *reinterpret_cast<const u16x4 *>(p);
+        const u16x4 u = *reinterpret_cast<const u16x4u *>(p);
         return floatx4{widen(u[0]), widen(u[1]), widen(u[2]), widen(u[3])};
     }
     __device__ static void store(char *p, float x) { *reinterpret_cast<uint16_t *>(p) = narrow(x); }
     __device__ static void store4(char *p, floatx4 x) {
-        *reinterpret_cast<u16x4 *>(p) = u16x4{narrow(x[0]), narrow(x[1]), narrow(x[2]), narrow(x[3])};
+        *reinterpret_cast<u16x4u *>(p) = u16x4{narrow(x[0]), narrow(x[1]), narrow(x[2]), narrow(x[3])};
     }
     // Sum of the 16-byte MFMA operand (8 16-bit values).
     __device__ static float sum(floatx4 v) {
@@ -224,6 +229,11 @@ struct OpKC {
     static constexpr int NL = BYTES / 1024;  // load instructions per stage
     static_assert(BYTES % 1024 == 0, "a stage is whole 1 KiB load instructions");
     __host__ __device__ static constexpr int swz(int r) { return (r >> 2) & 3; }
+    // Row (K-contiguous) or k-row and logical 16-byte chunk that physical chunk P of a stage holds.
+    __device__ static void coord(int P, int &line, int &lc) {
+        line = P / CH;
+        lc = (P % CH) ^ swz(line);
+    }
     // Lane offset of load instruction i from the stage origin (row 0, chunk 0 of the tile);
     // rows at or past `rows` re-read row rows - 1.
     __device__ static uint32_t voff(int i, int lane, const DView &v, int r0, int rows) {
@@ -257,6 +267,10 @@ struct OpKC2 {
     static constexpr int NL = BYTES / 1024;
     static_assert(BYTES % 1024 == 0, "a stage is whole 1 KiB load instructions");
     __host__ __device__ static constexpr int swz(int r) { return (r >> 1) & 7; }
+    __device__ static void coord(int P, int &line, int &lc) {
+        line = P / CH;
+        lc = (P % CH) ^ swz(line);
+    }
     __device__ static uint32_t voff(int i, int lane, const DView &v, int r0, int rows) {
         const int P = 64 * i + lane;
         const int r = P / CH;
@@ -276,11 +290,11 @@ struct OpKC2 {
     __host__ __device__ static constexpr int idx(int t, int i) { return 32 * t + i; }
 };
 
-// M/N-contiguous fp32 operand: 16 k-rows x R columns per stage, LDS [k][R] (row pitch 4 R).
-template <int R>
+// M/N-contiguous fp32 operand: KR k-rows (16 or 32) x R columns per stage, LDS [k][R] (row pitch 4 R).
+template <int R, int KR = 16>
 struct OpMN32 {
     static constexpr int CHR = R / 4;  // 16-byte chunks per k-row
-    static constexpr int BYTES = R * 64;
+    static constexpr int BYTES = R * 4 * KR;
     static constexpr int NL = BYTES / 1024;
     static constexpr bool ODD = (R / 32) % 2 == 1;  // rows alternate bank halves
     static_assert(R % 32 == 0 && R <= 128, "tile width 32, 64, 96 or 128");
@@ -288,6 +302,10 @@ struct OpMN32 {
     // physical chunk c ^ (8 ((kk >> 2) & 1)) (!ODD).  Both maps are involutions.
     __host__ __device__ static constexpr int rowpos(int kk) { return ODD ? kk ^ ((kk >> 2) & 1) : kk; }
     __host__ __device__ static constexpr int chunk(int kk, int c) { return ODD ? c : c ^ (((kk >> 2) & 1) << 3); }
+    __device__ static void coord(int P, int &line, int &lc) {
+        line = rowpos(P / CHR);
+        lc = chunk(line, P % CHR);
+    }
     // Columns at or past `cols` (a multiple of 4) re-read the last valid chunk.
     __device__ static uint32_t voff(int i, int lane, const DView &v, int c0, int cols) {
         const int P = 64 * i + lane;
@@ -354,6 +372,10 @@ struct OpMN16 {
     __host__ __device__ static constexpr int gsw(int kr) {
         return SEGS == 4 ? (kr & 3) : SEGS == 2 ? ((kr >> 1) & 1) : 0;
     }
+    __device__ static void coord(int P, int &line, int &lc) {
+        line = P / (R / 8);
+        lc = (P % (R / 8)) ^ (gsw(line) << 2);
+    }
     // Columns at or past `cols` (a multiple of 8) re-read the last valid chunk.
     __device__ static uint32_t voff(int i, int lane, const DView &v, int c0, int cols) {
         const int P = 64 * i + lane;
@@ -417,8 +439,9 @@ struct Args {
     int32_t chunks;      // K chunks over all segments
     int32_t seg_chunks;  // K chunks per segment
     int32_t cps;         // chunks per split
+    int32_t K;           // per segment (ragged products)
     int32_t beta;
-    int32_t vec_out;  // C takes 4-column vector stores
+    int32_t vec_out;  // 4 columns of C are contiguous (vector stores): 2, and N is a multiple of 4: 1, not
     int32_t act_mode, act_kind;  // fused activation (LinGemm::act_mode), aux in C's view
     char *aux[kLinMaxBatch];
 };
@@ -458,6 +481,50 @@ __device__ __forceinline__ void wait_tail(int r) {
 // Wave-uniform base of segment `seg` (seg < 3): a select, not an indexed register array.
 __device__ __forceinline__ const char *pick(const char *const (&arr)[kLinMaxSeg], int seg) {
     return seg == 0 ? arr[0] : seg == 1 ? arr[1] : arr[2];
+}
+
+// Stores 4 columns gn .. gn + 3 of row gm (x: the products): bias, beta, the fused activation.
+template <typename F>
+__device__ __forceinline__ void store_cols4(const Args &p, char *cz, const char *bz, int z, int64_t off, int gn,
+                                            floatx4 x) {
+    char *dst = cz + off;
+    if (bz != nullptr) x += F::load4(bz + int64_t(gn) * F::EB);
+    if (p.beta) x += F::load4(dst);
+    if (p.act_mode == 1) {
+        floatx4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = act_fwd(p.act_kind, F::round(x[e]));
+        F::store4(p.aux[z] + off, y);
+    } else if (p.act_mode == 2) {
+        const floatx4 pre = F::load4(p.aux[z] + off);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = act_bwd_value(p.act_kind, pre[e], F::round(x[e]));
+    }
+    F::store4(dst, x);
+}
+// The same where N is not a multiple of 4 or a group crosses heads (vec_out 0), kept out of the
+// common path.  GROUPS: whole groups at once where vec_out is 1, from their element-aligned
+// addresses -- faster for the wide rows of the shared tiles (bf16 256 x 50257 x 256 forward 50 ->
+// 36 us, 2048 x 5461 x 2048 95 -> 79), slower for the 64-wide ones (990 x 5003 x 256 25 -> 28).
+template <typename F, bool GROUPS>
+__device__ __forceinline__ void store_cols_edge(const Args &p, const DView &view_c, char *cz, const char *bz, int z,
+                                                int gm, int gn, floatx4 x) {
+    if (GROUPS && p.vec_out == 1 && gn + 4 <= p.N) {
+        store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (gn + e >= p.N) break;
+        const int64_t off = rowoff(view_c, gm) + coloff(view_c, gn + e);
+        char *de = cz + off;
+        float y = x[e];
+        if (bz != nullptr) y += F::load(bz + int64_t(gn + e) * F::EB);
+        if (p.beta) y += F::load(de);
+        if (p.act_mode == 1) F::store(p.aux[z] + off, act_fwd(p.act_kind, F::round(y)));
+        else if (p.act_mode == 2) y = act_bwd_value(p.act_kind, F::load(p.aux[z] + off), F::round(y));
+        F::store(de, y);
+    }
 }
 
 // GEN: some operand or the output is a head-split view, or K has several segments, so every K
@@ -654,8 +721,8 @@ __global__ __launch_bounds__(NW * 64) void lin_kernel(Args p) {
         for (int w = 1; w < NW; ++w) x += ld4(red + uint32_t(((w * BM + m) * BN + n) * 4));
         if (p.splits > 1) {
             float *dst = p.ws + ((int64_t(z) * p.splits + split) * p.M + gm) * p.N + gn;
-            if (p.N % 4 == 0) {
-                *reinterpret_cast<floatx4 *>(dst) = x;
+            if (gn + 4 <= p.N) {
+                *reinterpret_cast<floatx4u *>(dst) = x;
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -663,41 +730,16 @@ __global__ __launch_bounds__(NW * 64) void lin_kernel(Args p) {
             }
             continue;
         }
-        if (p.vec_out) {
-            const int64_t off = rowoff(view_c, gm) + coloff(view_c, gn);
-            char *dst = cz + off;
-            if (bz != nullptr) x += F::load4(bz + int64_t(gn) * F::EB);
-            if (p.beta) x += F::load4(dst);
-            if (p.act_mode == 1) {
-                floatx4 y;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] = act_fwd(p.act_kind, F::round(x[e]));
-                F::store4(p.aux[z] + off, y);
-            } else if (p.act_mode == 2) {
-                const floatx4 pre = F::load4(p.aux[z] + off);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = act_bwd_value(p.act_kind, pre[e], F::round(x[e]));
-            }
-            F::store4(dst, x);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (gn + e >= p.N) break;
-                const int64_t off = rowoff(view_c, gm) + coloff(view_c, gn + e);
-                char *de = cz + off;
-                float y = x[e];
-                if (bz != nullptr) y += F::load(bz + int64_t(gn + e) * F::EB);
-                if (p.beta) y += F::load(de);
-                if (p.act_mode == 1) F::store(p.aux[z] + off, act_fwd(p.act_kind, F::round(y)));
-                else if (p.act_mode == 2) y = act_bwd_value(p.act_kind, F::load(p.aux[z] + off), F::round(y));
-                F::store(de, y);
-            }
-        }
+        if (p.vec_out == 2)
+            store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
+        else
+            store_cols_edge<F, false>(p, view_c, cz, bz, z, gm, gn, x);
     }
 }
 
-// C_z(m, n) [+]= sum over splits s = 0, 1, ... of ws[z][s][m][n] (+ bias_z[n]), 4 columns per
-// thread when vec (N % 4 == 0, aligned C), else one.
+// C_z(m, n) [+]= sum over splits s = 0, 1, ... of ws[z][s][m][n] (+ bias_z[n]), with the fused
+// activation, 4 columns per
+// thread when vec (N % 4 == 0), else one.
 template <typename F>
 __global__ __launch_bounds__(256) void lin_splitk_reduce_kernel(Args p, int64_t items_per_batch, int vec) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -723,12 +765,30 @@ __global__ __launch_bounds__(256) void lin_splitk_reduce_kernel(Args p, int64_t 
         for (int s = 1; s < p.splits; ++s) x += *reinterpret_cast<const floatx4 *>(src + s * mn);
         if (bz != nullptr) x += F::load4(bz + int64_t(n) * F::EB);
         if (p.beta) x += F::load4(dst);
+        if (p.act_mode != 0) {
+            char *aux = p.aux[z] + (dst - p.c[z]);
+            if (p.act_mode == 1) {
+                floatx4 y;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] = act_fwd(p.act_kind, F::round(x[e]));
+                F::store4(aux, y);
+            } else {
+                const floatx4 pre = F::load4(aux);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = act_bwd_value(p.act_kind, pre[e], F::round(x[e]));
+            }
+        }
         F::store4(dst, x);
     } else {
         float x = src[0];
         for (int s = 1; s < p.splits; ++s) x += src[s * mn];
         if (bz != nullptr) x += F::load(bz + int64_t(n) * F::EB);
         if (p.beta) x += F::load(dst);
+        if (p.act_mode != 0) {
+            char *aux = p.aux[z] + (dst - p.c[z]);
+            if (p.act_mode == 1) F::store(aux, act_fwd(p.act_kind, F::round(x)));
+            else x = act_bwd_value(p.act_kind, F::load(aux), F::round(x));
+        }
         F::store(dst, x);
     }
 }
@@ -767,6 +827,150 @@ struct ShCfg {
     static_assert(LDS <= 160 * 1024, "LDS of one workgroup");
     static_assert(S >= 2 && (S - 1) * L < 64, "outstanding loads must fit vmcnt");
 };
+
+// One stage of the shared-tile kernels (NS steps of 8 fp32 or 16 16-bit k): wave (wm, wn)'s
+// 32 TM x 32 TN tile from the A operand at LDS address sa and B at sb.  sum_a: also the row sums
+// of A (bias gradient).
+template <typename F, bool A_KC, typename OA, typename OB, int TM, int TN, int NS>
+__device__ __forceinline__ void shared_stage(floatx16 (&acc)[TM][TN], float (&dsum)[TM], const typename OA::Lane &ra,
+                                             const typename OB::Lane &rb, uint32_t sa, uint32_t sb, int wm, int wn,
+                                             bool sum_a) {
+            if constexpr (!F::WIDE && A_KC) {
+                // 16-bit products with a K-contiguous A (forwards, dX): step s + 1's operands are
+                // read before step s's MFMAs, and the scheduling fence keeps the compiler from
+                // hoisting every step's reads to the top of the stage, so each step's MFMAs wait
+                // only for reads issued a whole step earlier.
+                floatx4 av[2][TM], bv[2][TN];
+    #pragma unroll
+                for (int tm = 0; tm < TM; ++tm) av[0][tm] = ra.read(sa, TM * wm + tm, 0);
+    #pragma unroll
+                for (int tn = 0; tn < TN; ++tn) bv[0][tn] = rb.read(sb, TN * wn + tn, 0);
+    #pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const int cur = s & 1;
+                    if (s + 1 < NS) {
+    #pragma unroll
+                        for (int tm = 0; tm < TM; ++tm) av[cur ^ 1][tm] = ra.read(sa, TM * wm + tm, s + 1);
+    #pragma unroll
+                        for (int tn = 0; tn < TN; ++tn) bv[cur ^ 1][tn] = rb.read(sb, TN * wn + tn, s + 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+                    for (int tm = 0; tm < TM; ++tm)
+    #pragma unroll
+                        for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = F::mfma(av[cur][tm], bv[cur][tn], acc[tm][tn]);
+                }
+            } else {
+                // fp32 and the 16-bit weight gradients: the compiler schedules the stage's reads
+                // (the same fence measured neutral in fp32 and 2-3.5 % slower on the transposed
+                // M/N-contiguous reads).
+    #pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    floatx4 av[TM], bv[TN];
+    #pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) av[tm] = ra.read(sa, TM * wm + tm, s);
+    #pragma unroll
+                    for (int tn = 0; tn < TN; ++tn) bv[tn] = rb.read(sb, TN * wn + tn, s);
+                    if (!A_KC && sum_a) {
+    #pragma unroll
+                        for (int tm = 0; tm < TM; ++tm) dsum[tm] += F::sum(av[tm]);
+                    }
+                    if constexpr (F::WIDE) {
+                        // fp32: the 16-byte operand is four k-steps of v_mfma_f32_32x32x2f32.
+    #pragma unroll
+                        for (int t = 0; t < 4; ++t)
+    #pragma unroll
+                            for (int tm = 0; tm < TM; ++tm)
+    #pragma unroll
+                                for (int tn = 0; tn < TN; ++tn)
+                                    acc[tm][tn] =
+                                        __builtin_amdgcn_mfma_f32_32x32x2f32(av[tm][t], bv[tn][t], acc[tm][tn], 0, 0, 0);
+                    } else {
+    #pragma unroll
+                        for (int tm = 0; tm < TM; ++tm)
+    #pragma unroll
+                            for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = F::mfma(av[tm], bv[tn], acc[tm][tn]);
+                    }
+                }
+            }
+}
+
+// The bias gradient and the stores of a shared-tile workgroup (`base`: its LDS, no longer read by
+// any wave once this one arrives at the first barrier): the K split's partials, or C with bias,
+// beta and the fused activation.
+template <typename F, bool A_KC, int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void shared_store(const floatx16 (&acc)[TM][TN], const float (&dsum)[TM], const Args &p,
+                                             const DView &view_c, uint32_t base, int m0, int n0, int z, int split,
+                                             int wm, int wn, int lane, bool want_db, bool sum_a) {
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN;
+    constexpr int EPI = 32 * TM * BN * 4;  // one wave row of the tile, fp32
+    const int h = lane >> 5, col = lane & 31;
+    const uint32_t ebuf = base;
+    if (!A_KC && want_db) {
+        // Lane (col, h) holds the sum over its k of A row 32 (TM wm + tm) + col: LDS [h][BM]
+        // past the store buffer; one thread per row adds the halves in order.
+        const uint32_t dbuf = base + uint32_t(EPI);
+        __syncthreads();  // the ring is no longer read
+        if (sum_a) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) st1(dbuf + uint32_t((h * BM + 32 * (TM * wm + tm) + col) * 4), dsum[tm]);
+        }
+        __syncthreads();
+        const int m = int(threadIdx.x);
+        if (m < BM && m0 + m < p.M) {
+            const float x = ld1(dbuf + uint32_t(m * 4)) + ld1(dbuf + uint32_t((BM + m) * 4));
+            if (p.splits > 1) {
+                p.ws[int64_t(p.nbatch) * p.splits * p.M * p.N + (int64_t(z) * p.splits + split) * p.M + m0 + m] = x;
+            } else {
+                char *dst = p.db[z] + int64_t(m0 + m) * F::EB;
+                F::store(dst, F::load(dst) + x);
+            }
+        }
+    }
+
+    // Stores, one wave row of the tile (32 TM rows x BN columns) at a time through LDS:
+    // register r of lane (col, h) holds row acc_row(r, h) of column col of each 32 x 32 tile.
+    char *const cz = p.c[z];
+    const char *const bz = p.bias[z];
+    constexpr int Q = 32 * TM * BN / 4;
+#pragma unroll 1
+    for (int pm = 0; pm < WM; ++pm) {
+        __syncthreads();  // the ring (or the previous pass) is no longer read
+        if (wm == pm) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        st1(ebuf + uint32_t(((32 * tm + acc_row(r, h)) * BN + 32 * (TN * wn + tn) + col) * 4),
+                            acc[tm][tn][r]);
+        }
+        __syncthreads();
+        for (int qi = int(threadIdx.x); qi < Q; qi += NW * 64) {
+            const int m = qi / (BN / 4);
+            const int n = (qi - m * (BN / 4)) * 4;
+            const int gm = m0 + pm * 32 * TM + m, gn = n0 + n;
+            if (gm >= p.M || gn >= p.N) continue;
+            floatx4 x = ld4(ebuf + uint32_t((m * BN + n) * 4));
+            if (p.splits > 1) {
+                float *dst = p.ws + ((int64_t(z) * p.splits + split) * p.M + gm) * p.N + gn;
+                if (gn + 4 <= p.N) {
+                    *reinterpret_cast<floatx4u *>(dst) = x;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (gn + e < p.N) dst[e] = x[e];
+                }
+                continue;
+            }
+            if (p.vec_out == 2)
+                store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
+            else
+                store_cols_edge<F, true>(p, view_c, cz, bz, z, gm, gn, x);
+        }
+    }
+}
 
 template <typename F, bool A_KC, bool B_KC, int WM, int WN, int TM, int TN, int S, int KS, bool GEN>
 __global__ __launch_bounds__(WM * WN * 64) void lin_shared_kernel(Args p) {
@@ -854,159 +1058,175 @@ __global__ __launch_bounds__(WM * WN * 64) void lin_shared_kernel(Args p) {
         if (j + S - 1 < nst) issue(islot, st0 + j + S - 1);
         const uint32_t sa = base + uint32_t(slot * C::STAGE);
         const uint32_t sb = sa + uint32_t(OA::BYTES);
-        if constexpr (!F::WIDE && A_KC) {
-            // 16-bit products with a K-contiguous A (forwards, dX): step s + 1's operands are
-            // read before step s's MFMAs, and the scheduling fence keeps the compiler from
-            // hoisting every step's reads to the top of the stage, so each step's MFMAs wait
-            // only for reads issued a whole step earlier.
-            floatx4 av[2][TM], bv[2][TN];
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) av[0][tm] = ra.read(sa, TM * wm + tm, 0);
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) bv[0][tn] = rb.read(sb, TN * wn + tn, 0);
-#pragma unroll
-            for (int s = 0; s < 2 * KS; ++s) {
-                const int cur = s & 1;
-                if (s + 1 < 2 * KS) {
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm) av[cur ^ 1][tm] = ra.read(sa, TM * wm + tm, s + 1);
-#pragma unroll
-                    for (int tn = 0; tn < TN; ++tn) bv[cur ^ 1][tn] = rb.read(sb, TN * wn + tn, s + 1);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = F::mfma(av[cur][tm], bv[cur][tn], acc[tm][tn]);
-            }
-        } else {
-            // fp32 and the 16-bit weight gradients: the compiler schedules the stage's reads
-            // (the same fence measured neutral in fp32 and 2-3.5 % slower on the transposed
-            // M/N-contiguous reads).
-#pragma unroll
-            for (int s = 0; s < 2 * KS; ++s) {
-                floatx4 av[TM], bv[TN];
-#pragma unroll
-                for (int tm = 0; tm < TM; ++tm) av[tm] = ra.read(sa, TM * wm + tm, s);
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn) bv[tn] = rb.read(sb, TN * wn + tn, s);
-                if (!A_KC && sum_a) {
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm) dsum[tm] += F::sum(av[tm]);
-                }
-                if constexpr (F::WIDE) {
-                    // fp32: the 16-byte operand is four k-steps of v_mfma_f32_32x32x2f32.
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-#pragma unroll
-                        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                            for (int tn = 0; tn < TN; ++tn)
-                                acc[tm][tn] =
-                                    __builtin_amdgcn_mfma_f32_32x32x2f32(av[tm][t], bv[tn][t], acc[tm][tn], 0, 0, 0);
-                } else {
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                        for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = F::mfma(av[tm], bv[tn], acc[tm][tn]);
-                }
-            }
-        }
+        shared_stage<F, A_KC, OA, OB, TM, TN, 2 * KS>(acc, dsum, ra, rb, sa, sb, wm, wn, sum_a);
         slot = slot + 1 == S ? 0 : slot + 1;
         islot = islot + 1 == S ? 0 : islot + 1;
     }
 
-    const uint32_t ebuf = base;
-    if (!A_KC && want_db) {
-        // Lane (col, h) holds the sum over its k of A row 32 (TM wm + tm) + col: LDS [h][BM]
-        // past the store buffer; one thread per row adds the halves in order.
-        const uint32_t dbuf = base + uint32_t(C::EPI);
-        __syncthreads();  // the ring is no longer read
-        if (sum_a) {
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) st1(dbuf + uint32_t((h * BM + 32 * (TM * wm + tm) + col) * 4), dsum[tm]);
-        }
-        __syncthreads();
-        const int m = int(threadIdx.x);
-        if (m < BM && m0 + m < p.M) {
-            const float x = ld1(dbuf + uint32_t(m * 4)) + ld1(dbuf + uint32_t((BM + m) * 4));
-            if (p.splits > 1) {
-                p.ws[int64_t(p.nbatch) * p.splits * p.M * p.N + (int64_t(z) * p.splits + split) * p.M + m0 + m] = x;
-            } else {
-                char *dst = p.db[z] + int64_t(m0 + m) * F::EB;
-                F::store(dst, F::load(dst) + x);
-            }
-        }
-    }
+    shared_store<F, A_KC, WM, WN, TM, TN>(acc, dsum, p, view_c, base, m0, n0, z, split, wm, wn, lane, want_db, sum_a);
+}
 
-    // Stores, one wave row of the tile (32 TM rows x BN columns) at a time through LDS:
-    // register r of lane (col, h) holds row acc_row(r, h) of column col of each 32 x 32 tile.
-    char *const cz = p.c[z];
-    const char *const bz = p.bias[z];
-    constexpr int Q = 32 * TM * BN / 4;
-#pragma unroll 1
-    for (int pm = 0; pm < WM; ++pm) {
-        __syncthreads();  // the ring (or the previous pass) is no longer read
-        if (wm == pm) {
+// ---- ragged products ----
+//
+// What the kernels above refuse because a direct global -> LDS load moves whole aligned 16-byte
+// chunks: any K, any pitch and alignment (a vocabulary of 50257: rows on 2-byte boundaries), M / N
+// extents that no chunk divides, and head-split views whose K stages straddle a batch (a weight
+// gradient over sequences of any length) or a head.  The shared-tile scheme (WM x WN waves on one
+// tile, one LDS copy of each stage), with the operands loaded to registers a stage ahead and
+// written to LDS after the stage's MFMAs: a chunk is one 16-byte load from its element-aligned
+// address, or element by element where it crosses the end of K or of the matrix; what lies past
+// the end of K is zero in both operands.  Two slots, one barrier per stage.
+//
+// Bound: the loads' address arithmetic and the LDS writes beside the MFMAs (about 500 TFLOP/s at
+// bf16 2048 x 5461 x 2048, where the direct loads reach 800-950 on aligned shapes: those keep
+// them).  Measured, us, the fp32-widening projection kernels -> this: bf16 dX 2048 x 5461 x 2048
+// 1960 -> 91, dW 1926 -> 188; dX 256 x 50257 x 256 8880 -> 49; forward 4096 x 4000 x 1000 412 ->
+// 71; 100 x 1000 x 1000 51 -> 14; fp32 dX 2048 x 5461 x 2048 995 -> 447, forward 4096 x 4000 x
+// 1000 346 -> 300, 100 x 1000 x 1000 36.9 -> 35.6; layer dW (B4 T1001 E768 H12 d64, bf16) 215 ->
+// 46 (Q, K, V) and 22 us.
+template <typename F, typename Op, bool KC>
+struct RagOp {
+    static constexpr int EPC = 16 / F::EB;          // elements per chunk
+    static constexpr int NC = Op::BYTES / 16 / 256;  // chunks per thread per stage
+    static_assert(NC * 16 * 256 == Op::BYTES, "a stage is whole chunks of 256 threads");
+    int64_t fix[NC];   // byte offset of the chunk's row (K-contiguous) or first column
+    int32_t line[NC];  // K-contiguous: its element offset in the stage; else its k-row
+    int32_t room[NC];  // elements of the chunk before the end of the matrix (not K)
+    u32x4 reg[NC];
+
+    __device__ __forceinline__ void init(const DView &v, int r0, int extent) {
 #pragma unroll
-            for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        st1(ebuf + uint32_t(((32 * tm + acc_row(r, h)) * BN + 32 * (TN * wn + tn) + col) * 4),
-                            acc[tm][tn][r]);
-        }
-        __syncthreads();
-        for (int qi = int(threadIdx.x); qi < Q; qi += NW * 64) {
-            const int m = qi / (BN / 4);
-            const int n = (qi - m * (BN / 4)) * 4;
-            const int gm = m0 + pm * 32 * TM + m, gn = n0 + n;
-            if (gm >= p.M || gn >= p.N) continue;
-            floatx4 x = ld4(ebuf + uint32_t((m * BN + n) * 4));
-            if (p.splits > 1) {
-                float *dst = p.ws + ((int64_t(z) * p.splits + split) * p.M + gm) * p.N + gn;
-                if (p.N % 4 == 0) {
-                    *reinterpret_cast<floatx4 *>(dst) = x;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (gn + e < p.N) dst[e] = x[e];
-                }
-                continue;
-            }
-            if (p.vec_out) {
-                const int64_t off = rowoff(view_c, gm) + coloff(view_c, gn);
-                char *dst = cz + off;
-                if (bz != nullptr) x += F::load4(bz + int64_t(gn) * F::EB);
-                if (p.beta) x += F::load4(dst);
-                if (p.act_mode == 1) {
-                    floatx4 y;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = act_fwd(p.act_kind, F::round(x[e]));
-                    F::store4(p.aux[z] + off, y);
-                } else if (p.act_mode == 2) {
-                    const floatx4 pre = F::load4(p.aux[z] + off);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = act_bwd_value(p.act_kind, pre[e], F::round(x[e]));
-                }
-                F::store4(dst, x);
+        for (int u = 0; u < NC; ++u) {
+            int l, lc;
+            Op::coord(256 * u + int(threadIdx.x), l, lc);
+            if constexpr (KC) {  // rows past the end re-read the last one; they are not stored
+                fix[u] = rowoff(v, min(r0 + l, extent - 1));
+                line[u] = EPC * lc;
+                room[u] = EPC;
             } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (gn + e >= p.N) break;
-                    const int64_t off = rowoff(view_c, gm) + coloff(view_c, gn + e);
-                    char *de = cz + off;
-                    float y = x[e];
-                    if (bz != nullptr) y += F::load(bz + int64_t(gn + e) * F::EB);
-                    if (p.beta) y += F::load(de);
-                    if (p.act_mode == 1) F::store(p.aux[z] + off, act_fwd(p.act_kind, F::round(y)));
-                    else if (p.act_mode == 2) y = act_bwd_value(p.act_kind, F::load(p.aux[z] + off), F::round(y));
-                    F::store(de, y);
-                }
+                const int c = r0 + EPC * lc;
+                fix[u] = coloff(v, min(c, extent - 1));
+                line[u] = l;
+                room[u] = extent - c;
             }
         }
     }
+    // The stage of K elements [k0, k0 + ...) of a segment of K elements at `base`.
+    __device__ __forceinline__ void load(const DView &v, const char *base, int k0, int K) {
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int k = k0 + line[u];
+            const int n = KC ? min(K - k, room[u]) : (k < K ? room[u] : 0);
+            reg[u] = u32x4{0, 0, 0, 0};
+            if (n <= 0) continue;
+            const char *p = base + fix[u] + (KC ? coloff(v, k) : rowoff(v, k));
+            if (n >= EPC) {
+                reg[u] = *reinterpret_cast<const u32x4u *>(p);
+            } else if constexpr (F::EB == 4) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (e < n) reg[u][e] = *reinterpret_cast<const uint32_t *>(p + 4 * e);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 7; ++e)
+                    if (e < n) reg[u][e / 2] |= uint32_t(*reinterpret_cast<const uint16_t *>(p + 2 * e)) << (16 * (e & 1));
+            }
+        }
+    }
+    __device__ __forceinline__ void store(uint32_t lds) const {
+#pragma unroll
+        for (int u = 0; u < NC; ++u)
+            *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(lds + 16u * (256u * u + threadIdx.x)) = reg[u];
+    }
+};
+
+template <typename F, bool A_KC, bool B_KC, int TM, int TN>
+struct RagCfg {
+    static constexpr int WM = 2, WN = 2, BM = 32 * TM * WM, BN = 32 * TN * WN;
+    static constexpr int KS = 2;            // 64-byte chunks per stage
+    static constexpr int KE = KS * F::KWE;  // K elements per stage
+    template <bool KC, int R>
+    using Op = std::conditional_t<KC, OpKC2<R>, std::conditional_t<F::WIDE, OpMN32<R, KE>, OpMN16<R, KE>>>;
+    using OA = Op<A_KC, BM>;
+    using OB = Op<B_KC, BN>;
+    static constexpr int STAGE = OA::BYTES + OB::BYTES;
+    static constexpr int EPI = 32 * TM * BN * 4 + (A_KC ? 0 : 2 * BM * 4);
+    static constexpr int LDS = 2 * STAGE > EPI ? 2 * STAGE : EPI;
+};
+
+template <typename F, bool A_KC, bool B_KC, int TM, int TN, bool GEN>
+__global__ __launch_bounds__(256) void lin_ragged_kernel(Args p) {
+    using C = RagCfg<F, A_KC, B_KC, TM, TN>;
+    using OA = typename C::OA;
+    using OB = typename C::OB;
+    __shared__ __attribute__((aligned(1024))) char smem[C::LDS];
+    DView view_a = p.av, view_b = p.bv, view_c = p.cv;
+    if constexpr (!GEN) view_a.heads = view_b.heads = view_c.heads = 0;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int wm = wave / C::WN, wn = wave % C::WN;
+
+    // XCD-aware order, as lin_kernel.
+    const int nblk = int(gridDim.x), blk = int(blockIdx.x);
+    const int q = nblk >> 3;
+    const int work = blk < 8 * q ? (blk & 7) * q + (blk >> 3) : blk;
+    const int ntiles = p.tiles_m * p.tiles_n;
+    const int per_batch = ntiles * p.splits;
+    const int z = work / per_batch;
+    const int rem = work - z * per_batch;
+    const int split = rem / ntiles;
+    const int tile = rem - split * ntiles;
+    const int ti = tile / p.tiles_n;
+    const int m0 = ti * C::BM, n0 = (tile - ti * p.tiles_n) * C::BN;
+    // This workgroup's stages (chunks, seg_chunks and cps count stages here).
+    const int st0 = split * p.cps;
+    const int nst = min(p.chunks - st0, p.cps);
+
+    RagOp<F, OA, A_KC> la;
+    RagOp<F, OB, B_KC> lb;
+    la.init(view_a, m0, p.M);
+    lb.init(view_b, n0, p.N);
+    typename OA::Lane ra;
+    typename OB::Lane rb;
+    ra.init(lane);
+    rb.init(lane);
+    const uint32_t base = lds_addr(smem);
+    auto load = [&](int c) {
+        int seg = 0;
+        if constexpr (GEN) seg = p.seg_chunks == p.chunks ? 0 : c / p.seg_chunks;
+        const int k0 = (c - seg * p.seg_chunks) * C::KE;
+        la.load(view_a, pick(p.a[z], seg), k0, p.K);
+        lb.load(view_b, pick(p.b[z], seg), k0, p.K);
+    };
+    auto store = [&](int slot) {
+        la.store(base + uint32_t(slot * C::STAGE));
+        lb.store(base + uint32_t(slot * C::STAGE + OA::BYTES));
+    };
+
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = zero16();
+    const bool want_db = !A_KC && p.db[z] != nullptr && n0 == 0;
+    const bool sum_a = want_db && wn == 0;
+    float dsum[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) dsum[i] = 0.f;
+
+    load(st0);
+    store(0);
+    __syncthreads();
+    for (int j = 0; j < nst; ++j) {
+        if (j + 1 < nst) load(st0 + j + 1);
+        const uint32_t sa = base + uint32_t((j & 1) * C::STAGE);
+        shared_stage<F, A_KC, OA, OB, TM, TN, 2 * C::KS>(acc, dsum, ra, rb, sa, sa + uint32_t(OA::BYTES), wm, wn, sum_a);
+        // The other slot was last read before the previous barrier.
+        if (j + 1 < nst) store((j + 1) & 1);
+        __syncthreads();
+    }
+    shared_store<F, A_KC, C::WM, C::WN, TM, TN>(acc, dsum, p, view_c, base, m0, n0, z, split, wm, wn, lane, want_db,
+                                                sum_a);
 }
 
 // ---- host side ----
@@ -1089,15 +1309,11 @@ inline int make_args(const LinGemm &g, const CfgInfo &c, int splits, void *ws, A
     a.nbatch = g.nbatch;
     a.seg_chunks = int32_t(g.K / chunk_elems(g.dtype));
     a.chunks = a.seg_chunks * g.nseg;
-    a.cps = (a.chunks + splits - 1) / splits;
+    a.cps = std::max(1, (a.chunks + splits - 1) / splits);
     a.splits = (a.chunks + a.cps - 1) / a.cps;  // no empty split
     a.beta = g.beta ? 1 : 0;
-    bool vec = g.N % 4 == 0;
-    for (int z = 0; z < g.nbatch; ++z)
-        vec = vec && uintptr_t(g.c[z]) % (4 * eb) == 0 && (g.bias[z] == nullptr || uintptr_t(g.bias[z]) % (4 * eb) == 0) &&
-              (g.act_mode == 0 || uintptr_t(g.aux[z]) % (4 * eb) == 0);
-    if (g.cv.heads == 0) vec = vec && g.cv.ld % 4 == 0;
-    a.vec_out = vec ? 1 : 0;
+    // Head-split columns 4 i .. 4 i + 3 lie in one head when d is a multiple of 4.
+    a.vec_out = g.cv.heads != 0 && g.cv.d % 4 != 0 ? 0 : g.N % 4 == 0 ? 2 : 1;
     return a.tiles_m * a.tiles_n * a.splits * g.nbatch;
 }
 
@@ -1109,10 +1325,11 @@ inline bool lin_gen(const LinGemm &g) {
 // The split-K reduction: C (and the bias gradients) from the partials of a.splits splits.
 template <typename F>
 hipError_t launch_reduce(const LinGemm &g, const Args &a, hipStream_t stream) {
-    const int64_t items = a.vec_out ? g.M * g.N / 4 : g.M * g.N;
+    const bool vec = a.vec_out == 2;
+    const int64_t items = vec ? g.M * g.N / 4 : g.M * g.N;
     const int64_t threads = std::max<int64_t>(items, g.M);  // bias gradients: one thread per row
     hipLaunchKernelGGL(lin_splitk_reduce_kernel<F>, dim3(unsigned((threads + 255) / 256), unsigned(g.nbatch)),
-                       dim3(256), 0, stream, a, items, a.vec_out);
+                       dim3(256), 0, stream, a, items, vec ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -1121,7 +1338,6 @@ hipError_t run(const LinGemm &g, const CfgInfo &c, int splits, void *ws, int64_t
     Args a{};
     const int nblk = make_args(g, c, splits, ws, a);
     if (a.splits > 1 && (ws == nullptr || ws_bytes < splits_bytes(g, a.splits))) return hipErrorInvalidValue;
-    if (a.splits > 1 && g.act_mode != 0) return hipErrorInvalidValue;  // the epilogue applies it
     hipError_t e = (lin_gen(g) ? c.launch_gen : c.launch)(a, nblk, stream);
     if (e != hipSuccess || a.splits == 1) return e;
     return launch_reduce<F>(g, a, stream);
@@ -1138,8 +1354,7 @@ hipError_t run_shared(const LinGemm &g, int splits, void *ws, int64_t ws_bytes, 
     if (a.seg_chunks % KS != 0) return hipErrorInvalidValue;
     a.cps = (a.cps + KS - 1) / KS * KS;  // whole stages per split
     a.splits = (a.chunks + a.cps - 1) / a.cps;
-    if (a.splits > 1 && (ws == nullptr || ws_bytes < splits_bytes(g, a.splits) || g.act_mode != 0))
-        return hipErrorInvalidValue;
+    if (a.splits > 1 && (ws == nullptr || ws_bytes < splits_bytes(g, a.splits))) return hipErrorInvalidValue;
     const int nblk = a.tiles_m * a.tiles_n * a.splits * g.nbatch;
     if (lin_gen(g))
         hipLaunchKernelGGL((lin_shared_kernel<F, A_KC, B_KC, WM, WN, TM, TN, S, KS, true>), dim3(unsigned(nblk)),
@@ -1150,6 +1365,61 @@ hipError_t run_shared(const LinGemm &g, int splits, void *ws, int64_t ws_bytes, 
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.splits == 1) return e;
     return launch_reduce<F>(g, a, stream);
+}
+
+// Launch of the ragged kernel on (64 TM) x (64 TN) tiles with K split across up to `splits`
+// workgroups.
+template <typename F, bool A_KC, bool B_KC, int TM, int TN>
+hipError_t run_ragged(const LinGemm &g, int splits, void *ws, int64_t ws_bytes, hipStream_t stream) {
+    using C = RagCfg<F, A_KC, B_KC, TM, TN>;
+    Args a{};
+    const CfgInfo c{TM * C::WM, TN * C::WN, C::WM * C::WN, 2, nullptr, nullptr};
+    make_args(g, c, 1, ws, a);
+    a.K = int32_t(g.K);
+    a.seg_chunks = int32_t((g.K + C::KE - 1) / C::KE);  // stages from here on
+    a.chunks = a.seg_chunks * g.nseg;
+    a.cps = (a.chunks + splits - 1) / splits;
+    a.splits = (a.chunks + a.cps - 1) / a.cps;
+    if (a.splits > 1 && (ws == nullptr || ws_bytes < splits_bytes(g, a.splits))) return hipErrorInvalidValue;
+    const unsigned nblk = unsigned(a.tiles_m * a.tiles_n * a.splits * g.nbatch);
+    if (lin_gen(g))
+        hipLaunchKernelGGL((lin_ragged_kernel<F, A_KC, B_KC, TM, TN, true>), dim3(nblk), dim3(256), 0, stream, a);
+    else
+        hipLaunchKernelGGL((lin_ragged_kernel<F, A_KC, B_KC, TM, TN, false>), dim3(nblk), dim3(256), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.splits == 1) return e;
+    return launch_reduce<F>(g, a, stream);
+}
+
+// The ragged plan: 128 x 128 tiles where they, with their K splits, give at least 192 workgroups
+// (three quarters of the CUs), else 64 x 64 tiles; K split (with workspace) up to 512 workgroups,
+// each keeping at least 4 stages.
+struct RaggedPlan {
+    bool big;
+    int splits;
+};
+inline RaggedPlan ragged_plan(const LinGemm &g, bool allow_split) {
+    const int64_t ke = 2 * chunk_elems(g.dtype);
+    const int64_t stages = (g.K + ke - 1) / ke * g.nseg;
+    auto tiles = [&](int64_t t) { return ((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.nbatch; };
+    auto splits = [&](int64_t t) {
+        if (!allow_split) return int64_t(1);
+        return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(512 / t, stages / 4), 16));
+    };
+    const int64_t big = tiles(128), sb = splits(big);
+    if (big * sb >= 192) return RaggedPlan{true, int(sb)};
+    return RaggedPlan{false, int(splits(tiles(64)))};
+}
+template <typename F, bool A_KC, bool B_KC>
+hipError_t run_ragged_tile(const LinGemm &g, const RaggedPlan &pl, void *ws, int64_t ws_bytes, hipStream_t stream) {
+    return pl.big ? run_ragged<F, A_KC, B_KC, 2, 2>(g, pl.splits, ws, ws_bytes, stream)
+                  : run_ragged<F, A_KC, B_KC, 1, 1>(g, pl.splits, ws, ws_bytes, stream);
+}
+template <typename F>
+hipError_t run_ragged_plan(const LinGemm &g, const RaggedPlan &pl, void *ws, int64_t ws_bytes, hipStream_t stream) {
+    if (!g.a_kc) return run_ragged_tile<F, false, false>(g, pl, ws, ws_bytes, stream);
+    return g.b_kc ? run_ragged_tile<F, true, true>(g, pl, ws, ws_bytes, stream)
+                  : run_ragged_tile<F, true, false>(g, pl, ws, ws_bytes, stream);
 }
 
 // The shared-tile plan of a supported product: ks 0 (not taken), or the stage depth in K
@@ -1334,6 +1604,25 @@ bool shape_ok(const LinGemm &g) {
     return wg * c.nw * 64 < (int64_t(1) << 32);
 }
 
+// A view of the ragged kernels: any pitch, or head-split with a 16-byte chunk along d inside one
+// head.
+bool ragged_view_ok(const LinView &v, int dtype) {
+    if (v.heads == 0) return v.ld >= 0;
+    return v.heads >= 1 && v.T >= 1 && v.d >= 1 && v.d % (16 / lin::elem_bytes(dtype)) == 0;
+}
+bool ragged_ok(const LinGemm &g) {
+    if (g.dtype < 0 || g.dtype > 2 || (!g.a_kc && g.b_kc)) return false;
+    if (g.act_mode != 0 && (g.act_mode > 2 || !g.a_kc || g.beta || g.act_kind < CTATTN_ACT_RELU ||
+                            g.act_kind > CTATTN_ACT_TANH))
+        return false;
+    if (g.nbatch < 1 || g.nbatch > kLinMaxBatch || g.nseg < 1 || g.nseg > kLinMaxSeg) return false;
+    if (g.M < 1 || g.N < 1 || g.K < 1 || g.M > (1 << 30) || g.N > (1 << 30) || g.K * g.nseg > (1 << 30)) return false;
+    if (!ragged_view_ok(g.av, g.dtype) || !ragged_view_ok(g.bv, g.dtype)) return false;
+    if (g.cv.heads == 0 ? g.cv.ld < g.N : (g.cv.d < 1 || g.cv.T < 1)) return false;
+    // Launch size: workgroups x threads below 2^32 for either tile, split or not.
+    return cdiv(g.M, 64) * cdiv(g.N, 64) * g.nbatch * 256 < (int64_t(1) << 32) / 16;
+}
+
 }  // namespace
 
 LinGemm lin_plain(int dtype, bool a_kc, bool b_kc, int64_t M, int64_t N, int64_t K, const void *a, int64_t lda,
@@ -1358,27 +1647,50 @@ LinGemm lin_plain(int dtype, bool a_kc, bool b_kc, int64_t M, int64_t N, int64_t
     return g;
 }
 
-bool lin_gemm_supported(const LinGemm &g) {
+namespace {
+
+// The shape, pitches and operand alignment of the direct-load kernels.
+bool direct_ok(const LinGemm &g) {
     if (!shape_ok(g)) return false;
-    for (int z = 0; z < g.nbatch; ++z) {
-        if (g.c[z] == nullptr || (g.act_mode != 0 && g.aux[z] == nullptr)) return false;
+    for (int z = 0; z < g.nbatch; ++z)
         for (int s = 0; s < g.nseg; ++s)
-            if (g.a[z][s] == nullptr || g.b[z][s] == nullptr || uintptr_t(g.a[z][s]) % 16 != 0 ||
-                uintptr_t(g.b[z][s]) % 16 != 0)
-                return false;
-    }
+            if (uintptr_t(g.a[z][s]) % 16 != 0 || uintptr_t(g.b[z][s]) % 16 != 0) return false;
     return true;
 }
 
-int64_t lin_gemm_workspace_bytes(const LinGemm &g) {
+}  // namespace
+
+bool lin_gemm_supported(const LinGemm &g) {
+    for (int z = 0; z < g.nbatch && z < kLinMaxBatch; ++z) {
+        if (g.c[z] == nullptr || (g.act_mode != 0 && g.aux[z] == nullptr)) return false;
+        for (int s = 0; s < g.nseg && s < kLinMaxSeg; ++s)
+            if (g.a[z][s] == nullptr || g.b[z][s] == nullptr) return false;
+    }
+    return direct_ok(g) || ragged_ok(g);
+}
+
+int64_t lin_gemm_workspace_min(const LinGemm &g) {
     if (!shape_ok(g)) return 0;
     // The launch trims empty splits, never adds any: this is an upper bound.
     const lin::SharedPlan sp = lin::shared_plan(g, true);
     return lin::splits_bytes(g, sp.ks != 0 ? sp.splits : plan(g, true).splits);
 }
 
+int64_t lin_gemm_workspace_bytes(const LinGemm &g) {
+    if (shape_ok(g)) return lin_gemm_workspace_min(g);
+    return ragged_ok(g) ? lin::splits_bytes(g, lin::ragged_plan(g, true).splits) : 0;
+}
+
 hipError_t launch_lin_gemm(const LinGemm &g, void *ws, int64_t ws_bytes, hipStream_t stream) {
     if (!lin_gemm_supported(g)) return hipErrorInvalidValue;
+    if (!direct_ok(g)) {
+        lin::RaggedPlan pl = lin::ragged_plan(g, true);
+        if (pl.splits > 1 && (ws == nullptr || uintptr_t(ws) % 16 != 0 || ws_bytes < lin::splits_bytes(g, pl.splits)))
+            pl = lin::ragged_plan(g, false);
+        return g.dtype == 0   ? lin::run_ragged_plan<F32Fmt>(g, pl, ws, ws_bytes, stream)
+               : g.dtype == 1 ? lin::run_ragged_plan<BF16Fmt>(g, pl, ws, ws_bytes, stream)
+                              : lin::run_ragged_plan<F16Fmt>(g, pl, ws, ws_bytes, stream);
+    }
     lin::SharedPlan sp = lin::shared_plan(g, true);
     if (sp.splits > 1 && (ws == nullptr || ws_bytes < lin::splits_bytes(g, sp.splits))) sp = lin::shared_plan(g, false);
     if (sp.ks != 0)

@@ -3,10 +3,9 @@
 //
 // Each entry point validates its arguments on the host, describes its products as
 // separable views (row-major [B*T, E] activations, [B, H, T, d] attention tensors, [out][in]
-// weights) and launches the split-K-in-workgroup MFMA GEMMs of linear_gemm.hip (fp32, bf16,
-// fp16) on the caller's stream.  fp64, shapes outside that family's domain (K not a multiple
-// of the K chunk, an unaligned operand, head dims that split a chunk) and the GENERIC policy
-// take the projection family of proj_gemm.hip.
+// weights) and launches the MFMA GEMMs of linear_gemm.hip (fp32, bf16, fp16) on the caller's
+// stream.  fp64, shapes outside that family's domain (head dims that are no multiple of a
+// 16-byte chunk) and the GENERIC policy take the projection family of proj_gemm.hip.
 #include "capi_util.h"
 #include "ctattn.h"
 #include "linear_gemm.h"
@@ -152,8 +151,12 @@ ctattn::LinGemm lin_out_dx(int dtype, const ProjShape &s) {
                     ctattn::lin_linear(s.hd()), ctattn::lin_heads(s.T, s.H, s.d), false);
 }
 
-// Split-K bytes for either family's plan of a weight gradient.
+// Split-K bytes of the direct-load GEMMs' plan of a weight gradient (the least a call must bring,
+// with the projection family's) and of whichever GEMM's (what the workspace queries ask for).
 int64_t lin_split_bytes(int dtype, const ctattn::LinGemm &g) {
+    return lin_policy(dtype) ? align_up(ctattn::lin_gemm_workspace_min(g)) : 0;
+}
+int64_t lin_query_bytes(int dtype, const ctattn::LinGemm &g) {
     return lin_policy(dtype) ? align_up(ctattn::lin_gemm_workspace_bytes(g)) : 0;
 }
 
@@ -196,12 +199,19 @@ int ctattn_qkv_proj_fwd(int dtype, const void *x, const void *wq, const void *wk
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 3, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
+namespace {
+int64_t qkv_bwd_need(int dtype, const ProjShape &s) {
+    return std::max(splitk_bytes(dtype, s.hd(), s.E, s.rows(), 3), lin_split_bytes(dtype, lin_qkv_dw(dtype, s))) +
+           align_up(ctattn::colsum_workspace_bytes(dtype, s.rows(), s.hd()));
+}
+}  // namespace
+
 int64_t ctattn_qkv_proj_bwd_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t E, int64_t H, int64_t d) {
     const ProjShape s{B, T, E, H, d};
     if (validate_proj("ctattn_qkv_proj_bwd_workspace_bytes", dtype, s)) return -1;
     ok();
-    return std::max(splitk_bytes(dtype, s.hd(), E, s.rows(), 3), lin_split_bytes(dtype, lin_qkv_dw(dtype, s))) +
-           align_up(ctattn::colsum_workspace_bytes(dtype, s.rows(), s.hd()));
+    return std::max({qkv_bwd_need(dtype, s), lin_query_bytes(dtype, lin_qkv_dw(dtype, s)),
+                     lin_query_bytes(dtype, lin_qkv_dx(dtype, s))});
 }
 
 int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk, const void *dv,
@@ -217,7 +227,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
     if (want_dw && !(dwq && dwk && dwv)) return fail(hipErrorInvalidValue, "%s: give all of dwq/dwk/dwv or none", fn);
     if (want_db && !(dbq && dbk && dbv)) return fail(hipErrorInvalidValue, "%s: give all of dbq/dbk/dbv or none", fn);
     if (dx && !(wq && wk && wv)) return fail(hipErrorInvalidValue, "%s: dx needs wq/wk/wv", fn);
-    const int64_t need = ctattn_qkv_proj_bwd_workspace_bytes(dtype, B, T, E, H, d);
+    const int64_t need = qkv_bwd_need(dtype, s);
     if ((want_dw || want_db) && (workspace == nullptr || workspace_bytes < need))
         return fail(hipErrorInvalidValue,
                     "%s: workspace of %lld bytes given, %lld needed (ctattn_qkv_proj_bwd_workspace_bytes)", fn,
@@ -242,7 +252,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
             lg.db[z] = ob[z];
         }
         if (ctattn::lin_gemm_supported(lg)) {
-            e = ctattn::launch_lin_gemm(lg, workspace, split_bytes, st);
+            e = ctattn::launch_lin_gemm(lg, workspace, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dw_done = true;
             db_done = want_db;
@@ -257,7 +267,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
         }
         lg.c[0] = dx;
         if (ctattn::lin_gemm_supported(lg)) {
-            e = ctattn::launch_lin_gemm(lg, nullptr, 0, st);
+            e = ctattn::launch_lin_gemm(lg, workspace, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dx_done = true;
         }
@@ -330,12 +340,19 @@ int ctattn_out_proj_fwd(int dtype, const void *c, const void *wo, const void *bo
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 1, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
+namespace {
+int64_t out_bwd_need(int dtype, const ProjShape &s) {
+    return std::max(splitk_bytes(dtype, s.E, s.hd(), s.rows(), 1), lin_split_bytes(dtype, lin_out_dw(dtype, s))) +
+           align_up(ctattn::colsum_workspace_bytes(dtype, s.rows(), s.E));
+}
+}  // namespace
+
 int64_t ctattn_out_proj_bwd_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t E, int64_t H, int64_t d) {
     const ProjShape s{B, T, E, H, d};
     if (validate_proj("ctattn_out_proj_bwd_workspace_bytes", dtype, s)) return -1;
     ok();
-    return std::max(splitk_bytes(dtype, E, s.hd(), s.rows(), 1), lin_split_bytes(dtype, lin_out_dw(dtype, s))) +
-           align_up(ctattn::colsum_workspace_bytes(dtype, s.rows(), E));
+    return std::max({out_bwd_need(dtype, s), lin_query_bytes(dtype, lin_out_dw(dtype, s)),
+                     lin_query_bytes(dtype, lin_out_dx(dtype, s))});
 }
 
 int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo, void *dwo, void *dbo,
@@ -348,7 +365,7 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
     if (!dy) return fail(hipErrorInvalidValue, "%s: null dy pointer", fn);
     if (dwo && !c) return fail(hipErrorInvalidValue, "%s: dwo needs the attention output c", fn);
     if (dc && !wo) return fail(hipErrorInvalidValue, "%s: dc needs wo", fn);
-    const int64_t need = ctattn_out_proj_bwd_workspace_bytes(dtype, B, T, E, H, d);
+    const int64_t need = out_bwd_need(dtype, s);
     if ((dwo || dbo) && (workspace == nullptr || workspace_bytes < need))
         return fail(hipErrorInvalidValue,
                     "%s: workspace of %lld bytes given, %lld needed (ctattn_out_proj_bwd_workspace_bytes)", fn,
@@ -366,7 +383,7 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
         g.c[0] = dwo;
         g.db[0] = dbo;  // the bias gradient (column sums of dy) from the same launch
         if (ctattn::lin_gemm_supported(g)) {
-            e = ctattn::launch_lin_gemm(g, workspace, split_bytes, st);
+            e = ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dwo = nullptr;
             dbo = nullptr;
@@ -395,7 +412,8 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
         g.a[0][0] = dy;
         g.b[0][0] = wo;
         g.c[0] = dc;
-        if (ctattn::lin_gemm_supported(g)) return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, st), st);
+        if (ctattn::lin_gemm_supported(g))
+            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st), st);
     }
     if (dc) {
         // dc(r, c) = sum_e dy[r][e] wo[e][c]: A = dy (K-contiguous), B = wo stored [k][n]; out
@@ -479,10 +497,18 @@ int ctattn_linear_fwd(int dtype, const void *x, const void *w, const void *b, vo
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 1, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
+namespace {
+int64_t linear_bwd_need(int dtype, int64_t M, int64_t N, int64_t K) {
+    return linear_split_bytes(dtype, M, N, K) + align_up(ctattn::colsum_workspace_bytes(dtype, M, N));
+}
+}  // namespace
+
 int64_t ctattn_linear_bwd_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
     if (validate_linear("ctattn_linear_bwd_workspace_bytes", dtype, M, N, K)) return -1;
     ok();
-    return linear_split_bytes(dtype, M, N, K) + align_up(ctattn::colsum_workspace_bytes(dtype, M, N));
+    return std::max({linear_bwd_need(dtype, M, N, K),
+                     lin_query_bytes(dtype, lin_dw(dtype, nullptr, nullptr, nullptr, M, N, K)),
+                     lin_query_bytes(dtype, lin_dx(dtype, nullptr, nullptr, nullptr, M, N, K))});
 }
 
 int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, void *dx, void *dw, void *db,
@@ -493,7 +519,7 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
     if (!dy) return fail(hipErrorInvalidValue, "%s: null dy pointer", fn);
     if (dw && !x) return fail(hipErrorInvalidValue, "%s: dw needs x", fn);
     if (dx && !w) return fail(hipErrorInvalidValue, "%s: dx needs w", fn);
-    const int64_t need = ctattn_linear_bwd_workspace_bytes(dtype, M, N, K);
+    const int64_t need = linear_bwd_need(dtype, M, N, K);
     if ((dw || db) && (workspace == nullptr || workspace_bytes < need))
         return fail(hipErrorInvalidValue,
                     "%s: workspace of %lld bytes given, %lld needed (ctattn_linear_bwd_workspace_bytes)", fn,
@@ -507,7 +533,7 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
         ctattn::LinGemm g = lin_dw(dtype, x, dy, dw, M, N, K);
         g.db[0] = db;  // the bias gradient (column sums of dy) from the same launch
         if (ctattn::lin_gemm_supported(g)) {
-            e = ctattn::launch_lin_gemm(g, workspace, split_bytes, st);
+            e = ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dw = nullptr;
             db = nullptr;
@@ -533,7 +559,8 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
     }
     if (dx && lin_policy(dtype)) {
         const ctattn::LinGemm g = lin_dx(dtype, dy, w, dx, M, N, K);
-        if (ctattn::lin_gemm_supported(g)) return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, st), st);
+        if (ctattn::lin_gemm_supported(g))
+            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st), st);
     }
     if (dx) {
         // dx[m][k] = sum_n dy[m][n] w[n][k]: A = dy [M][N] (K-contiguous), B = w stored [k'][n'].
@@ -585,7 +612,7 @@ int ctattn_linear_act_bwd(int dtype, int act, const void *x, const void *w, cons
         g.act_kind = act;
         g.aux[0] = const_cast<void *>(pre);
         if (ctattn::lin_gemm_supported(g))
-            return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, as_stream(stream)), as_stream(stream));
+            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, as_stream(stream)), as_stream(stream));
     }
     if (int rc = ctattn_linear_bwd(dtype, x, w, dy, dpre, nullptr, nullptr, workspace, workspace_bytes, M, N, K, stream))
         return rc;

@@ -891,21 +891,27 @@ int ctattn_tensor_matmul(int dtype, const void *a, const void *b, void *c, int64
         return finish(fn, e, st);
     }
     // fp32 / bf16 / fp16 on the plain GEMMs of linear_gemm.hip (A [M][K] K-contiguous, B stored
-    // [K][N]): one launch when the batches stack (one B), one per batch for up to 16 batches.
+    // [K][N]): one launch when the batches stack (one B), one per three for up to 16 batches.
     const int64_t rows = batch_b == 1 ? batch * M : M;
     if ((dtype == CTATTN_F32 || dtype == CTATTN_BF16 || dtype == CTATTN_F16) &&
         ctattn_get_policy() != CTATTN_POLICY_GENERIC && (batch_b == 1 || batch <= 16)) {
         const int ld = dtype == CTATTN_F32 ? 0 : dtype == CTATTN_BF16 ? 1 : 2;
         const int64_t es1 = elem_size(dtype);
         const int64_t calls = batch_b == 1 ? 1 : batch;
-        auto product = [&](int64_t z) {
-            return ctattn::lin_plain(ld, true, false, rows, N, K, static_cast<const char *>(a) + z * M * K * es1, K,
-                                     static_cast<const char *>(b) + z * K * N * es1, N,
-                                     static_cast<char *>(c) + z * M * N * es1, N, nullptr, false);
+        auto product = [&](int64_t z0) {  // batches z0 .. of one launch
+            ctattn::LinGemm g = ctattn::lin_plain(ld, true, false, rows, N, K, nullptr, K, nullptr, N, nullptr, N,
+                                                  nullptr, false);
+            g.nbatch = int(std::min<int64_t>(ctattn::kLinMaxBatch, calls - z0));
+            for (int j = 0; j < g.nbatch; ++j) {
+                g.a[j][0] = static_cast<const char *>(a) + (z0 + j) * M * K * es1;
+                g.b[j][0] = static_cast<const char *>(b) + (z0 + j) * K * N * es1;
+                g.c[j] = static_cast<char *>(c) + (z0 + j) * M * N * es1;
+            }
+            return g;
         };
         bool all = true;
-        for (int64_t z = 0; z < calls && all; ++z) all = ctattn::lin_gemm_supported(product(z));
-        for (int64_t z = 0; z < calls && all; ++z) {
+        for (int64_t z = 0; z < calls && all; z += ctattn::kLinMaxBatch) all = ctattn::lin_gemm_supported(product(z));
+        for (int64_t z = 0; z < calls && all; z += ctattn::kLinMaxBatch) {
             const hipError_t e = ctattn::launch_lin_gemm(product(z), nullptr, 0, st);
             if (e != hipSuccess) return finish(fn, e, st);
         }
