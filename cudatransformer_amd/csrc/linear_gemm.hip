@@ -69,6 +69,7 @@
 #include "act_math.h"
 #include "attn_common.h"
 #include "attn_mfma_common.h"
+#include "row_vec.h"
 
 namespace ctattn {
 namespace lin {
@@ -173,25 +174,6 @@ using BF16Fmt = H16Fmt<true>;
 using F16Fmt = H16Fmt<false>;
 
 // ---- views ----
-
-// Division by a run-time divisor D >= 1 of indices 0 <= i < 2^31 as a multiply and a shift
-// (Granlund & Montgomery, "Division by invariant integers using multiplication", 1994, the
-// unsigned case): with l = ceil(log2 D) and m = floor(2^32 (2^l - D) / D) + 1,
-// i / D = (mulhi(i, m) + i) >> l exactly for every 32-bit i; mulhi(i, m) < i keeps the sum
-// below 2^32 for i < 2^31.
-struct FastDiv {
-    uint32_t mul, shift;
-};
-inline FastDiv make_fastdiv(uint32_t D) {
-    if (D == 0) return FastDiv{0, 0};  // no index to divide (an empty view)
-    uint32_t l = 0;
-    while (l < 32 && (uint64_t(1) << l) < D) ++l;
-    const uint64_t m = ((uint64_t(1) << 32) * ((uint64_t(1) << l) - D)) / D + 1;
-    return FastDiv{uint32_t(m), l};
-}
-__device__ __forceinline__ int fastdiv(int i, FastDiv f) {
-    return int((__umulhi(uint32_t(i), f.mul) + uint32_t(i)) >> f.shift);
-}
 
 // A LinView on the device, in bytes.  Indices are below 2^31 (checked on the host).  The
 // head-split offsets divide by T and d through FastDiv: the store loops of a tile compute

@@ -1,0 +1,89 @@
+"""LayerNorm, softmax and the fused softmax-cross-entropy gradient at the edges of their row
+kernels: waves per row, 16-byte granules per lane, rows off 16-byte boundaries (odd lengths, a
+tensor one element into its storage), and the lengths past which the general kernels take over,
+against float64.
+
+Tolerance: fp32 sums of up to 66000 terms, 1e-5 relative; 16-bit outputs round once more, at most
+2^-8 (bf16) or 2^-11 (fp16) of a value, so of the 2-norm too; dgamma / dbeta accumulate in storage
+from 0 and round once.
+"""
+import pytest
+import torch
+
+from cudatransformer_amd import _capi
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+TOL = {"f32": 1e-5, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}
+
+
+def rnd(shape, dt, seed, std=1.0, shift=0.0, offset=1):
+    """Random values `offset` elements past a 16-byte boundary."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    n = 1
+    for s in shape:
+        n *= s
+    buf = torch.empty(n + 16, dtype=dt, device="cuda")
+    t = buf[offset:offset + n].view(shape)
+    t.copy_(shift + std * torch.randn(shape, generator=g, device="cuda"))
+    return t
+
+
+def close(got, want, tol, what):
+    err = (got.double() - want).norm() / want.norm().clamp_min(1e-30)
+    assert err <= tol, (what, float(err))
+
+
+@pytest.mark.parametrize("d", [1, 7, 64, 255, 256, 511, 512, 513, 1024, 1029, 2048, 2056, 4096, 4100, 8192, 8200])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_layernorm_edges(name, d):
+    dt, n = DT[name], 37  # one full 32-row chunk and a ragged one
+    print(f"layernorm {name} D={d}", flush=True)
+    for offset in (0, 1):
+        x, dy = rnd((n, d), dt, 1, 2.0, 0.5, offset), rnd((n, d), dt, 2, offset=offset)
+        g, b = rnd((d,), dt, 3, 0.1, 1.0, offset), rnd((d,), dt, 4, 0.1, 0.0, offset)
+        y, mean, rstd = _capi.layernorm_fwd(x, g, b)
+        dg, db = torch.zeros_like(g), torch.zeros_like(b)
+        dx = _capi.layernorm_bwd(x, g, dy, mean, rstd, dg, db)
+        torch.cuda.synchronize()
+        x64, g64, b64, dy64 = x.double(), g.double(), b.double(), dy.double()
+        mu = x64.mean(-1, keepdim=True)
+        rs = torch.rsqrt(((x64 - mu) ** 2).mean(-1, keepdim=True) + 1e-5)
+        xh = (x64 - mu) * rs
+        dxh = dy64 * g64
+        close(mean, mu[:, 0], 1e-5, "mean")
+        close(rstd, rs[:, 0], 1e-5, "rstd")
+        close(y, xh * g64 + b64, TOL[name], "y")
+        # D = 1: dx vanishes; its scale is the terms that cancel.
+        want = rs * (dxh - dxh.mean(-1, keepdim=True) - xh * (dxh * xh).mean(-1, keepdim=True))
+        scale = (rs * dxh).norm()
+        assert ((dx.double() - want).norm() / scale) <= TOL[name], "dx"
+        if d > 1:
+            close(dg, (dy64 * xh).sum(0), TOL[name], "dgamma")
+        close(db, dy64.sum(0), TOL[name], "dbeta")
+
+
+@pytest.mark.parametrize("v", [1, 3, 65, 256, 257, 512, 1025, 2048, 4097, 8193, 16385, 32769, 65536, 65537])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_softmax_and_gradient_edges(name, v):
+    dt, n = DT[name], 6
+    print(f"softmax {name} V={v}", flush=True)
+    z = rnd((n, v), dt, 5, 3.0)
+    if v > 3:
+        z[1, 2:] = float("-inf")  # masked classes
+        z[2] = torch.finfo(dt).min  # a row at the type's lowest value
+    t = torch.randint(0, v, (n,), device="cuda", dtype=torch.int32)
+    t[3], t[4] = -1, v
+    p = _capi.softmax_fwd(z, 0.7)
+    dz = _capi.softmax_cross_entropy_bwd(p, t, 0.7)
+    torch.cuda.synchronize()
+    want = torch.softmax(z.double() / 0.7, -1)
+    # fp16: probabilities below its subnormals' half step round to 0.
+    floor = 2.0 ** -25 if name == "f16" else 0.0
+    assert ((p.double() - want).abs() <= TOL[name] * want + floor + 1e-5 * (name == "f32") * want).all()
+    onehot = torch.zeros_like(want)
+    ok = (t >= 0) & (t < v)
+    onehot[ok.nonzero()[:, 0], t[ok].long()] = 1.0
+    ref = (p.double() - onehot) * ok[:, None] / (n * 0.7)
+    assert ((dz.double() - ref).abs() <= TOL[name] * ref.abs() + floor + 1e-7).all()
