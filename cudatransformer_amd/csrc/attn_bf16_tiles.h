@@ -139,6 +139,42 @@ __device__ __forceinline__ void load_tile_dma(const char *tile, const uint16_t *
     }
 }
 
+// 16 zero bytes: what tile columns past a head dim below the tile's width are loaded from.
+__device__ __attribute__((aligned(16))) const uint32_t tile_zeros[4] = {0, 0, 0, 0};
+
+// load_tile_dma of a tensor with rows of ld <= D elements (a multiple of 8; `block` and `ld` give
+// 16-byte aligned chunks): the tile's chunks at and past ld are zeros, so they add nothing to a
+// contraction over the head dim.
+template <int D, int ROWS, int NW>
+__device__ __forceinline__ void load_tile_dma_ld(const char *tile, const uint16_t *block, int ld, int rows, int wave,
+                                                 int lane) {
+    using L = Tile<D>;
+    constexpr int TOTAL = ROWS * L::CH;
+    constexpr int NL = (TOTAL + NW * kWave - 1) / (NW * kWave);
+    static_assert(TOTAL % kWave == 0, "tile size");
+    const uint32_t tile_lds = uint32_t(uintptr_t((__attribute__((address_space(3))) const char *)tile));
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int P = (wave * NL + i) * kWave + lane;
+        if (TOTAL % (NW * kWave) == 0 || (wave * NL + i) * kWave < TOTAL) {
+            const int r = P / L::CH;
+            const int c = 8 * ((P % L::CH) ^ L::swz(r));
+            const uint16_t *g = c < ld ? block + uint32_t(min(r, rows - 1) * ld + c)
+                                       : reinterpret_cast<const uint16_t *>(tile_zeros);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(tile_lds + uint32_t((wave * NL + i) * kWave * 16));
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(dst)
+                         : "memory", "m0");
+        }
+    }
+}
+// load_tile_dma (PAD false: rows of D elements, ld unused) or load_tile_dma_ld.
+template <int D, int ROWS, int NW, bool PAD>
+__device__ __forceinline__ void load_tile_any(const char *tile, const uint16_t *block, int ld, int rows, int wave,
+                                              int lane) {
+    if constexpr (PAD) load_tile_dma_ld<D, ROWS, NW>(tile, block, ld, rows, wave, lane);
+    else load_tile_dma<D, ROWS, NW>(tile, block, rows, wave, lane);
+}
+
 // One dword per lane, global -> LDS, through inline asm like load_tile_dma: lane l's value
 // lands at LDS byte address `dst` + 4 l (`dst` wave-uniform).
 __device__ __forceinline__ void load_dword_dma(const void *g, uint32_t dst) {

@@ -76,13 +76,13 @@ __device__ __forceinline__ int ds_col_row(int c) {
 // ---------------------------------------------------------------------------------------
 // dK / dV (key-major)
 // ---------------------------------------------------------------------------------------
-template <int D>
+template <int D, int W = D>
 struct KvCfg {
     static constexpr int NW = 8;       // waves: 4 key slices (ks = wave & 3) x 2 row slices (rs = wave >> 2)
     static constexpr int BN = 128;     // keys per workgroup; key slice ks: 32 ks .. 32 ks + 31
     static constexpr int BM = 64;      // query rows per iteration; row slice rs: 32 rs .. 32 rs + 31
-    static constexpr int DT = D / 32;
-    static constexpr int KSTEPS = D / 16;
+    static constexpr int DT = W / 32;
+    static constexpr int KSTEPS = W / 16;
     static constexpr int ROW = 2 * D;            // bytes per tile row
     static constexpr int KV_BYTES = BN * ROW;    // K (or V) tile
     static constexpr int Q_BYTES = BM * ROW;     // Q (or dO) tile
@@ -105,11 +105,11 @@ struct KvCfg {
 //   ac0/1: col_base of the wave's Q rows (dO at + Q_BYTES)
 //   anl  : address of nl2[32 rs + 4 half] of the block (delta at + BM * 4)
 //   dsw  : when DS, where the tile's dS goes (a 32 x 32 DsTile, rows = keys)
-template <int D, bool MASK, bool DS, typename F>
-__device__ __forceinline__ void kv_block(floatx16 (&dk_acc)[D / 32], floatx16 (&dv_acc)[D / 32], uint32_t aq,
+template <int D, int W, bool MASK, bool DS, typename F>
+__device__ __forceinline__ void kv_block(floatx16 (&dk_acc)[W / 32], floatx16 (&dv_acc)[W / 32], uint32_t aq,
                                          uint32_t ak, uint32_t ac0, uint32_t ac1, uint32_t anl, int r0w,
                                          int key, int T, int causal, float c, int half, uint16_t *dsw) {
-    using C = KvCfg<D>;
+    using C = KvCfg<D, W>;
     using V = typename F::vec;
     // dP starts from -delta of the rows (register r: row acc_row(r, half)), so the
     // accumulator ends as dP - delta and dS = P * acc.
@@ -190,13 +190,13 @@ __device__ __forceinline__ void kv_block(floatx16 (&dk_acc)[D / 32], floatx16 (&
     }
 }
 
-template <int D, bool DS, typename F>
+template <int D, int W, bool PAD, bool DS, typename F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_bf16_dkdv_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     const uint16_t *__restrict__ dout, const float *__restrict__ nl2, const float *__restrict__ delta,
     uint16_t *__restrict__ dk, uint16_t *__restrict__ dv, uint16_t *__restrict__ ds, int T, int BH, int causal,
-    float c, float inv_sqrt_d) {
-    using C = KvCfg<D>;
+    float c, float inv_sqrt_d, int d) {
+    using C = KvCfg<D, W>;
     __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
     const uint32_t L = lds_addr(smem);
 
@@ -211,7 +211,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int bh = id % BH;
     const int kb = id / BH;  // causal: key block 0 has the most query blocks -> launched first
     const int k0 = kb * C::BN;
-    const int64_t base = int64_t(bh) * T * D;
+    const int ld = PAD ? d : D;  // elements per row in memory
+    const int64_t base = int64_t(bh) * T * ld;
     const int64_t rbase = int64_t(bh) * T;
     const int kw0 = k0 + 32 * ks;
     const int key = kw0 + col;
@@ -219,8 +220,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Tile loads go through load_tile_dma / load_dword_dma, which the compiler does not see:
     // it would otherwise make the block's first LDS read wait for the next block's prefetch.
     // The loop waits for each block's loads itself, before the barrier that publishes them.
-    load_tile_dma<D, C::BN, C::NW>(smem + C::K_OFF, k + base + int64_t(k0) * D, T - k0, wave, lane);
-    load_tile_dma<D, C::BN, C::NW>(smem + C::V_OFF, v + base + int64_t(k0) * D, T - k0, wave, lane);
+    load_tile_any<D, C::BN, C::NW, PAD>(smem + C::K_OFF, k + base + int64_t(k0) * ld, ld, T - k0, wave, lane);
+    load_tile_any<D, C::BN, C::NW, PAD>(smem + C::V_OFF, v + base + int64_t(k0) * ld, ld, T - k0, wave, lane);
     floatx16 dk_acc[C::DT], dv_acc[C::DT];
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) {
@@ -239,8 +240,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int qb_first = causal ? k0 / C::BM : 0;
     auto issue = [&](int r0, int buf) {
         char *qt = smem + C::Q_OFF + buf * 2 * C::Q_BYTES;
-        load_tile_dma<D, C::BM, C::NW>(qt, q + base + int64_t(r0) * D, T - r0, wave, lane);
-        load_tile_dma<D, C::BM, C::NW>(qt + C::Q_BYTES, dout + base + int64_t(r0) * D, T - r0, wave, lane);
+        load_tile_any<D, C::BM, C::NW, PAD>(qt, q + base + int64_t(r0) * ld, ld, T - r0, wave, lane);
+        load_tile_any<D, C::BM, C::NW, PAD>(qt + C::Q_BYTES, dout + base + int64_t(r0) * ld, ld, T - r0, wave, lane);
         if (wave >= C::NW - 2) {  // nl2 / delta of the block's rows, one dword per lane
             const bool is_nl = wave == C::NW - 2;
             load_dword_dma((is_nl ? nl2 : delta) + rbase + min(r0 + lane, T - 1),
@@ -274,10 +275,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const bool masked = (r0w + 32 > T) || (kw0 + 32 > T) || (causal && kw0 + 31 > r0w);
         uint16_t *dsw = DS ? ds + ds_tile_index(bh, r0w / 32, kw0 / 32, T, causal) * kDsTileElems : nullptr;
         if (masked)
-            kv_block<D, true, DS, F>(dk_acc, dv_acc, qt + rq, ak, qt + cq0, qt + cq1, anl, r0w, key, T, causal, c,
+            kv_block<D, W, true, DS, F>(dk_acc, dv_acc, qt + rq, ak, qt + cq0, qt + cq1, anl, r0w, key, T, causal, c,
                                      half, dsw);
         else
-            kv_block<D, false, DS, F>(dk_acc, dv_acc, qt + rq, ak, qt + cq0, qt + cq1, anl, r0w, key, T, causal, c,
+            kv_block<D, W, false, DS, F>(dk_acc, dv_acc, qt + rq, ak, qt + cq0, qt + cq1, anl, r0w, key, T, causal, c,
                                       half, dsw);
     }
 
@@ -297,12 +298,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     __syncthreads();
     if (rs == 0 && key < T) {
-        uint16_t *dkr = dk + base + int64_t(key) * D;
-        uint16_t *dvr = dv + base + int64_t(key) * D;
+        uint16_t *dkr = dk + base + int64_t(key) * ld;
+        uint16_t *dvr = dv + base + int64_t(key) * ld;
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if (PAD && dt * 32 + 8 * g >= ld) continue;
                 u16x4 xk, xv;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
@@ -322,13 +324,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---------------------------------------------------------------------------------------
 // dQ (query-major)
 // ---------------------------------------------------------------------------------------
-template <int D>
+template <int D, int W = D>
 struct QCfg {
     static constexpr int NW = 4;
     static constexpr int BM = 32 * NW;  // query rows per workgroup
     static constexpr int BN = 32;       // keys per iteration
-    static constexpr int DT = D / 32;
-    static constexpr int KSTEPS = D / 16;
+    static constexpr int DT = W / 32;
+    static constexpr int KSTEPS = W / 16;
     static constexpr int KB = BN * 2 * D;       // bytes of a K (or V) tile
     static constexpr int LDS_BYTES = 4 * KB;    // buffer b: K at 2 b KB, V at 2 b KB + KB
 };
@@ -336,12 +338,12 @@ struct QCfg {
 // One 32-key block for one wave (32 rows): S^T, dP^T, P^T, dS^T and the dQ update.
 //   ak   : row_base of the block's K tile for key `col` (V at + KB)
 //   ac0/1: col_base of the K tile
-template <int D, bool MASK, typename F>
-__device__ __forceinline__ void dq_block(floatx16 (&dq_acc)[D / 32], const typename F::vec (&qB)[D / 16],
-                                         const typename F::vec (&doB)[D / 16], uint32_t ak, uint32_t ac0,
+template <int D, int W, bool MASK, typename F>
+__device__ __forceinline__ void dq_block(floatx16 (&dq_acc)[W / 32], const typename F::vec (&qB)[W / 16],
+                                         const typename F::vec (&doB)[W / 16], uint32_t ak, uint32_t ac0,
                                          uint32_t ac1, float nlr, const floatx16 &ndl, int j0, int row, int T,
                                          int causal, float c, int half) {
-    using C = QCfg<D>;
+    using C = QCfg<D, W>;
     using V = typename F::vec;
     // dP^T starts from -delta of the lane's row, so the accumulator ends as dP^T - delta.
     floatx16 s = zero16(), dp = ndl;
@@ -388,12 +390,12 @@ __device__ __forceinline__ void dq_block(floatx16 (&dq_acc)[D / 32], const typen
     }
 }
 
-template <int D, typename F>
+template <int D, int W, bool PAD, typename F>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_bf16_dq_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     const uint16_t *__restrict__ dout, const float *__restrict__ nl2, const float *__restrict__ delta,
-    uint16_t *__restrict__ dq, int T, int BH, int causal, float c, float inv_sqrt_d) {
-    using C = QCfg<D>;
+    uint16_t *__restrict__ dq, int T, int BH, int causal, float c, float inv_sqrt_d, int d) {
+    using C = QCfg<D, W>;
     using V = typename F::vec;
     __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
     const uint32_t L = lds_addr(smem);
@@ -408,7 +410,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int id = blockIdx.x;
     const int bh = id % BH;
     const int qb = causal ? (nqb - 1 - id / BH) : id / BH;  // causal: longest first
-    const int64_t base = int64_t(bh) * T * D;
+    const int ld = PAD ? d : D;  // elements per row in memory
+    const int64_t base = int64_t(bh) * T * ld;
     const int64_t rbase = int64_t(bh) * T;
     const int r0 = qb * C::BM;
     const int wave_first_row = r0 + 32 * wave;
@@ -420,9 +423,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int st = 0; st < C::KSTEPS; ++st) {
         u16x8 xq = {0, 0, 0, 0, 0, 0, 0, 0}, xd = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (row < T) {
-            xq = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * D + 16 * st + 8 * half);
-            xd = *reinterpret_cast<const u16x8 *>(dout + base + int64_t(row) * D + 16 * st + 8 * half);
+        if (row < T && (!PAD || 16 * st + 8 * half < ld)) {
+            xq = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * ld + 16 * st + 8 * half);
+            xd = *reinterpret_cast<const u16x8 *>(dout + base + int64_t(row) * ld + 16 * st + 8 * half);
         }
         qB[st] = __builtin_bit_cast(V, xq);
         doB[st] = __builtin_bit_cast(V, xd);
@@ -444,8 +447,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // K / V blocks through load_tile_dma (invisible to the compiler, so the block's LDS reads do
     // not wait for the next block's prefetch); the loop awaits each block before its barrier.
     auto issue = [&](int j0, int buf) {
-        load_tile_dma<D, C::BN, C::NW>(smem + 2 * buf * C::KB, k + base + int64_t(j0) * D, T - j0, wave, lane);
-        load_tile_dma<D, C::BN, C::NW>(smem + 2 * buf * C::KB + C::KB, v + base + int64_t(j0) * D, T - j0, wave, lane);
+        load_tile_any<D, C::BN, C::NW, PAD>(smem + 2 * buf * C::KB, k + base + int64_t(j0) * ld, ld, T - j0, wave, lane);
+        load_tile_any<D, C::BN, C::NW, PAD>(smem + 2 * buf * C::KB + C::KB, v + base + int64_t(j0) * ld, ld, T - j0, wave,
+                                            lane);
     };
 
     // Block kb: wait for its loads (this wave's, then everyone's through the barrier, which
@@ -468,12 +472,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int kb = 0;
     for (; kb < jm; ++kb) {
         const uint32_t kt = step(kb);
-        dq_block<D, false, F>(dq_acc, qB, doB, kt + rk, kt + ck0, kt + ck1, nlr, ndl, kb * C::BN, row, T, causal, c,
+        dq_block<D, W, false, F>(dq_acc, qB, doB, kt + rk, kt + ck0, kt + ck1, nlr, ndl, kb * C::BN, row, T, causal, c,
                            half);
     }
     for (; kb < wave_nkb; ++kb) {
         const uint32_t kt = step(kb);
-        dq_block<D, true, F>(dq_acc, qB, doB, kt + rk, kt + ck0, kt + ck1, nlr, ndl, kb * C::BN, row, T, causal, c,
+        dq_block<D, W, true, F>(dq_acc, qB, doB, kt + rk, kt + ck0, kt + ck1, nlr, ndl, kb * C::BN, row, T, causal, c,
                           half);
     }
     for (; kb < nkb; ++kb) step(kb);
@@ -484,9 +488,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int r = 0; r < 16; ++r) {
         const int rr = wave_first_row + acc_row(r, half);
         if (rr >= T) continue;
-        uint16_t *p = dq + base + int64_t(rr) * D + col;
+        uint16_t *p = dq + base + int64_t(rr) * ld + col;
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt) p[32 * dt] = F::bits(dq_acc[dt][r] * inv_sqrt_d);
+        for (int dt = 0; dt < C::DT; ++dt)
+            if (!PAD || 32 * dt + col < ld) p[32 * dt] = F::bits(dq_acc[dt][r] * inv_sqrt_d);
     }
 }
 
@@ -498,12 +503,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // blocks: the block's K rows (a Tile<D>) and each wave's two dS tiles go global -> LDS
 // directly, three blocks in flight; dS^T columns (read_col<32>) are the A operands, K^T columns
 // (read_col<D>) the B operands, both in the same key order.  Bound by the dS stream from HBM.
-template <int D>
+template <int D, int W = D>
 struct DqDsCfg {
     static constexpr int NW = 8;
     static constexpr int BM = 32 * NW;        // query rows per workgroup
     static constexpr int BN = 64;             // keys per iteration: key tiles 2 kb, 2 kb + 1
-    static constexpr int DT = D / 32;
+    static constexpr int DT = W / 32;
     static constexpr int ROW = 2 * D;
     static constexpr int D8 = D / 8;          // 16-byte chunks per row
     static constexpr int KB = BN * ROW;       // K tile
@@ -528,11 +533,11 @@ __device__ __forceinline__ void dma_2k(const uint16_t *src, uint32_t dst, int la
     }
 }
 
-template <int D, typename F>
+template <int D, int W, bool PAD, typename F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_bf16_dq_ds_kernel(
     const uint16_t *__restrict__ k, const uint16_t *__restrict__ ds, uint16_t *__restrict__ dq, int T, int BH,
-    int causal, float inv_sqrt_d) {
-    using C = DqDsCfg<D>;
+    int causal, float inv_sqrt_d, int d) {
+    using C = DqDsCfg<D, W>;
     using V = typename F::vec;
     __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
     const uint32_t L = lds_addr(smem);
@@ -547,7 +552,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int id = blockIdx.x;
     const int bh = id % BH;
     const int qb = causal ? (nqb - 1 - id / BH) : id / BH;  // causal: longest first
-    const int64_t base = int64_t(bh) * T * D;
+    const int ld = PAD ? d : D;  // elements per row in memory
+    const int64_t base = int64_t(bh) * T * ld;
     const int r0 = qb * C::BM;
     const int nt = (T + 31) / 32;
     const int rt = r0 / 32 + wave;  // this wave's row tile
@@ -564,7 +570,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     auto issue = [&](int kb, int buf) {
         char *b = smem + buf * C::BUF;
-        load_tile_dma<D, C::BN, C::NW>(b, k + base + int64_t(kb) * C::BN * D, T - kb * C::BN, wave, lane);
+        load_tile_any<D, C::BN, C::NW, PAD>(b, k + base + int64_t(kb) * C::BN * ld, ld, T - kb * C::BN, wave, lane);
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
             const int kt = 2 * kb + tt;
@@ -615,9 +621,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int r = 0; r < 16; ++r) {
         const int row = 32 * rt + ds_col_row(acc_row(r, half));
         if (row >= T) continue;
-        uint16_t *p = dq + base + int64_t(row) * D + col;
+        uint16_t *p = dq + base + int64_t(row) * ld + col;
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt) p[32 * dt] = F::bits(dq_acc[dt][r] * inv_sqrt_d);
+        for (int dt = 0; dt < C::DT; ++dt)
+            if (!PAD || 32 * dt + col < ld) p[32 * dt] = F::bits(dq_acc[dt][r] * inv_sqrt_d);
     }
 }
 
@@ -625,12 +632,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // flash_attention.cu:269-273: the dP accumulators of both kernels start from it) and
 // nl2[row] = -LSE[row] * log2(e), the per-row term of P = exp2(S log2(e)/sqrt(d) + nl2).
 // D / 8 lanes per row, one 16-byte load of O and of dO each.
-template <int D, typename F>
+template <int D, bool PAD, typename F>
 __global__ __launch_bounds__(256) void bwd_preprocess_bf16_kernel(const uint16_t *__restrict__ o,
                                                                  const uint16_t *__restrict__ dout,
                                                                  const float *__restrict__ lse,
                                                                  float *__restrict__ delta,
-                                                                 float *__restrict__ nl2, int64_t rows) {
+                                                                 float *__restrict__ nl2, int64_t rows, int d) {
+    const int ld = PAD ? d : D;
     constexpr int LPR = D / 8;  // lanes per row
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     // Grid-stride; the block size and the stride are multiples of LPR, so the LPR lanes of a
@@ -639,9 +647,9 @@ __global__ __launch_bounds__(256) void bwd_preprocess_bf16_kernel(const uint16_t
         const int64_t row = t / LPR;
         const int c8 = int(t % LPR);
         float s = 0.f;
-        if (row < rows) {
-            const u16x8 a = *reinterpret_cast<const u16x8 *>(o + row * D + 8 * c8);
-            const u16x8 b = *reinterpret_cast<const u16x8 *>(dout + row * D + 8 * c8);
+        if (row < rows && (!PAD || 8 * c8 < ld)) {
+            const u16x8 a = *reinterpret_cast<const u16x8 *>(o + row * ld + 8 * c8);
+            const u16x8 b = *reinterpret_cast<const u16x8 *>(dout + row * ld + 8 * c8);
 #pragma unroll
             for (int e = 0; e < 8; ++e) s += F::widen(a[e]) * F::widen(b[e]);
         }
@@ -653,21 +661,22 @@ __global__ __launch_bounds__(256) void bwd_preprocess_bf16_kernel(const uint16_t
     }
 }
 
-template <int D, typename F>
+template <int D, int W, bool PAD, typename F>
 hipError_t bwd_bf16(const void *q, const void *k, const void *v, const void *o, const void *dout,
                     const float *lse, float *delta, void *dq, void *dk, void *dv, float *nl2, uint16_t *ds,
                     const AttnShape &s, hipStream_t stream) {
-    using KC = KvCfg<D>;
-    using QC = QCfg<D>;
+    using KC = KvCfg<D, W>;
+    using QC = QCfg<D, W>;
     const int64_t kv_blocks = ((s.T + KC::BN - 1) / KC::BN) * s.bh();
     const int64_t q_blocks = ((s.T + QC::BM - 1) / QC::BM) * s.bh();
     if (!grid_fits(kv_blocks, KC::NW * kWave) || !grid_fits(q_blocks, QC::NW * kWave) || s.T > 2147483647 / D)
         return hipErrorInvalidValue;
     const int64_t rows = s.rows();
+    const int d = int(s.scale_dim());  // PAD: elements per row in memory
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     const int64_t pre_threads = rows * (D / 8);
-    hipLaunchKernelGGL((bwd_preprocess_bf16_kernel<D, F>), dim3(stride_grid((pre_threads + 255) / 256, 256)), dim3(256), 0, stream,
-                       u16(o), u16(dout), lse, delta, nl2, rows);
+    hipLaunchKernelGGL((bwd_preprocess_bf16_kernel<D, PAD, F>), dim3(stride_grid((pre_threads + 255) / 256, 256)), dim3(256), 0, stream,
+                       u16(o), u16(dout), lse, delta, nl2, rows, d);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const float c = kLog2e / sqrtf(float(s.scale_dim()));
@@ -675,27 +684,53 @@ hipError_t bwd_bf16(const void *q, const void *k, const void *v, const void *o, 
     if constexpr (D == 128) {
         if (ds != nullptr) {
             // dS through the workspace: the dK/dV kernel stores it, the dQ kernel multiplies it by K.
-            hipLaunchKernelGGL((bwd_bf16_dkdv_kernel<D, true, F>), dim3(unsigned(kv_blocks)), dim3(KC::NW * kWave), 0,
+            hipLaunchKernelGGL((bwd_bf16_dkdv_kernel<D, W, PAD, true, F>), dim3(unsigned(kv_blocks)), dim3(KC::NW * kWave), 0,
                                stream, u16(q), u16(k), u16(v), u16(dout), nl2, delta, static_cast<uint16_t *>(dk),
-                               static_cast<uint16_t *>(dv), ds, int(s.T), int(s.bh()), int(s.causal), c, inv_sqrt_d);
+                               static_cast<uint16_t *>(dv), ds, int(s.T), int(s.bh()), int(s.causal), c, inv_sqrt_d, d);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
-            using DC = DqDsCfg<D>;
+            using DC = DqDsCfg<D, W>;
             const int64_t dq_blocks = ((s.T + DC::BM - 1) / DC::BM) * s.bh();
-            hipLaunchKernelGGL((bwd_bf16_dq_ds_kernel<D, F>), dim3(unsigned(dq_blocks)), dim3(DC::NW * kWave), 0, stream,
-                               u16(k), ds, static_cast<uint16_t *>(dq), int(s.T), int(s.bh()), int(s.causal), inv_sqrt_d);
+            hipLaunchKernelGGL((bwd_bf16_dq_ds_kernel<D, W, PAD, F>), dim3(unsigned(dq_blocks)), dim3(DC::NW * kWave), 0, stream,
+                               u16(k), ds, static_cast<uint16_t *>(dq), int(s.T), int(s.bh()), int(s.causal), inv_sqrt_d, d);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((bwd_bf16_dkdv_kernel<D, false, F>), dim3(unsigned(kv_blocks)), dim3(KC::NW * kWave), 0,
+    hipLaunchKernelGGL((bwd_bf16_dkdv_kernel<D, W, PAD, false, F>), dim3(unsigned(kv_blocks)), dim3(KC::NW * kWave), 0,
                        stream, u16(q), u16(k), u16(v), u16(dout), nl2, delta, static_cast<uint16_t *>(dk),
-                       static_cast<uint16_t *>(dv), nullptr, int(s.T), int(s.bh()), int(s.causal), c, inv_sqrt_d);
+                       static_cast<uint16_t *>(dv), nullptr, int(s.T), int(s.bh()), int(s.causal), c, inv_sqrt_d, d);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((bwd_bf16_dq_kernel<D, F>), dim3(unsigned(q_blocks)), dim3(QC::NW * kWave), 0, stream, u16(q),
+    hipLaunchKernelGGL((bwd_bf16_dq_kernel<D, W, PAD, F>), dim3(unsigned(q_blocks)), dim3(QC::NW * kWave), 0, stream, u16(q),
                        u16(k), u16(v), u16(dout), nl2, delta, static_cast<uint16_t *>(dq), int(s.T), int(s.bh()),
-                       int(s.causal), c, inv_sqrt_d);
+                       int(s.causal), c, inv_sqrt_d, d);
     return hipGetLastError();
+}
+
+// By tile width, and for rows of another length in place (AttnShape::in_place) by how many of the
+// tile's 32-column head-dim tiles they reach: 96 of the 128 for d in (64, 96].
+template <typename F>
+hipError_t bwd_bf16_width(const void *q, const void *k, const void *v, const void *o, const void *dout,
+                          const float *lse, float *delta, void *dq, void *dk, void *dv, float *nl2, uint16_t *ds,
+                          const AttnShape &s, hipStream_t stream) {
+    auto run = [&](auto fn, uint16_t *tiles) {
+        return fn(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, tiles, s, stream);
+    };
+    if (s.in_place) {
+        switch (s.d) {
+            case 32: return run(bwd_bf16<32, 32, true, F>, nullptr);
+            case 64: return run(bwd_bf16<64, 64, true, F>, nullptr);
+            case 128:
+                return s.scale_dim() <= 96 ? run(bwd_bf16<128, 96, true, F>, ds) : run(bwd_bf16<128, 128, true, F>, ds);
+            default: return hipErrorNotSupported;
+        }
+    }
+    switch (s.d) {
+        case 32: return run(bwd_bf16<32, 32, false, F>, nullptr);
+        case 64: return run(bwd_bf16<64, 64, false, F>, nullptr);
+        case 128: return run(bwd_bf16<128, 128, false, F>, ds);
+        default: return hipErrorNotSupported;
+    }
 }
 
 }  // namespace
@@ -729,12 +764,7 @@ hipError_t launch_bf16_bwd(const void *q, const void *k, const void *v, const vo
     uint16_t *ds = dsb > 0 && extra_bytes >= nl2_bytes(s) + dsb
                        ? reinterpret_cast<uint16_t *>(static_cast<char *>(extra) + nl2_bytes(s))
                        : nullptr;
-    switch (s.d) {
-        case 32: return bwd_bf16<32, Bf16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, nullptr, s, stream);
-        case 64: return bwd_bf16<64, Bf16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, nullptr, s, stream);
-        case 128: return bwd_bf16<128, Bf16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, ds, s, stream);
-        default: return hipErrorNotSupported;
-    }
+    return bwd_bf16_width<Bf16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, ds, s, stream);
 }
 
 hipError_t launch_f16_bwd(const void *q, const void *k, const void *v, const void *o, const void *dout,
@@ -745,12 +775,7 @@ hipError_t launch_f16_bwd(const void *q, const void *k, const void *v, const voi
     uint16_t *ds = dsb > 0 && extra_bytes >= nl2_bytes(s) + dsb
                        ? reinterpret_cast<uint16_t *>(static_cast<char *>(extra) + nl2_bytes(s))
                        : nullptr;
-    switch (s.d) {
-        case 32: return bwd_bf16<32, F16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, nullptr, s, stream);
-        case 64: return bwd_bf16<64, F16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, nullptr, s, stream);
-        case 128: return bwd_bf16<128, F16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, ds, s, stream);
-        default: return hipErrorNotSupported;
-    }
+    return bwd_bf16_width<F16Fmt>(q, k, v, o, dout, lse, delta, dq, dk, dv, nl2, ds, s, stream);
 }
 
 }  // namespace ctattn

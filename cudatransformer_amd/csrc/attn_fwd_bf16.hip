@@ -30,14 +30,14 @@ namespace {
 
 using namespace bf16tile;
 
-template <int D>
+template <int D, int W = D>
 struct FwdBf16Cfg {
     static constexpr int NW = 4;
     static constexpr int BM = 32 * NW;   // query rows per workgroup
     static constexpr int BN = 64;        // keys per block
     static constexpr int KT = BN / 32;   // 32-key tiles per block
-    static constexpr int DT = D / 32;    // 32-wide d tiles of O^T
-    static constexpr int KSTEPS = D / 16;
+    static constexpr int DT = W / 32;    // 32-wide d tiles of O^T
+    static constexpr int KSTEPS = W / 16;
     static constexpr int ROW = 2 * D;             // bytes per tile row
     static constexpr int KB = BN * ROW;           // bytes of a K (or V) block tile
     static constexpr int LDS_BYTES = 4 * KB;      // buffer b: K at 2 b KB, V at 2 b KB + KB
@@ -158,10 +158,10 @@ __device__ __forceinline__ void fwd_bf16_block(FwdBf16State<D> &st, const typena
     }
 }
 
-template <int D, typename F, bool SPLIT>
+template <int D, bool PAD, typename F, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd_bf16_mfma_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
-    uint16_t *__restrict__ o, float *__restrict__ lse, int T, int BH, int causal, float c) {
+    uint16_t *__restrict__ o, float *__restrict__ lse, int T, int BH, int causal, float c, int d) {
     using C = FwdBf16Cfg<D>;
     using V = typename F::vec;
     // SPLIT (causal): 64 query rows per workgroup; waves 2 h and 2 h + 1 (rows q0 .. q0 + 31
@@ -185,7 +185,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int id = blockIdx.x;
     const int bh = id % BH;
     const int qblk = causal ? (nqb - 1 - id / BH) : id / BH;  // causal: longest first
-    const int64_t base = int64_t(bh) * T * D;
+    const int ld = PAD ? d : D;  // elements per row in memory
+    const int64_t base = int64_t(bh) * T * ld;
     const int q0 = qblk * RB;
     const int row = q0 + wl * 32 + col;
     const int wave_first_row = q0 + wl * 32;
@@ -196,7 +197,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int s = 0; s < C::KSTEPS; ++s) {
         u16x8 x = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (row < T) x = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * D + 16 * s + 8 * half);
+        if (row < T && (!PAD || 16 * s + 8 * half < ld))
+            x = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * ld + 16 * s + 8 * half);
         qb[s] = __builtin_bit_cast(V, x);
     }
 
@@ -217,8 +219,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int kb_hi = SPLIT && !hk ? n0 : nkb_all;
     const int iters = SPLIT ? n0 : nkb_all;
     auto issue = [&](int j0, int buf) {
-        load_tile<D, C::BN, GW>(smem + 2 * buf * C::KB, k + base, j0, T, wl, lane);
-        load_tile<D, C::BN, GW>(smem + 2 * buf * C::KB + C::KB, v + base, j0, T, wl, lane);
+        if constexpr (PAD) {
+            load_tile_dma_ld<D, C::BN, GW>(smem + 2 * buf * C::KB, k + base + int64_t(j0) * ld, ld, T - j0, wl, lane);
+            load_tile_dma_ld<D, C::BN, GW>(smem + 2 * buf * C::KB + C::KB, v + base + int64_t(j0) * ld, ld, T - j0, wl,
+                                           lane);
+        } else {
+            load_tile<D, C::BN, GW>(smem + 2 * buf * C::KB, k + base, j0, T, wl, lane);
+            load_tile<D, C::BN, GW>(smem + 2 * buf * C::KB + C::KB, v + base, j0, T, wl, lane);
+        }
     };
 
     if (kb_lo < kb_hi) issue(kb_lo * C::BN, 0);
@@ -277,11 +285,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float l_tot = st.l_run + __shfl_xor(st.l_run, 32, kWave);
     const float inv_l = 1.f / l_tot;
     if (row < T) {
-        uint16_t *orow = o + base + int64_t(row) * D;
+        uint16_t *orow = o + base + int64_t(row) * ld;
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if (PAD && dt * 32 + 8 * g >= ld) continue;
                 u16x4 x;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) x[t] = F::bits(st.oacc[dt][4 * g + t] * inv_l);
@@ -312,24 +321,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Short causal grids take the split kernel when they have at most this many whole
 // workgroups per CU (two per CU made B1 H32 T4096 and B2 H16 T4096 slower, 136 -> 160 us).
 constexpr int kPpSplitWorkgroupsPerCu = 1;
-template <int D>
+template <int D, int W = D>
 struct FwdPpCfg {
     static constexpr int NW = 8;          // waves: group A = 0-3, group B = 4-7
     static constexpr int BM = 32 * NW;    // query rows per workgroup
     static constexpr int BN = 64;         // keys per block
     static constexpr int KT = BN / 32;
-    static constexpr int DT = D / 32;
-    static constexpr int KSTEPS = D / 16;
+    static constexpr int DT = W / 32;
+    static constexpr int KSTEPS = W / 16;
     static constexpr int ROW = 2 * D;
     static constexpr int KB = BN * ROW;   // bytes of one K or V tile
     static constexpr int LDS_BYTES = 4 * KB;  // K0, K1, V0, V1
 };
 
-template <int D, typename F, bool SPLIT>
+template <int D, int W, bool PAD, typename F, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd_bf16_pp_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
-    uint16_t *__restrict__ o, float *__restrict__ lse, int T, int BH, int causal, float c) {
-    using C = FwdPpCfg<D>;
+    uint16_t *__restrict__ o, float *__restrict__ lse, int T, int BH, int causal, float c, int d) {
+    using C = FwdPpCfg<D, W>;
     using V = typename F::vec;
     // SPLIT (causal): the workgroup owns 128 query rows; both groups hold the same rows
     // (waves w and w + 4 the same 32), group A walks the first half of the key blocks and
@@ -353,7 +362,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int id = blockIdx.x;
     const int bh = id % BH;
     const int qblk = causal ? (nqb - 1 - id / BH) : id / BH;  // causal: longest first
-    const int64_t base = int64_t(bh) * T * D;
+    const int ld = PAD ? d : D;  // elements per row in memory
+    const int64_t base = int64_t(bh) * T * ld;
     const int q0 = qblk * RB;
     const int row = q0 + wl * 32 + col;
     const int wave_first_row = q0 + wl * 32;
@@ -363,7 +373,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int s = 0; s < C::KSTEPS; ++s) {
         u16x8 x = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (row < T) x = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * D + 16 * s + 8 * half);
+        if (row < T && (!PAD || 16 * s + 8 * half < ld))
+            x = *reinterpret_cast<const u16x8 *>(q + base + int64_t(row) * ld + 16 * s + 8 * half);
         qb[s] = __builtin_bit_cast(V, x);
     }
 
@@ -404,11 +415,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto issue = [&](int j) __attribute__((always_inline)) {
         const int jk = kb_lo + j + 1, jv = kb_lo + j;  // global key blocks of K_{j+1} and V_j
         if (j + 1 < len)
-            load_tile_dma<D, C::BN, GW>(ktile(j + 1), k + base + int64_t(jk) * C::BN * D, T - jk * C::BN,
-                                        SPLIT ? wl : wave, lane);
+            load_tile_any<D, C::BN, GW, PAD>(ktile(j + 1), k + base + int64_t(jk) * C::BN * ld, ld, T - jk * C::BN,
+                                             SPLIT ? wl : wave, lane);
         if (j < len)
-            load_tile_dma<D, C::BN, GW>(vtile(j), v + base + int64_t(jv) * C::BN * D, T - jv * C::BN,
-                                        SPLIT ? wl : wave, lane);
+            load_tile_any<D, C::BN, GW, PAD>(vtile(j), v + base + int64_t(jv) * C::BN * ld, ld, T - jv * C::BN,
+                                             SPLIT ? wl : wave, lane);
     };
 
     // M(j): O += V_{j-1} P_{j-1} (16 MFMAs at d = 128), then S_j = K_j Q^T (16), as one
@@ -559,8 +570,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // K_0 before the first phase; batch 0 (K_1, V_0) lands during the first iteration.
     if (len > 0)
-        load_tile_dma<D, C::BN, GW>(ktile(0), k + base + int64_t(kb_lo) * C::BN * D, T - kb_lo * C::BN,
-                                    SPLIT ? wl : wave, lane);
+        load_tile_any<D, C::BN, GW, PAD>(ktile(0), k + base + int64_t(kb_lo) * C::BN * ld, ld, T - kb_lo * C::BN,
+                                         SPLIT ? wl : wave, lane);
     wait_loads();
     lds_barrier();
     if (group == 1) {
@@ -615,11 +626,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
     const float inv_l = 1.f / l_tot;
     if (row < T) {
-        uint16_t *orow = o + base + int64_t(row) * D;
+        uint16_t *orow = o + base + int64_t(row) * ld;
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if (PAD && dt * 32 + 8 * g >= ld) continue;
                 u16x4 x;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) x[t] = F::bits(oacc[dt][4 * g + t] * inv_l);
@@ -630,10 +642,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-template <int D, typename F>
+template <int D, int W, bool PAD, typename F>
 hipError_t fwd_bf16_pp(const void *q, const void *k, const void *v, void *o, float *lse, const AttnShape &s,
                        hipStream_t stream) {
-    using C = FwdPpCfg<D>;
+    using C = FwdPpCfg<D, W>;
     const int64_t nqb = (s.T + C::BM - 1) / C::BM;
     const int64_t blocks = nqb * s.bh();
     if (!grid_fits(blocks, C::NW * kWave) || s.T > 2147483647 / D) return hipErrorInvalidValue;
@@ -648,14 +660,14 @@ hipError_t fwd_bf16_pp(const void *q, const void *k, const void *v, void *o, flo
         hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(C::NW * kWave), 0, stream,
                            static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k),
                            static_cast<const uint16_t *>(v), static_cast<uint16_t *>(o), lse, int(s.T), int(s.bh()),
-                           int(s.causal), c);
+                           int(s.causal), c, int(s.scale_dim()));
     };
-    if (split) launch(fwd_bf16_pp_kernel<D, F, true>);
-    else launch(fwd_bf16_pp_kernel<D, F, false>);
+    if (split) launch(fwd_bf16_pp_kernel<D, W, PAD, F, true>);
+    else launch(fwd_bf16_pp_kernel<D, W, PAD, F, false>);
     return hipGetLastError();
 }
 
-template <int D, typename F>
+template <int D, bool PAD, typename F>
 hipError_t fwd_bf16(const void *q, const void *k, const void *v, void *o, float *lse, const AttnShape &s,
                     hipStream_t stream) {
     using C = FwdBf16Cfg<D>;
@@ -673,33 +685,46 @@ hipError_t fwd_bf16(const void *q, const void *k, const void *v, void *o, float 
         hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(C::NW * kWave), 0, stream,
                            static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k),
                            static_cast<const uint16_t *>(v), static_cast<uint16_t *>(o), lse, int(s.T), int(s.bh()),
-                           int(s.causal), c);
+                           int(s.causal), c, int(s.scale_dim()));
     };
-    if (split) launch(fwd_bf16_mfma_kernel<D, F, true>);
-    else launch(fwd_bf16_mfma_kernel<D, F, false>);
+    if (split) launch(fwd_bf16_mfma_kernel<D, PAD, F, true>);
+    else launch(fwd_bf16_mfma_kernel<D, PAD, F, false>);
     return hipGetLastError();
+}
+
+// By tile width, and for rows of another length in place (AttnShape::in_place) by how many of the
+// tile's 32-column head-dim tiles they reach: 96 of the 128 for d in (64, 96].
+template <typename F>
+hipError_t fwd_bf16_width(const void *q, const void *k, const void *v, void *o, float *lse, const AttnShape &s,
+                          hipStream_t stream) {
+    if (s.in_place) {
+        switch (s.d) {
+            case 32: return fwd_bf16<32, true, F>(q, k, v, o, lse, s, stream);
+            case 64: return fwd_bf16<64, true, F>(q, k, v, o, lse, s, stream);
+            case 128:
+                return s.scale_dim() <= 96 ? fwd_bf16_pp<128, 96, true, F>(q, k, v, o, lse, s, stream)
+                                           : fwd_bf16_pp<128, 128, true, F>(q, k, v, o, lse, s, stream);
+            default: return hipErrorNotSupported;
+        }
+    }
+    switch (s.d) {
+        case 32: return fwd_bf16<32, false, F>(q, k, v, o, lse, s, stream);
+        case 64: return fwd_bf16<64, false, F>(q, k, v, o, lse, s, stream);
+        case 128: return fwd_bf16_pp<128, 128, false, F>(q, k, v, o, lse, s, stream);
+        default: return hipErrorNotSupported;
+    }
 }
 
 }  // namespace
 
 hipError_t launch_bf16_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                            const AttnShape &s, hipStream_t stream) {
-    switch (s.d) {
-        case 32: return fwd_bf16<32, Bf16Fmt>(q, k, v, o, lse, s, stream);
-        case 64: return fwd_bf16<64, Bf16Fmt>(q, k, v, o, lse, s, stream);
-        case 128: return fwd_bf16_pp<128, Bf16Fmt>(q, k, v, o, lse, s, stream);
-        default: return hipErrorNotSupported;
-    }
+    return fwd_bf16_width<Bf16Fmt>(q, k, v, o, lse, s, stream);
 }
 
 hipError_t launch_f16_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                           const AttnShape &s, hipStream_t stream) {
-    switch (s.d) {
-        case 32: return fwd_bf16<32, F16Fmt>(q, k, v, o, lse, s, stream);
-        case 64: return fwd_bf16<64, F16Fmt>(q, k, v, o, lse, s, stream);
-        case 128: return fwd_bf16_pp<128, F16Fmt>(q, k, v, o, lse, s, stream);
-        default: return hipErrorNotSupported;
-    }
+    return fwd_bf16_width<F16Fmt>(q, k, v, o, lse, s, stream);
 }
 
 }  // namespace ctattn

@@ -14,6 +14,9 @@ struct AttnShape {
     // Head dim whose 1 / sqrt scales the scores: d itself, unless the tensors are copies
     // zero-padded from a smaller head dim (scale_d), whose scale the kernels must keep.
     int64_t scale_d = 0;
+    // The tensors themselves, not copies: rows of scale_d elements, which the 16-bit kernels of
+    // width d load into zero-filled tiles (scale_d a multiple of 8).
+    bool in_place = false;
     int64_t bh() const { return B * H; }
     int64_t rows() const { return B * H * T; }
     int64_t scale_dim() const { return scale_d > 0 ? scale_d : d; }

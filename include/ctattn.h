@@ -28,7 +28,9 @@
  *     the tensors, still scaled by 1/sqrt(d) (zero columns add nothing to a score; the
  *     padded columns of the outputs are dropped): the backward keeps the copies in its
  *     workspace, the forward takes them from a stream-ordered memory pool the library owns
- *     per device (hipMallocFromPoolAsync / hipFreeAsync on `stream`).  d above 128 runs on
+ *     per device (hipMallocFromPoolAsync / hipFreeAsync on `stream`); bf16 and fp16 with d a
+ *     multiple of 8 and 16-byte-aligned tensors need no copies (the tiles are filled with
+ *     zeros past d) but the same workspace.  d above 128 runs on
  *     MFMA too in fp32, bf16 and fp16 where d is a multiple of 8 (T >= 8; fp32 T >= 32, its
  *     backward T >= 96), with P and dS at fp32 precision, and on the generic kernels
  *     otherwise.  Tensors must be element-aligned; the MFMA kernels at d in {32, 64, 128} and

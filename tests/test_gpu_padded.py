@@ -117,3 +117,42 @@ def test_padded_on_a_side_stream():
     side.synchronize()
     got = {n: t.double().cpu().numpy() for n, t in (("o", o), ("lse", lse), ("dq", dq), ("dk", dk), ("dv", dv))}
     check(got, want, "f32", "side stream d=72")
+
+
+def shifted(t):
+    """The same values two elements past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+    v = buf[2:2 + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+@pytest.mark.parametrize("d", [8, 24, 40, 56, 72, 80, 96, 104, 120])
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("name", ["bf16", "f16"])
+def test_in_place_equals_copies(name, causal, d):
+    """16-bit rows of whole 16-byte chunks are read in place; tensors off a 16-byte boundary still
+    go through the zero-padded copies.  The tiles hold the same values (a width of 96 of 128 skips MFMAs
+    of zeros, which add nothing), so the results are the same bits, but for fp16 gradients: the
+    compiler contracts fp16 products into rowsum(dO O) differently in the two preprocess kernels, a
+    relative e of 1e-6 of delta, which moves a share e / 2u of the values rounded to fp16
+    (u = 2^-11) by one step 2u: sqrt(2 u e) = 3e-5 of the norm, 1e-4 allowed."""
+    for shape in [(1, 2, 1, d), (1, 1, 65, d), (2, 3, 150, d), (1, 2, 513, d)]:
+        say(f"in place {name} causal={causal} {shape}")
+        g = torch.Generator(device=DEV).manual_seed(d)
+        q, k, v, do = (torch.randn(shape, generator=g, device=DEV).to(TORCH[name]) for _ in range(4))
+        o, lse = ct.flash_attn_fwd(q, k, v, causal)
+        o2, lse2 = ct.flash_attn_fwd(shifted(q), k, v, causal)
+        assert torch.equal(o, o2) and torch.equal(lse, lse2)
+        for fastest in (False, True):  # with and without the dS tiles
+            need = ct.bwd_workspace_bytes(q.dtype, *shape, causal, fastest=fastest)
+            ws = [torch.empty(need, dtype=torch.uint8, device=DEV) for _ in range(2)]
+            a = ct.flash_attn_bwd(q, k, v, o, do, lse, causal, workspace=ws[0])
+            b = ct.flash_attn_bwd(shifted(q), k, v, o, do, lse, causal, workspace=ws[1])
+            torch.cuda.synchronize()
+            for x, y in zip(a, b):
+                if name == "bf16":
+                    assert torch.equal(x, y), fastest
+                else:
+                    scale = max(y.double().norm(), b[2].double().norm())  # dQ, dK of one key vanish
+                    assert (x.double() - y.double()).norm() <= 1e-4 * scale, fastest
