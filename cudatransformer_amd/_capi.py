@@ -147,8 +147,13 @@ def set_policy(policy: int) -> int:
 
 
 def _stream_handle(stream) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    """hipStream_t of `stream`, or of the current stream.  The current one is read as a raw handle:
+    torch.cuda.current_stream() builds a Stream object for it, 2.7 us of a small call's 12."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check_qkv(name, *ts):
@@ -157,12 +162,13 @@ def _check_qkv(name, *ts):
         raise ValueError(f"{name}: tensors must be [B, H, T, d], got {tuple(ref.shape)}")
     if ref.dtype not in _DTYPE_CODE:
         raise ValueError(f"{name}: dtype {ref.dtype} unsupported (float32, bfloat16, float16, float64)")
+    shape, dtype = ref.shape, ref.dtype
     for t in ts:
         if not t.is_cuda:
             raise ValueError(f"{name}: tensors must live on the GPU")
-        if t.shape != ref.shape or t.dtype != ref.dtype:
+        if t.shape != shape or t.dtype != dtype:
             raise ValueError(f"{name}: shape/dtype mismatch {tuple(t.shape)} {t.dtype} vs "
-                             f"{tuple(ref.shape)} {ref.dtype}")
+                             f"{tuple(shape)} {dtype}")
         if not t.is_contiguous():
             raise ValueError(f"{name}: tensors must be contiguous")
 
@@ -171,20 +177,21 @@ def flash_attn_fwd(q, k, v, causal: bool = False, out=None, lse=None, stream=Non
     """O, LSE = attention(q, k, v); q, k, v contiguous [B, H, T, d] on the GPU."""
     _check_qkv("flash_attn_fwd", q, k, v)
     b, h, t, d = q.shape
+    stat = _stat_dtype(q.dtype)
     if out is None:
         out = torch.empty_like(q)
-    stat = _stat_dtype(q.dtype)
+    else:
+        _check_qkv("flash_attn_fwd", q, out)
     if lse is None:
-        lse = torch.empty((b, h, t), dtype=stat, device=q.device)
-    _check_qkv("flash_attn_fwd", q, out)
-    if lse.dtype != stat or tuple(lse.shape) != (b, h, t) or not lse.is_contiguous():
+        lse = q.new_empty((b, h, t), dtype=stat)
+    elif lse.dtype != stat or tuple(lse.shape) != (b, h, t) or not lse.is_contiguous():
         raise ValueError(f"flash_attn_fwd: lse must be contiguous {stat} [B, H, T]")
     lib = load()
     code = _DTYPE_CODE[q.dtype]
     need = lib.ctattn_fwd_workspace_bytes(code, b, h, t, d)
     if need < 0:
         raise RuntimeError(f"ctattn_fwd_workspace_bytes failed: {last_error()}")
-    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
+    ws = q.new_empty(need, dtype=torch.uint8) if need > 0 else None
     rc = lib.ctattn_fwd_ws(code, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                            _ptr(ws), need, b, h, t, d, int(bool(causal)), _stream_handle(stream))
     _check(rc, "ctattn_fwd_ws")
@@ -211,16 +218,18 @@ def flash_attn_bwd(q, k, v, o, do, lse, causal: bool = False, dq=None, dk=None, 
     bwd_workspace_bytes(..., fastest=True)) lets the bf16 / fp16 d = 128 path store dS."""
     _check_qkv("flash_attn_bwd", q, k, v, o, do)
     b, h, t, d = q.shape
+    given = [g for g in (dq, dk, dv) if g is not None]
+    if given:
+        _check_qkv("flash_attn_bwd", q, *given)
     dq = torch.empty_like(q) if dq is None else dq
     dk = torch.empty_like(q) if dk is None else dk
     dv = torch.empty_like(q) if dv is None else dv
-    _check_qkv("flash_attn_bwd", q, dq, dk, dv)
     stat = _stat_dtype(q.dtype)
     if lse.dtype != stat or tuple(lse.shape) != (b, h, t) or not lse.is_contiguous():
         raise ValueError(f"flash_attn_bwd: lse must be contiguous {stat} [B, H, T]")
     need = bwd_workspace_bytes(q.dtype, b, h, t, d, causal)
     if workspace is None:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
+        workspace = q.new_empty(max(need, 1), dtype=torch.uint8)
     if workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"flash_attn_bwd: workspace too small ({need} bytes needed)")
     rc = load().ctattn_bwd(_DTYPE_CODE[q.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(),
@@ -643,10 +652,7 @@ def adam_update(param, grad, m, v, step: int, lr=1e-3, beta1=0.9, beta2=0.999, e
 
 
 def _ptr_table(ts):
-    arr = (ctypes.c_void_p * max(len(ts), 1))()
-    for i, t in enumerate(ts):
-        arr[i] = None if t is None else t.data_ptr()
-    return arr
+    return (ctypes.c_void_p * max(len(ts), 1))(*[None if t is None else t.data_ptr() for t in ts])
 
 
 def adam_update_multi(params, grads, ms, vs, step: int, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8,
