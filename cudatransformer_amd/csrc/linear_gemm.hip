@@ -1485,10 +1485,13 @@ using lin::F32Fmt;
 template <typename F>
 struct Tables {
     static constexpr CfgInfo fwd[] = {cfg_info<F, true, true, 2, 1, 4, 2>(), cfg_info<F, true, true, 2, 1, 1, 2>(),
-                                      cfg_info<F, true, true, 2, 1, 1, 3>()};
-    // An M/N-contiguous B is read through the two-tile interleaved operand (32 x 64 tiles).
+                                      cfg_info<F, true, true, 2, 1, 1, 3>(), cfg_info<F, true, true, 1, 1, 8, 2>(),
+                                      cfg_info<F, true, true, 1, 1, 4, 2>()};
+    // An M/N-contiguous B is read through the two-tile interleaved operand (32 x 64 tiles), in
+    // small grids through the one-tile one.
     static constexpr CfgInfo dx[] = {cfg_info<F, true, false, 1, 2, 4, 2>(), cfg_info<F, true, false, 1, 2, 1, 2>(),
-                                     cfg_info<F, true, false, 1, 2, 1, 3>()};
+                                     cfg_info<F, true, false, 1, 2, 1, 3>(), cfg_info<F, true, false, 1, 1, 8, 2>(),
+                                     cfg_info<F, true, false, 1, 1, 4, 2>()};
     static constexpr CfgInfo dw[] = {cfg_info<F, false, false, 1, 2, 4, 2>(), cfg_info<F, false, false, 2, 2, 8, 2>(),
                                      cfg_info<F, false, false, 1, 2, 8, 2>()};
 };
@@ -1496,12 +1499,27 @@ struct Tables {
 // 64 x 32 tiles of fp32 leave the 16-bit kernels bound by L2 and LDS bandwidth).
 template <typename F>
 struct Tables16 {
-    static constexpr CfgInfo fwd[] = {cfg_info<F, true, true, 4, 2, 1, 3>(), cfg_info<F, true, true, 2, 2, 4, 2>()};
-    static constexpr CfgInfo dx[] = {cfg_info<F, true, false, 2, 4, 1, 2>(), cfg_info<F, true, false, 2, 2, 4, 2>()};
+    static constexpr CfgInfo fwd[] = {cfg_info<F, true, true, 4, 2, 1, 3>(), cfg_info<F, true, true, 2, 2, 4, 2>(),
+                                      cfg_info<F, true, true, 1, 1, 4, 2>()};
+    static constexpr CfgInfo dx[] = {cfg_info<F, true, false, 2, 4, 1, 2>(), cfg_info<F, true, false, 2, 2, 4, 2>(),
+                                     cfg_info<F, true, false, 1, 1, 4, 2>()};
     static constexpr CfgInfo dw[] = {cfg_info<F, false, false, 2, 2, 2, 2>()};
 };
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Forward / dX products whose larger tiles would leave CUs without a workgroup: 32 x 32 tiles.
+// Up to `any_k` of them (fp32 256, one per CU, of 8 waves; 16-bit 384, of 4 waves) at any
+// contraction, up to 768 at a contraction of at most 512, where the shorter chain of each wave
+// outweighs the operands read twice as often.  Measured, us, larger tiles -> these:
+//   fp32    256 x 384, K 384   7.1 -> 5.3     512 x 512, K 2048   21.1 -> 13.1
+//           2048 x 384, K 384 (768 tiles, of 4 waves) 10.3 -> 9.1; 1024 x 384, K 1536 (384) 17.6 / 18.7
+//   16-bit  256 x 384, K 384   6.0 -> 3.7     1024 x 384, K 1536   10.1 -> 7.5
+//           2048 x 384, K 384  6.2 -> 5.4     2048 x 512, K 2048 (1024 tiles) 12.1 / 18.0
+bool small_grid(const LinGemm &g, int64_t any_k) {
+    const int64_t t32 = cdiv(g.M, 32) * cdiv(g.N, 32) * g.nbatch;
+    return t32 <= any_k || (t32 <= 768 && g.K * g.nseg <= 512);
+}
 
 // Chooses a configuration (index into the layout's table) and a K split count.
 // allow_split: the caller has workspace for split-K partials.
@@ -1512,18 +1530,19 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //     workgroups otherwise, each wave keeping >= 8 K chunks.
 //   * Otherwise 64 x 32 (forward) or 32 x 64 (dX) tiles: 4 waves (K split inside the
 //     workgroup) while there are fewer than 3072 tiles, else one wave per tile (3 stages once
-//     K reaches 64 chunks, else 2).
+//     K reaches 64 chunks, else 2).  Small grids: see small_grid.
 // bf16 / fp16:
 //   * weight gradients: 64 x 64 tiles of 2 waves, K split across workgroups below 512 tiles
 //     (up to 1024 workgroups, each wave keeping >= 12 K chunks);
 //   * the shared-tile kernel where shared_plan takes the product (chosen before this plan);
 //   * otherwise, with at least 1024 64 x 64 tiles and 24 K chunks: one wave per 128 x 64
-//     (forward) or 64 x 128 (dX) tile; else 64 x 64 tiles of 4 waves.
+//     (forward) or 64 x 128 (dX) tile; else 64 x 64 tiles of 4 waves.  Small grids: see
+//     small_grid.
 lin::Plan plan(const LinGemm &g, bool allow_split) {
     const int64_t chunks = g.K / lin::chunk_elems(g.dtype) * g.nseg;
     if (g.dtype != 0) {
         const int64_t t64 = cdiv(g.M, 64) * cdiv(g.N, 64) * g.nbatch;
-        if (g.a_kc) return lin::Plan{t64 >= 1024 && chunks >= 24 ? 0 : 1, 1};
+        if (g.a_kc) return lin::Plan{small_grid(g, 384) ? 2 : t64 >= 1024 && chunks >= 24 ? 0 : 1, 1};
         if (t64 >= 512 || !allow_split) return lin::Plan{0, 1};
         const int64_t sp = std::min<int64_t>(cdiv(1024, t64), chunks / 24);
         return lin::Plan{0, int(std::max<int64_t>(1, std::min<int64_t>(sp, 16)))};
@@ -1536,6 +1555,7 @@ lin::Plan plan(const LinGemm &g, bool allow_split) {
         sp = allow_split ? std::max<int64_t>(1, std::min<int64_t>(sp, 16)) : 1;
         return lin::Plan{few ? 2 : 0, int(sp)};
     }
+    if (small_grid(g, 256)) return lin::Plan{cdiv(g.M, 32) * cdiv(g.N, 32) * g.nbatch <= 256 ? 3 : 4, 1};
     const int64_t tiles = cdiv(g.M, 64) * cdiv(g.N, 32) * g.nbatch;
     return lin::Plan{tiles < 3072 ? 0 : chunks >= 64 ? 2 : 1, 1};
 }
