@@ -8,7 +8,9 @@
 //   * one workgroup = 4 waves = BM = 128 query rows of one (batch, head); each wave owns
 //     32 rows and keeps them for the whole key loop.  A causal grid (d <= 64) too short to
 //     fill the chip twice over instead runs split workgroups: 64 rows, the key range halved
-//     between two wave pairs, merged through LDS (fwd_split).
+//     between two wave pairs, merged through LDS (fwd_split).  A grid of about one or two
+//     32-row blocks per CU gives each block a workgroup whose waves share out its keys
+//     (fwd_f32_small_kernel).
 //   * the key loop walks BN-key blocks.  K and V blocks go straight from global memory to
 //     LDS (global_load_lds_dwordx4, no staging registers), double-buffered: the next
 //     block's loads are in flight during the current block's MFMAs, one barrier per block.
@@ -416,6 +418,133 @@ __device__ __forceinline__ void fwd_split(float *k_lds, float *v_lds,
     }
 }
 
+// Small grids: 32 query rows per workgroup, wave w takes the 32-key blocks w, w + NW, ... of
+// their range and the waves' (O^T, m, l) are merged through LDS.  K and V go straight from
+// global memory into MFMA operand registers -- no tile is shared between waves, so the key
+// loop has no barrier -- with V's loads in flight behind the S product and the next block's K
+// behind the softmax and the P V product.
+template <int D>
+struct SmallCfg {
+    static constexpr int NW = D == 128 ? 4 : 8;  // 4 waves: 512 registers each for d = 128's operands
+    static constexpr int DT = D / 32;
+};
+
+template <int D>
+__global__ __launch_bounds__(SmallCfg<D>::NW *kWave) __attribute__((amdgpu_waves_per_eu(SmallCfg<D>::NW / 4, SmallCfg<D>::NW / 4)))
+void fwd_f32_small_kernel(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
+                          float *__restrict__ o, float *__restrict__ lse, int T, int BH, int causal, float qscale) {
+    using C = SmallCfg<D>;
+    constexpr int NW = C::NW;
+    __shared__ __attribute__((aligned(16))) floatx4 ot[NW][D / 8][kWave];  // O^T register groups of every wave
+    __shared__ float ml[NW][2][kWave];
+
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int col = lane & 31, half = lane >> 5;
+    const int nrb = (T + 31) / 32;
+    const int id = blockIdx.x, bh = id % BH;
+    const int rb = causal ? nrb - 1 - id / BH : id / BH;  // causal: longest first
+    const int row = rb * 32 + col;
+    const int64_t base = int64_t(bh) * T * D;
+    const int nk = causal ? rb + 1 : nrb;
+
+    float kreg[D / 2], vreg[C::DT * 16];
+    auto load_k = [&](int kb) __attribute__((always_inline)) {  // keys past T re-read key T - 1 (masked)
+        const float *kp = k + base + int64_t(min(kb * 32 + col, T - 1)) * D + 4 * half;
+#pragma unroll
+        for (int m = 0; m < D / 8; ++m) {
+            const floatx4 x = *reinterpret_cast<const floatx4 *>(kp + 8 * m);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) kreg[4 * m + t] = x[t];
+        }
+    };
+    if (wave < nk) load_k(wave);
+    float qreg[D / 2];
+    load_qT<D>(qreg, q, base, row, T, qscale, half);
+
+    FwdState<D> st;
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) st.oacc[dt] = zero16();
+    st.m_run = -INFINITY;
+    st.l_run = 0.f;
+
+    for (int kb = wave; kb < nk; kb += NW) {
+        const int j0 = kb * 32;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const float *vp = v + base + int64_t(min(j0 + kstep_index(s, half), T - 1)) * D + col;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) vreg[dt * 16 + s] = vp[dt * 32];
+        }
+        floatx16 sacc = zero16();
+#pragma unroll
+        for (int i = 0; i < D / 2; ++i) sacc = mfma32x32x2(kreg[i], qreg[i], sacc);
+        if (kb + NW < nk) load_k(kb + NW);
+
+        if (j0 + 32 > T || (causal && kb == rb)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = j0 + acc_row(r, half);
+                if (key >= T || (causal && key > row)) sacc[r] = -INFINITY;
+            }
+        }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sacc[r]);
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
+        if (__any(mloc > st.m_run + kRescaleThreshold)) {
+            const float m_new = fmaxf(st.m_run, mloc);
+            const float resc = fast_exp2(st.m_run - m_new);  // 0 on the first block (m_run = -inf)
+            st.m_run = m_new;
+            st.l_run *= resc;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) st.oacc[dt] *= resc;
+        }
+        float psum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            sacc[r] = fast_exp2(sacc[r] - st.m_run);
+            psum += sacc[r];
+        }
+        st.l_run += psum;
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) st.oacc[dt] = mfma32x32x2(vreg[dt * 16 + s], sacc[s], st.oacc[dt]);
+    }
+
+    // Merge, all relative to m = the largest of the waves' running maxima: wave 0 always holds
+    // key 0 of its rows, a wave without a block has m = -inf and weight 0.  Each wave adds up
+    // the 4-column groups wave, wave + NW, ... of every row in wave order and stores them.
+    ml[wave][0][lane] = st.m_run;
+    ml[wave][1][lane] = st.l_run;
+    __syncthreads();
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, ml[w][0][lane]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) l += ml[w][1][lane] * fast_exp2(ml[w][0][lane] - m);
+    l += __shfl_xor(l, 32, kWave);
+    const float a = fast_exp2(st.m_run - m);
+#pragma unroll
+    for (int g = 0; g < D / 8; ++g) {
+        floatx4 x;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = st.oacc[g / 4][4 * (g % 4) + t] * a;
+        ot[wave][g][lane] = x;
+    }
+    __syncthreads();
+    const float inv_l = 1.f / l;
+    if (row < T) {
+        const int nw = min(NW, nk);  // the waves that had a block
+        for (int g = wave; g < D / 8; g += NW) {
+            floatx4 x = ot[0][g][lane];
+            for (int w = 1; w < nw; ++w) x += ot[w][g][lane];
+            *reinterpret_cast<floatx4 *>(o + base + int64_t(row) * D + 8 * g + 4 * half) = x * inv_l;
+        }
+        if (lse != nullptr && wave == 0 && half == 0) lse[int64_t(bh) * T + row] = (m + __log2f(l)) * kLn2;
+    }
+}
+
 template <int D, int BN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void fwd_f32_mfma_kernel(
     const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, float *__restrict__ o,
@@ -441,16 +570,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     fwd_whole<D, BN>(&k_lds[0][0], &v_lds[0][0], q, k, v, o, lse, T, bh, qb, causal, qscale, wave, lane);
 }
 
-// Split workgroups pay for themselves when the causal grid of whole 128-row blocks has no more
-// workgroups than the chip has slots (two per CU): then the longest blocks are the whole
-// kernel, and cutting every block into two 64-row workgroups with halved key ranges shortens
-// them four times over.  Measured (B x H x T, d = 64): 1x4x2048 83.6 -> 50.7 us, 2x16x1024
-// 76.7 -> 61.7, 8x12x512 55.6 -> 47.9; at 768 and more whole blocks splitting is within
+// Of the grids left by the 32-row kernel (below), split workgroups pay for themselves when the
+// causal grid of whole 128-row blocks has no more workgroups than the chip has slots (two per
+// CU): then the longest blocks are the whole kernel, and cutting every block into two 64-row
+// workgroups with halved key ranges shortens them four times over.  Measured (B x H x T,
+// d = 64): 2x16x1024 76.7 -> 61.7 us, 8x12x512 55.6 -> 47.9; at 768 and more whole blocks splitting is within
 // +-3 % (8x12x1024 133.4 / 132.1, 1x12x8192 859.5 / 877.4, 32x12x1024 479.4 / 494.2), so
 // those keep whole blocks.
 bool fwd_use_split(const AttnShape &s, hipStream_t stream) {
     const int cus = device_cus(stream);
     return cus > 0 && (s.T + 127) / 128 * s.bh() <= int64_t(2) * cus;
+}
+
+// The 32-row kernel, by its workgroups per CU: one at any T above a single key block (there is
+// nothing to split up to T = 32: d = 128 T 32 8.0 / 10.3 us), two once T = 512 amortises the
+// merge, and where a row of operands is 128 wide -- the whole kernel has no split form there --
+// or 32 wide, up to three, causal d = 128 up to four.  Measured, us, whole or split -> this
+// (B x H x T):
+//   d 32    1x4x128 causal 6.7 -> 5.2; 1x8x1024 43.3 -> 16.9, causal 26.9 -> 15.7; 1x16x1024
+//           (two per CU) 43.2 -> 30.1; 4x16x256 causal 9.8 / 10.6; 1x28x1024 (four) 45.6 / 53.1
+//   d 64    1x6x256 causal 14.2 -> 11.4; 1x4x2048 142 -> 59.8, causal 80.3 -> 55.8; 2x16x512
+//           38.6 -> 36.6, causal 24.2 / 24.6; 1x24x1024 (three) 73.7 / 90.9, causal 54.4 / 55.8
+//   d 128   1x12x512 73.4 -> 27.1; 1x24x1024 (three) 148 -> 126, causal 148 -> 83.9; 2x16x1024
+//           (four) 150 / 168, causal 149 -> 107; 8x16x1024 (16) 529 / 671, causal 319 / 424
+bool fwd_use_small(const AttnShape &s, hipStream_t stream) {
+    const int64_t cus = device_cus(stream), wgs = (s.T + 31) / 32 * s.bh();
+    if (s.T <= 32) return false;
+    if (wgs <= cus) return true;
+    if (wgs <= 2 * cus) return s.T >= (s.d == 128 ? 128 : 512);
+    if (s.d == 128) return s.T >= 512 && wgs <= (s.causal ? 4 : 3) * cus;
+    return s.d == 32 && s.T >= 1024 && wgs <= 3 * cus;
 }
 
 template <int D, int BN>
@@ -461,6 +610,12 @@ hipError_t fwd_f32(const float *q, const float *k, const float *v, float *o, flo
     const int64_t blocks = nqb * s.bh();
     if (!grid_fits(blocks, C::NW * kWave) || s.T > 2147483647 / D) return hipErrorInvalidValue;
     const float qscale = kLog2e / sqrtf(float(s.scale_dim()));
+    if (fwd_use_small(s, stream)) {
+        hipLaunchKernelGGL((fwd_f32_small_kernel<D>), dim3(unsigned((s.T + 31) / 32 * s.bh())),
+                           dim3(SmallCfg<D>::NW * kWave), 0, stream, q, k, v, o, lse, int(s.T), int(s.bh()),
+                           int(s.causal), qscale);
+        return hipGetLastError();
+    }
     const int split = BN == 64 && s.causal && fwd_use_split(s, stream);
     const int64_t grid = split ? (s.T + 63) / 64 * s.bh() : blocks;
     if (!grid_fits(grid, C::NW * kWave)) return hipErrorInvalidValue;
