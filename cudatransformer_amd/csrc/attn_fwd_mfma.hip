@@ -493,16 +493,18 @@ void fwd_f32_small_kernel(const float *__restrict__ q, const float *__restrict__
         mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
         if (__any(mloc > st.m_run + kRescaleThreshold)) {
             const float m_new = fmaxf(st.m_run, mloc);
-            const float resc = fast_exp2(st.m_run - m_new);  // 0 on the first block (m_run = -inf)
+            const float resc = m_new == -INFINITY ? 0.f : fast_exp2(st.m_run - m_new);  // 0 on the first block
             st.m_run = m_new;
             st.l_run *= resc;
 #pragma unroll
             for (int dt = 0; dt < C::DT; ++dt) st.oacc[dt] *= resc;
         }
+        // A block of nothing but -inf scores (infinite keys) adds nothing, also as a wave's first.
+        const float m_use = st.m_run == -INFINITY ? 0.f : st.m_run;
         float psum = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            sacc[r] = fast_exp2(sacc[r] - st.m_run);
+            sacc[r] = fast_exp2(sacc[r] - m_use);
             psum += sacc[r];
         }
         st.l_run += psum;

@@ -1023,14 +1023,17 @@ int ctattn_softmax_fwd(int dtype, const void *z, void *p, int64_t N, int64_t V, 
                                    1.f / float(temperature));
                 return hipGetLastError();
             };
-            if (V <= 64 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<1>{});
-            if (V <= 128 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<2>{});
-            if (V <= 512 * EPC) return rows(ctattn::Int<4>{}, ctattn::Int<2>{});
-            if (V <= 1024 * EPC) return rows(ctattn::Int<4>{}, ctattn::Int<4>{});
-            if (V <= 4096 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<4>{});
-            if (V <= 8192 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<8>{});
+            // A temperature past fp32's range makes every class alike (a factor of 0), which the fill of
+            // -inf past V would turn into NaN: the general kernel's.
+            const bool fits = 1.f / float(temperature) > 0.f;
+            if (fits && V <= 64 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<1>{});
+            if (fits && V <= 128 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<2>{});
+            if (fits && V <= 512 * EPC) return rows(ctattn::Int<4>{}, ctattn::Int<2>{});
+            if (fits && V <= 1024 * EPC) return rows(ctattn::Int<4>{}, ctattn::Int<4>{});
+            if (fits && V <= 4096 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<4>{});
+            if (fits && V <= 8192 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<8>{});
             if constexpr (sizeof(T) == 4)
-                if (V <= 16384 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<16>{});
+                if (fits && V <= 16384 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<16>{});
         }
         hipLaunchKernelGGL(ctattn::softmax_fwd_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st,
                            static_cast<const T *>(z), static_cast<T *>(p), N, int(V), A(1) / A(temperature));

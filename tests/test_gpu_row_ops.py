@@ -87,3 +87,13 @@ def test_softmax_and_gradient_edges(name, v):
     onehot[ok.nonzero()[:, 0], t[ok].long()] = 1.0
     ref = (p.double() - onehot) * ok[:, None] / (n * 0.7)
     assert ((dz.double() - ref).abs() <= TOL[name] * ref.abs() + floor + 1e-7).all()
+
+
+@pytest.mark.parametrize("temperature", [3e38, 1e39, float("inf")])
+@pytest.mark.parametrize("v", [5, 129, 3001])
+def test_softmax_temperatures_past_fp32(v, temperature):
+    """A temperature whose fp32 reciprocal is subnormal or 0: every class alike, at lengths off the granules."""
+    print(f"softmax V={v} temperature={temperature}", flush=True)
+    for name, dt in DT.items():
+        p = _capi.softmax_fwd(rnd((3, v), dt, 7), temperature)
+        assert ((p.double() * v - 1).abs() <= TOL[name] + (2.0 ** -25 * v if name == "f16" else 0)).all()

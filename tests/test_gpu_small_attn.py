@@ -54,3 +54,22 @@ def test_small_grid_forward(d, causal, bht):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
     for buf, x in ops + outs:
         assert torch.isnan(buf[:PAD]).all() and torch.isnan(buf[PAD + x.numel():]).all()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_small_grid_forward_infinite_keys(d, causal):
+    """Key blocks whose every score is -inf add nothing, also where they are the first block of a wave."""
+    b, h, t = 1, 2, 400
+    print(f"small grid forward, infinite keys d={d} causal={causal}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v = [torch.randn((b, h, t, d), generator=g, device="cuda") for _ in range(3)]
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, :, 32:96, 0] = float("-inf")
+    k[:, :, 352:, 0] = float("-inf")
+    o, lse = _capi.flash_attn_fwd(q, k, v, causal)
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) / math.sqrt(d)
+    if causal:
+        s = s.masked_fill(torch.ones(t, t, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    assert (o.double() - torch.softmax(s, -1) @ v.double()).abs().max() <= 2e-5
+    assert (lse.double() - torch.logsumexp(s, -1)).abs().max() <= 1e-5
