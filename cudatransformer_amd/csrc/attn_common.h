@@ -17,13 +17,16 @@ struct bf16_t {
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16_t x) { return __uint_as_float(uint32_t(x.bits) << 16); }
 
-// Round-to-nearest-even fp32 -> bf16 (NaN stays a quiet NaN).
-__device__ __forceinline__ bf16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return bf16_t{uint16_t((u >> 16) | 0x40)};
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return bf16_t{uint16_t(u >> 16)};
+// Round-to-nearest-even fp32 -> bf16 (NaN stays a quiet NaN): the hardware conversion, one
+// v_cvt_pk_bf16_f32 for two values.  The same rounding written out in integers took a branch per
+// element for the NaN, in every bf16 store: MLP 8192 x 1024 x 4096 fwd+bwd 651 -> 621 us, attention
+// layer of 8 x 1024 rows 522 -> 508, LayerNorm 8192 x 2048 48.2 -> 44.5, all outputs bitwise equal.
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t f32_to_bf16x2(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
 }
+__device__ __forceinline__ bf16_t f32_to_bf16(float f) { return bf16_t{uint16_t(f32_to_bf16x2(f, f))}; }
 
 // IEEE binary16, carried as its raw 16-bit pattern; arithmetic is fp32 (hardware conversion,
 // round to nearest even).

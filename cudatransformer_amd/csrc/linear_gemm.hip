@@ -87,6 +87,8 @@ typedef u16x4 u16x4u __attribute__((aligned(2)));
 typedef floatx4 floatx4u __attribute__((aligned(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4u __attribute__((aligned(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2u __attribute__((aligned(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -159,7 +161,10 @@ struct H16Fmt {
     }
     __device__ static void store(char *p, float x) { *reinterpret_cast<uint16_t *>(p) = narrow(x); }
     __device__ static void store4(char *p, floatx4 x) {
-        *reinterpret_cast<u16x4u *>(p) = u16x4{narrow(x[0]), narrow(x[1]), narrow(x[2]), narrow(x[3])};
+        if constexpr (BF)
+            *reinterpret_cast<u32x2u *>(p) = u32x2{f32_to_bf16x2(x[0], x[1]), f32_to_bf16x2(x[2], x[3])};
+        else
+            *reinterpret_cast<u16x4u *>(p) = u16x4{narrow(x[0]), narrow(x[1]), narrow(x[2]), narrow(x[3])};
     }
     // Sum of the 16-byte MFMA operand (8 16-bit values).
     __device__ static float sum(floatx4 v) {

@@ -43,9 +43,11 @@ template <typename T> struct Gran {
         gran_raw x = {0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < EPC; ++e) {
-            if constexpr (sizeof(T) == 2) {
+            if constexpr (std::is_same_v<T, bf16_t>) {
+                if (e % 2 == 0) x[e / 2] = f32_to_bf16x2(v[e], v[e + 1]);
+            } else if constexpr (sizeof(T) == 2) {
                 float f = v[e];
-                if constexpr (std::is_same_v<T, f16_t>) asm volatile("" : "+v"(f));
+                asm volatile("" : "+v"(f));
                 x[e / 2] |= uint32_t(from_f32<T>(f).bits) << (16 * (e & 1));
             } else {
                 x[e] = __float_as_uint(v[e]);
