@@ -20,7 +20,7 @@ __device__ __forceinline__ float to_f32(bf16_t x) { return __uint_as_float(uint3
 // Round-to-nearest-even fp32 -> bf16 (NaN stays a quiet NaN): the hardware conversion, one
 // v_cvt_pk_bf16_f32 for two values.  The same rounding written out in integers took a branch per
 // element for the NaN, in every bf16 store: MLP 8192 x 1024 x 4096 fwd+bwd 651 -> 621 us, attention
-// layer of 8 x 1024 rows 522 -> 508, LayerNorm 8192 x 2048 48.2 -> 44.5, all outputs bitwise equal.
+// layer of 8 x 1024 rows 528 -> 513, LayerNorm 8192 x 2048 48.2 -> 44.5, all outputs bitwise equal.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t f32_to_bf16x2(float lo, float hi) {

@@ -458,11 +458,22 @@ __global__ __launch_bounds__(256) void softmax_fwd_kernel(const T *__restrict__ 
     for (int c = lane; c < V; c += kWave) st(pr, c, acc_exp((ld(zr, c) - m) * inv_temp) * inv_s);
 }
 
+// e^x for x <= 0 (-inf gives 0, NaN stays): x log2(e) in two terms, its nearest integer r taken off
+// exactly and put back by ldexp, so subnormal results are kept.  No overflow to guard against: 8
+// operations where expf takes 13.  r stops at -200, below which 2^f 2^r is 0 anyway, so that -inf has
+// a finite one.  log2(e) = kHi + kLo, both positive.
+__device__ __forceinline__ float exp_neg(float x) {
+    constexpr float kHi = 1.44269502162933349609375f, kLo = 1.92596299112661746887e-8f;
+    const float r = fmaxf(rintf(x * kHi), -200.f);
+    return ldexpf(__builtin_amdgcn_exp2f(fmaf(x, kLo, fmaf(x, kHi, -r))), int(r));
+}
+
 // The same with the row in registers (z read once, one exponential per element): GW waves per row,
 // CPT granules per lane (V <= 64 GW CPT EPC); GW = 1: four rows per workgroup.  Bound by HBM and, in
 // the widest rows, by one row filling the registers of a CU, so that its loads, exponentials and
-// stores follow one another: bf16 2048 x 50257 903 -> 156 us (keeping the 16-bit scores instead,
-// two rows per CU and every exponential twice: 153).
+// stores follow one another: bf16 2048 x 50257 903 -> 127 us (150 with expf and the last granule
+// loaded element by element; keeping the 16-bit scores instead, two rows per CU and every
+// exponential twice, did not help).
 template <typename T, int GW, int CPT>
 __global__ __launch_bounds__(GW == 1 ? 256 : kWave *GW) void softmax_fwd_rows_kernel(const T *z, T *p, int64_t N, int V,
                                                                                    float inv_temp) {
@@ -476,7 +487,7 @@ __global__ __launch_bounds__(GW == 1 ? 256 : kWave *GW) void softmax_fwd_rows_ke
     float v[CPT][G::EPC], m = -INFINITY;
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-        const gran_raw raw = G::load(zr, (lane + kWave * GW * j) * G::EPC, V, -INFINITY);
+        const gran_raw raw = G::load_tail(zr, (lane + kWave * GW * j) * G::EPC, V, -INFINITY);
 #pragma unroll
         for (int e = 0; e < G::EPC; ++e) v[j][e] = G::get(raw, e);
     }
@@ -490,7 +501,7 @@ __global__ __launch_bounds__(GW == 1 ? 256 : kWave *GW) void softmax_fwd_rows_ke
     for (int j = 0; j < CPT; ++j)
 #pragma unroll
         for (int e = 0; e < G::EPC; ++e) {
-            v[j][e] = acc_exp((v[j][e] - m) * inv_temp);
+            v[j][e] = exp_neg((v[j][e] - m) * inv_temp);
             s += v[j][e];
         }
     const float inv_s = 1.f / row_sum<GW>(s, red[1]);

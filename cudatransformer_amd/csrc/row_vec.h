@@ -32,6 +32,31 @@ template <typename T> struct Gran {
         }
         return x;
     }
+    // The same; the granule that crosses the end is read as the row's last EPC elements and shifted
+    // down past those before c0: one access beside the others', where element by element takes a
+    // chain of them.  For rows of many granules and mostly odd lengths (in the LayerNorm backward the
+    // shift costs 40 registers).
+    __device__ static __forceinline__ gran_raw load_tail(const T *row, int c0, int D, float fill) {
+        if (D < EPC) return load(row, c0, D, fill);
+        uint32_t pat;  // one dword of fill
+        if constexpr (sizeof(T) == 2) pat = uint32_t(from_f32<T>(fill).bits) * 0x10001u;
+        else pat = __float_as_uint(fill);
+        if (c0 >= D) return gran_raw{pat, pat, pat, pat};
+        const gran_raw x = *reinterpret_cast<const raw_t *>(row + min(c0, D - EPC));
+        if (c0 + EPC <= D) return x;
+        const int bits = 8 * int(sizeof(T)) * (c0 + EPC - D);  // one element .. 128 less one
+        const uint64_t f = uint64_t(pat) << 32 | pat;
+        uint64_t lo = uint64_t(x[1]) << 32 | x[0], hi = uint64_t(x[3]) << 32 | x[2];
+        if (bits >= 64) {
+            lo = hi;
+            hi = f;
+        }
+        if (const int n = bits & 63) {
+            lo = lo >> n | hi << (64 - n);
+            hi = hi >> n | f << (64 - n);
+        }
+        return gran_raw{uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32)};
+    }
     __device__ static __forceinline__ float get(gran_raw x, int e) {
         if constexpr (sizeof(T) == 2) return to_f32(T{uint16_t(x[e / 2] >> (16 * (e & 1)))});
         else return __uint_as_float(x[e]);
