@@ -117,3 +117,20 @@ def test_ragged_projections(name, dims):
     close(rows(dc), dy64 @ wo.double(), name, "dc")
     close(dwo, dy64.T @ rows(c), name, "dwo")
     close(dbo, dy64.sum(0), name, "dbo")
+
+
+# Stages taken whole and the last one not: every tile inside the matrix, one row or column past it, K
+# at a stage, one more and one less.
+@pytest.mark.parametrize("mnk", [(256, 128, 128), (129, 256, 127), (256, 257, 193), (1280, 1281, 64), (300, 128, 1087)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", sorted(DT))
+def test_ragged_linear_whole_stages(name, mnk):
+    test_ragged_linear(name, mnk)
+
+
+# Head-split stages inside one batch or head and across two: T and d at, past and below the stages.
+@pytest.mark.parametrize("dims", [(3, 64, 260, 4, 64), (2, 130, 196, 3, 80), (3, 127, 256, 2, 128), (5, 96, 132, 4, 32)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", sorted(DT))
+def test_ragged_projections_whole_stages(name, dims):
+    test_ragged_projections(name, dims)
