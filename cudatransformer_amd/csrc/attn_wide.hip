@@ -2,12 +2,15 @@
 // fp32 on v_mfma_f32_32x32x2f32, bf16 / fp16 on v_mfma_f32_32x32x16_{bf16,f16}, gfx950.
 //
 // Same math as the generic kernels that take these head dims otherwise (attn_generic.hip;
-// flash_attention.cu:97-161, :269-311): P and dS keep their fp32 precision.  The 16-bit MFMA
-// takes 16-bit operands, so P and dS go in as two terms, x = hi + lo with hi = round16(x) and
-// lo = round16(x - hi), one MFMA each into the same fp32 accumulator (16 significant bits for
-// bf16, 22 for fp16; the inputs are exact).  fp16 has fp32's precision but not its range:
-// P (<= 2^8) is scaled by a constant power of two, and dS by a running one per wave that
-// follows the largest |dS| seen, the accumulator rescaled when it grows (as the softmax
+// flash_attention.cu:97-161, :269-311), which hold P and dS in fp32.  The 16-bit MFMA takes
+// 16-bit operands, so P and dS go in as a sum of terms, each the rounding to 16 bits of what
+// the terms before it leave, one MFMA each into the same fp32 accumulator (the inputs are exact):
+// three for bf16 (24 significant bits, as fp32), two for fp16 (22).  Share of outputs that are
+// not the 64-bit result rounded once, B2 H8 T1024 d256 unmasked: bf16 generic 0.050-0.053 %, two
+// terms 0.241-0.247 %, three 0.033-0.044 %; fp16 generic 0.42-0.46 %, two terms 0.18-0.25 %.
+// The third bf16 term costs 10 % (forward and backward 214 -> 237 us).  fp16 has fp32's precision
+// but not its range: P (<= 2^8) is scaled by a constant power of two, and dS by a running one per
+// wave that follows the largest |dS| seen, the accumulator rescaled when it grows (as the softmax
 // rescales O).
 //
 // One kernel, four passes (MODE), all of one form: every lane owns one row of the "own"
@@ -32,10 +35,9 @@
 // workgroups of 128 rows, for grids of a few heads.  fp32: 128 own rows, tiles of twice the
 // bytes shared by all four.  128 KB of tiles, one workgroup per CU, one wave per SIMD with up to
 // 512 registers.  Bound: MFMA issue of one wave per SIMD, which its own exponentials and
-// conversions interrupt; per 32 x 32 tile of the mask the 16-bit passes execute 3 + 4 + 4 + 3
-// units (hi and lo) for the convention's 2 + 5, fp32 2 + 3 + 3 + 2.  Measured, B2 H8 T1024 d256
-// unmasked, generic kernels -> this: bf16 forward 10 600 -> 52 us, backward 50 200 -> 201 us
-// (214 TFLOP/s by the convention); B1 H16 T4096 causal bf16 411 and 280 TFLOP/s.
+// conversions interrupt; per 32 x 32 tile of the mask the passes execute, for the convention's
+// 2 + 5 units, bf16 4 + 5 + 5 + 4, fp16 3 + 4 + 4 + 3 and fp32 2 + 3 + 3 + 2.  Measured, B2 H8
+// T1024 d256 bf16 unmasked, forward and backward: generic kernels 60 700 us, this 237.
 #include "attn_bf16_tiles.h"
 #include "attn_launch.h"
 
@@ -68,6 +70,7 @@ struct Wide16 {
     using Vec = typename F::vec;
     static constexpr bool WIDE = false;
     static constexpr bool RANGE = std::is_same_v<F, F16Fmt>;  // 16-bit exponent range to guard
+    static constexpr int TERMS = RANGE ? 2 : 3;               // of P and dS (see the head of the file)
     static constexpr int EB = 2, CH = 32, GROUPS = 2, SLOTS = 2;
     static constexpr int STEPS_PER_TILE = 2;  // contraction steps per 32 head-dim columns
     static constexpr float kPscaleFwd = RANGE ? 64.f : 1.f, kPscaleBwd = RANGE ? 16384.f : 1.f;
@@ -193,14 +196,17 @@ __device__ __forceinline__ void wide_accumulate(floatx16 (&acc)[NT], uint32_t ti
     } else {
         using V = typename E::Vec;
         using el = typename E::Fmt::elem;
-        V hi[2], lo[2];
+        V w[E::TERMS][2];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const el h = (el)p[r];
-            hi[r / 8][r % 8] = h;
-            lo[r / 8][r % 8] = (el)(p[r] - (float)h);
+            float x = p[r];
+#pragma unroll
+            for (int t = 0; t < E::TERMS; ++t) {
+                const el h = (el)x;
+                w[t][r / 8][r % 8] = h;
+                x -= (float)h;
+            }
         }
-        // Steps in pairs of head-dim tiles: the four MFMAs of a pair alternate accumulators.
         constexpr int NS = 2 * NT, AHEAD = 3;
         V a[4];
 #pragma unroll
@@ -209,8 +215,8 @@ __device__ __forceinline__ void wide_accumulate(floatx16 (&acc)[NT], uint32_t ti
         for (int i = 0; i < NS; ++i) {
             if (i + AHEAD < NS) a[(i + AHEAD) & 3] = E::col(tile, ln, (i + AHEAD) / NT, (i + AHEAD) % NT);
             read_fence();
-            acc[i % NT] = E::mma(a[i & 3], hi[i / NT], acc[i % NT]);
-            acc[i % NT] = E::mma(a[i & 3], lo[i / NT], acc[i % NT]);
+#pragma unroll
+            for (int t = 0; t < E::TERMS; ++t) acc[i % NT] = E::mma(a[i & 3], w[t][i / NT], acc[i % NT]);
         }
     }
 }

@@ -32,8 +32,8 @@
  *     multiple of 8 and 16-byte-aligned tensors need no copies (the tiles are filled with
  *     zeros past d) but the same workspace.  d above 128 runs on
  *     MFMA too in fp32, bf16 and fp16 where d is a multiple of 8 (T >= 8; fp32 T >= 32, its
- *     backward T >= 96), with P and dS at fp32 precision, and on the generic kernels
- *     otherwise.  Tensors must be element-aligned; the MFMA kernels at d in {32, 64, 128} and
+ *     backward T >= 96), P and dS entering the 16-bit MFMAs as three bf16 or two fp16
+ *     terms (24 and 22 significant bits), and on the generic kernels otherwise.  Tensors must be element-aligned; the MFMA kernels at d in {32, 64, 128} and
  *     above 128 also need 16-byte-aligned q, k, v, o, lse (and dout, dq, dk, dv, workspace in
  *     the backward); calls whose pointers are not take the generic kernels (same results,
  *     slower).
