@@ -10,8 +10,8 @@
 // terms 0.241-0.247 %, three 0.033-0.044 %; fp16 generic 0.42-0.46 %, two terms 0.18-0.25 %.
 // The third bf16 term costs 10 % (forward and backward 214 -> 237 us).  fp16 has fp32's precision
 // but not its range: P (<= 2^8) is scaled by a constant power of two, and dS by a running one per
-// wave that follows the largest |dS| seen, the accumulator rescaled when it grows (as the softmax
-// rescales O).
+// own row that follows the largest |dS| of the row, the accumulator rescaled when it grows (as the
+// softmax rescales O).
 //
 // One kernel, four passes (MODE), all of one form: every lane owns one row of the "own"
 // tensors, kept in registers as the B operand, and walks 32-row blocks of two "stream" tensors
@@ -239,7 +239,7 @@ struct WidePass {
     floatx16 acc[NT];
     float m_run, l_run;    // kFwd: running max (log2 units) and this half's share of the denominator
     float lse2, ndelta;    // kDq: LSE log2(e) and -delta of the lane's row
-    float es;              // RANGE, dS: the accumulator's scale
+    float es;              // RANGE, dS: the scale of the lane's row in the accumulator
     typename E::Lane ln;
 
     // One 32 x 32 tile of the wave; masked: it crosses the diagonal or the end of the sequence.
@@ -334,7 +334,8 @@ struct WidePass {
         wide_accumulate<E, NT>(acc, TWO ? xt : yt, ln, w);
     }
 
-    // fp16 P / dS into the format's range (see the head of the file).
+    // fp16 P / dS into the format's range (see the head of the file).  Each row by itself: a row past
+    // T (kDk: scores of 0 against LSEs far below 0) may hold anything.
     __device__ __forceinline__ void scale(float (&w)[16]) {
         if constexpr (!TWO) {
 #pragma unroll
@@ -344,16 +345,17 @@ struct WidePass {
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(w[r]));
             if (__any(mx * es > 16384.f)) {
-                mx = wave_max(mx);
-                if (mx < INFINITY) {
+                mx = max_xor32(mx);  // of the row's two lanes
+                float f = 1.f;
+                if (mx * es > 16384.f && mx < INFINITY) {
                     // es = 2^(8 - exponent of mx), from the exponent bits: |dS| es in [2^8, 2^9).
                     const int e = int(__float_as_uint(mx) >> 23) - 127;
                     const float es_new = __uint_as_float(uint32_t(min(8 - e, 100) + 127) << 23);
-                    const float f = es_new / es;
+                    f = es_new / es;
                     es = es_new;
-#pragma unroll
-                    for (int dt = 0; dt < NT; ++dt) acc[dt] *= f;
                 }
+#pragma unroll
+                for (int dt = 0; dt < NT; ++dt) acc[dt] *= f;
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) w[r] *= es;

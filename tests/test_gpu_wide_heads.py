@@ -141,3 +141,32 @@ def test_wide_rounds_as_often_right_as_generic(name, causal):
         ct.set_policy(prev)
     for key in wide:
         assert wide[key] <= 4 / 3 * generic[key], (key, wide[key], generic[key])
+
+
+def rel(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("a", [1.1, 1.4, 2.6])  # mean row LSE about -14, -26, -103
+@pytest.mark.parametrize("shape", [(1, 2, 33, 160), (1, 2, 33, 256), (1, 2, 97, 160), (1, 2, 97, 256)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_rows_past_the_end_do_not_reach_dk(name, shape, a):
+    """Queries that oppose an offset the keys share (row LSE far below 0) at a T that leaves the
+    last 32-key tile partly empty: the empty keys' scores are 0, so exp(0 - LSE) there is up to
+    e^103, and must not move the scale of the fp16 dS of the keys beside them.  dK against
+    float64, keys of the partial tile by themselves: a unit roundoff u and the fp32 error of
+    scores of up to 2000 (1e-4)."""
+    print(f"wide heads negative LSE {name} {shape} {a}", flush=True)
+    x = inputs(shape, name, seed=13)
+    x[0] = (x[0].float() - a).to(DT[name])
+    x[1] = (x[1].float() + a).to(DT[name])
+    _, lse, o_in, lse_in, grads = reference(x, False, DT[name])
+    assert float(lse.max()) < 0
+    q, k, v, do = x
+    got = dict(zip(("dq", "dk", "dv"), ct.flash_attn_bwd(q, k, v, o_in, do, lse_in, False)))
+    tol = {"f32": 0.0, "bf16": 2.0 ** -9, "f16": 2.0 ** -11}[name] + 1e-4
+    tail = shape[2] // 32 * 32
+    assert rel(got["dk"][:, :, tail:], grads["dk"][:, :, tail:]) <= tol
+    for key in grads:
+        assert rel(got[key], grads[key]) <= tol, key
