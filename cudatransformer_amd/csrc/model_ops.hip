@@ -326,21 +326,25 @@ __global__ __launch_bounds__(1024) void layernorm_bwd_reduce_kernel(const A *__r
                                                                    T *__restrict__ db, int64_t chunks, int D) {
     __shared__ A red[32][33];
     const int cl = threadIdx.x & 31, rl = threadIdx.x >> 5;
-    const int64_t c = int64_t(blockIdx.x) * 32 + cl;
-    A s = 0;
-    if (c < 2 * int64_t(D)) {
+    for (int64_t c0 = int64_t(blockIdx.x) * 32; c0 < 2 * int64_t(D); c0 += int64_t(gridDim.x) * 32) {
+        const int64_t c = c0 + cl;
+        A s = 0;
+        if (c < 2 * int64_t(D)) {
 #pragma unroll 8
-        for (int64_t k = rl; k < chunks; k += 32) s += part[k * 2 * D + c];
-    }
-    red[rl][cl] = s;
-    __syncthreads();
-    if (rl != 0 || c >= 2 * int64_t(D)) return;
-    s = 0;
+            for (int64_t k = rl; k < chunks; k += 32) s += part[k * 2 * D + c];
+        }
+        red[rl][cl] = s;
+        __syncthreads();
+        if (rl == 0 && c < 2 * int64_t(D)) {
+            s = 0;
 #pragma unroll
-    for (int l = 0; l < 32; ++l) s += red[l][cl];
-    T *dst = c < D ? dg : db;
-    const int64_t i = c < D ? c : c - D;
-    if (dst != nullptr) st(dst, i, ld(dst, i) + s);
+            for (int l = 0; l < 32; ++l) s += red[l][cl];
+            T *dst = c < D ? dg : db;
+            const int64_t i = c < D ? c : c - D;
+            if (dst != nullptr) st(dst, i, ld(dst, i) + s);
+        }
+        __syncthreads();  // red is read
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -749,6 +753,19 @@ unsigned grid_for(int64_t n) {
 
 unsigned rows_grid(int64_t rows) { return unsigned((rows + 3) / 4); }  // 4 waves (rows) per block
 
+// Launches over N rows, `per` of them in a workgroup of `threads`: f(first row, rows, workgroups) for
+// each launch.  More than one where a single launch would hold more than 2^32 - 1 work-items: past
+// that the runtime drops workgroups without an error.
+template <typename F> hipError_t by_rows(int64_t N, int per, int threads, F f) {
+    const int64_t most = (int64_t(1) << 31) / threads * per;
+    for (int64_t n0 = 0; n0 < N; n0 += most) {
+        const int64_t n = N - n0 < most ? N - n0 : most;
+        f(n0, n, unsigned((n + per - 1) / per));
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 }  // namespace
 }  // namespace ctattn
 
@@ -832,12 +849,13 @@ int ctattn_layernorm_fwd(int dtype, const void *x, const void *gamma, const void
             constexpr int EPC = ctattn::Gran<T>::EPC;
             auto rows = [&](auto gw, auto cpt) {
                 constexpr int GW = decltype(gw)::value, CPT = decltype(cpt)::value;
-                hipLaunchKernelGGL((ctattn::layernorm_fwd_rows_kernel<T, GW, CPT>),
-                                   dim3(GW == 1 ? ctattn::rows_grid(N) : unsigned(N)), dim3(256), 0, st,
-                                   static_cast<const T *>(x), static_cast<const T *>(gamma),
-                                   static_cast<const T *>(beta), static_cast<T *>(y), static_cast<float *>(mean),
-                                   static_cast<float *>(rstd), N, int(D), float(eps));
-                return hipGetLastError();
+                return ctattn::by_rows(N, GW == 1 ? 4 : 1, 256, [&](int64_t n0, int64_t n, unsigned wgs) {
+                    hipLaunchKernelGGL((ctattn::layernorm_fwd_rows_kernel<T, GW, CPT>), dim3(wgs), dim3(256), 0, st,
+                                       static_cast<const T *>(x) + n0 * D, static_cast<const T *>(gamma),
+                                       static_cast<const T *>(beta), static_cast<T *>(y) + n0 * D,
+                                       static_cast<float *>(mean) + n0, static_cast<float *>(rstd) + n0, n, int(D),
+                                       float(eps));
+                });
             };
             if (D <= 64 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<1>{});
             if (D <= 128 * EPC) return rows(ctattn::Int<1>{}, ctattn::Int<2>{});
@@ -847,10 +865,12 @@ int ctattn_layernorm_fwd(int dtype, const void *x, const void *gamma, const void
             if constexpr (sizeof(T) == 4)
                 if (D <= 2048 * EPC) return rows(ctattn::Int<4>{}, ctattn::Int<8>{});
         }
-        hipLaunchKernelGGL(ctattn::layernorm_fwd_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st,
-                           static_cast<const T *>(x), static_cast<const T *>(gamma), static_cast<const T *>(beta),
-                           static_cast<T *>(y), static_cast<A *>(mean), static_cast<A *>(rstd), N, int(D), A(eps));
-        return hipGetLastError();
+        return ctattn::by_rows(N, 4, 256, [&](int64_t n0, int64_t n, unsigned wgs) {
+            hipLaunchKernelGGL(ctattn::layernorm_fwd_kernel<T>, dim3(wgs), dim3(256), 0, st,
+                               static_cast<const T *>(x) + n0 * D, static_cast<const T *>(gamma),
+                               static_cast<const T *>(beta), static_cast<T *>(y) + n0 * D,
+                               static_cast<A *>(mean) + n0, static_cast<A *>(rstd) + n0, n, int(D), A(eps));
+        });
     });
     return finish(fn, e, st);
 }
@@ -919,8 +939,9 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
             if (!one_pass)
                 hipLaunchKernelGGL(ctattn::layernorm_bwd_part_kernel<T>, dim3(unsigned((D + 63) / 64), unsigned(chunks)),
                                    dim3(256), 0, st, xt, dyt, mu, rs, part, N, int(D));
-            hipLaunchKernelGGL(ctattn::layernorm_bwd_reduce_kernel<T>, dim3(unsigned((2 * D + 31) / 32)), dim3(1024), 0,
-                               st, static_cast<const A *>(part), static_cast<T *>(dgamma), static_cast<T *>(dbeta),
+            const int64_t groups = std::min<int64_t>((2 * D + 31) / 32, 65536);  // of columns; the kernel loops
+            hipLaunchKernelGGL(ctattn::layernorm_bwd_reduce_kernel<T>, dim3(unsigned(groups)), dim3(1024), 0, st,
+                               static_cast<const A *>(part), static_cast<T *>(dgamma), static_cast<T *>(dbeta),
                                chunks, int(D));
         }
         return hipGetLastError();
@@ -1028,11 +1049,12 @@ int ctattn_softmax_fwd(int dtype, const void *z, void *p, int64_t N, int64_t V, 
             constexpr int EPC = ctattn::Gran<T>::EPC;
             auto rows = [&](auto gw, auto cpt) {
                 constexpr int GW = decltype(gw)::value, CPT = decltype(cpt)::value;
-                hipLaunchKernelGGL((ctattn::softmax_fwd_rows_kernel<T, GW, CPT>),
-                                   dim3(GW == 1 ? ctattn::rows_grid(N) : unsigned(N)), dim3(GW == 1 ? 256 : 64 * GW), 0,
-                                   st, static_cast<const T *>(z), static_cast<T *>(p), N, int(V),
-                                   1.f / float(temperature));
-                return hipGetLastError();
+                constexpr int threads = GW == 1 ? 256 : 64 * GW;
+                return ctattn::by_rows(N, GW == 1 ? 4 : 1, threads, [&](int64_t n0, int64_t n, unsigned wgs) {
+                    hipLaunchKernelGGL((ctattn::softmax_fwd_rows_kernel<T, GW, CPT>), dim3(wgs), dim3(threads), 0, st,
+                                       static_cast<const T *>(z) + n0 * V, static_cast<T *>(p) + n0 * V, n, int(V),
+                                       1.f / float(temperature));
+                });
             };
             // A temperature past fp32's range makes every class alike (a factor of 0), which the fill of
             // -inf past V would turn into NaN: the general kernel's.
@@ -1046,9 +1068,11 @@ int ctattn_softmax_fwd(int dtype, const void *z, void *p, int64_t N, int64_t V, 
             if constexpr (sizeof(T) == 4)
                 if (fits && V <= 16384 * EPC) return rows(ctattn::Int<16>{}, ctattn::Int<16>{});
         }
-        hipLaunchKernelGGL(ctattn::softmax_fwd_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st,
-                           static_cast<const T *>(z), static_cast<T *>(p), N, int(V), A(1) / A(temperature));
-        return hipGetLastError();
+        return ctattn::by_rows(N, 4, 256, [&](int64_t n0, int64_t n, unsigned wgs) {
+            hipLaunchKernelGGL(ctattn::softmax_fwd_kernel<T>, dim3(wgs), dim3(256), 0, st,
+                               static_cast<const T *>(z) + n0 * V, static_cast<T *>(p) + n0 * V, n, int(V),
+                               A(1) / A(temperature));
+        });
     });
     return finish(fn, e, st);
 }
@@ -1065,10 +1089,11 @@ int ctattn_softmax_bwd(int dtype, const void *p, const void *dp, void *dz, int64
     const hipError_t e = by_dtype(dtype, [&](auto *tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         using A = acc_t<T>;
-        hipLaunchKernelGGL(ctattn::softmax_bwd_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st,
-                           static_cast<const T *>(p), static_cast<const T *>(dp), static_cast<T *>(dz), N, int(V),
-                           A(1) / A(temperature));
-        return hipGetLastError();
+        return ctattn::by_rows(N, 4, 256, [&](int64_t n0, int64_t n, unsigned wgs) {
+            hipLaunchKernelGGL(ctattn::softmax_bwd_kernel<T>, dim3(wgs), dim3(256), 0, st,
+                               static_cast<const T *>(p) + n0 * V, static_cast<const T *>(dp) + n0 * V,
+                               static_cast<T *>(dz) + n0 * V, n, int(V), A(1) / A(temperature));
+        });
     });
     return finish(fn, e, st);
 }
@@ -1148,10 +1173,11 @@ int ctattn_mse_loss_fwd(int dtype, const void *x, const void *target, void *loss
     hipStream_t st = as_stream(stream);
     const hipError_t e = by_dtype(dtype, [&](auto *tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
-        hipLaunchKernelGGL(ctattn::mse_fwd_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st,
-                           static_cast<const T *>(x), static_cast<const T *>(target), static_cast<acc_t<T> *>(loss), N,
-                           int(D));
-        return hipGetLastError();
+        return ctattn::by_rows(N, 4, 256, [&](int64_t n0, int64_t n, unsigned wgs) {
+            hipLaunchKernelGGL(ctattn::mse_fwd_kernel<T>, dim3(wgs), dim3(256), 0, st,
+                               static_cast<const T *>(x) + n0 * D, static_cast<const T *>(target) + n0 * D,
+                               static_cast<acc_t<T> *>(loss) + n0, n, int(D));
+        });
     });
     return finish(fn, e, st);
 }

@@ -10,7 +10,9 @@ kernels with grid-stride loops, so both limits are gone:
   d = 128 both with the recomputing dQ kernel and with the dS tiles stored in the workspace
   (2.7 GB of tiles at 131073 heads of T = 128);
 * more than 2^26 rows on the generic kernels (one wave per row: 2^26 rows x 64 lanes is the
-  2^32 work-item limit of one launch), again first and last slices against the oracle.
+  2^32 work-item limit of one launch), again first and last slices against the oracle;
+* more rows (or columns) than one launch of the row kernels holds work-items for: softmax, and
+  LayerNorm's forward and backward, against float64 around the end of a launch's share.
 
 Inputs are generated on the GPU (seeded); only the checked slices come back to the host.
 """
@@ -118,4 +120,68 @@ def test_more_than_2_26_rows_generic():
             del t
     finally:
         ct.set_policy(prev)
+    torch.cuda.empty_cache()
+
+
+def rows64(t, idx):
+    return torch.stack([t[i] for i in idx]).double()
+
+
+def test_softmax_rows_past_one_launch():
+    """Softmax in place over 4,200,000 rows of 8200 bf16 logits (69 GB): a workgroup of 1024 work-items
+    per row is more than the 2^32 - 1 of one launch, past which it drops rows without an error."""
+    n, v = 4_200_000, 8200
+    assert n * 1024 > 2 ** 32
+    say(f"softmax {n} x {v}")
+    z = torch.empty((n, v), dtype=torch.bfloat16, device=DEV)
+    for i in range(0, n, n // 8):
+        z[i:i + n // 8].normal_()
+    idx = [0, 1, n // 2, 2 ** 21 - 1, 2 ** 21, 2 ** 21 + 1, n - 2, n - 1]
+    want = torch.softmax(rows64(z, idx), -1)
+    rc = ct._capi.load().ctattn_softmax_fwd(1, z.data_ptr(), z.data_ptr(), n, v, 1.0, None)
+    assert rc == 0, ct._capi.last_error()
+    torch.cuda.synchronize()
+    got = rows64(z, idx)
+    # One rounding to bf16 (8 significant bits: at most 2^-8 of the value) and fp32 arithmetic.
+    assert float(((got - want).abs() / want).max()) <= 2.0 ** -8 + 1e-5
+    del z
+    torch.cuda.empty_cache()
+
+
+def test_layernorm_rows_past_one_launch():
+    """LayerNorm over 16,800,000 rows of 1032 bf16 features (35 GB a tensor): 256 work-items per row."""
+    n, d = 16_800_000, 1032
+    assert n * 256 > 2 ** 32
+    say(f"layernorm {n} x {d}")
+    x = torch.empty((n, d), dtype=torch.bfloat16, device=DEV)
+    for i in range(0, n, n // 8):
+        x[i:i + n // 8].normal_()
+    g, b = (torch.randn(d, device=DEV).bfloat16() for _ in range(2))
+    y, mean, rstd = ct._capi.layernorm_fwd(x, g, b)
+    torch.cuda.synchronize()
+    idx = [0, 1, n // 2, 2 ** 23 - 1, 2 ** 23, 2 ** 23 + 1, n - 2, n - 1]
+    xd = rows64(x, idx)
+    want = torch.nn.functional.layer_norm(xd, (d,), g.double(), b.double(), 1e-5)
+    # One rounding to bf16 (2^-8 of the value) and fp32 arithmetic on terms of up to about 10.
+    assert bool(((rows64(y, idx) - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
+    assert float((rows64(mean, idx) - xd.mean(-1)).abs().max()) <= 1e-6
+    assert float((rows64(rstd, idx) * (xd.var(-1, unbiased=False) + 1e-5).sqrt() - 1).abs().max()) <= 1e-5
+    del x, y
+    torch.cuda.empty_cache()
+
+
+def test_layernorm_bwd_columns_past_one_launch():
+    """dgamma and dbeta of 2^26 + 40 fp32 features: 1024 work-items per 32 of the 2 D column sums."""
+    n, d = 2, 2 ** 26 + 40
+    say(f"layernorm backward {n} x {d}")
+    x, dy = torch.randn((n, d), device=DEV), torch.randn((n, d), device=DEV)
+    g = torch.ones(d, device=DEV)
+    mean, rstd = torch.zeros(n, device=DEV), torch.ones(n, device=DEV)
+    dg, db = torch.zeros_like(g), torch.zeros_like(g)
+    ct._capi.layernorm_bwd(x, g, dy, mean, rstd, dg, db)
+    torch.cuda.synchronize()
+    # Two terms in fp32: half an ulp of each and of the sum.
+    assert bool(((db - dy.sum(0)).abs() <= 1e-6 * dy.abs().sum(0)).all())
+    assert bool(((dg - (x * dy).sum(0)).abs() <= 1e-6 * (x * dy).abs().sum(0)).all())
+    del x, dy
     torch.cuda.empty_cache()
