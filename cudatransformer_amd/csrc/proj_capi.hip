@@ -151,6 +151,10 @@ ctattn::LinGemm lin_out_dx(int dtype, const ProjShape &s) {
                     ctattn::lin_linear(s.hd()), ctattn::lin_heads(s.T, s.H, s.d), false);
 }
 
+// What dX may split K in: the caller's workspace where a weight or bias gradient is asked for too.  A
+// call for dX alone needs none and leaves it alone (another stream may hold it).
+void *dx_workspace(void *workspace, bool with_gradients) { return with_gradients ? workspace : nullptr; }
+
 // Split-K bytes of the direct-load GEMMs' plan of a weight gradient (the least a call must bring,
 // with the projection family's) and of whichever GEMM's (what the workspace queries ask for).
 int64_t lin_split_bytes(int dtype, const ctattn::LinGemm &g) {
@@ -237,6 +241,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
     const void *g[3] = {dq, dk, dv};
     hipError_t e = hipSuccess;
     float *ws = static_cast<float *>(workspace);
+    void *const dx_ws = dx_workspace(workspace, want_dw || want_db);
     const int64_t split_bytes =
         std::max(splitk_bytes(dtype, s.hd(), E, s.rows(), 3), lin_split_bytes(dtype, lin_qkv_dw(dtype, s)));
     bool dw_done = false, dx_done = false;
@@ -267,7 +272,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
         }
         lg.c[0] = dx;
         if (ctattn::lin_gemm_supported(lg)) {
-            e = ctattn::launch_lin_gemm(lg, workspace, workspace_bytes, st);
+            e = ctattn::launch_lin_gemm(lg, dx_ws, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dx_done = true;
         }
@@ -373,6 +378,7 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
     hipStream_t st = as_stream(stream);
     const bool v4 = vec4_ok(dtype, s, {c, dy, wo, dwo, dc});
     float *ws = static_cast<float *>(workspace);
+    void *const dc_ws = dx_workspace(workspace, dwo || dbo);
     hipError_t e = hipSuccess;
     const int64_t split_bytes =
         std::max(splitk_bytes(dtype, E, s.hd(), s.rows(), 1), lin_split_bytes(dtype, lin_out_dw(dtype, s)));
@@ -413,7 +419,7 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
         g.b[0][0] = wo;
         g.c[0] = dc;
         if (ctattn::lin_gemm_supported(g))
-            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st), st);
+            return finish(fn, ctattn::launch_lin_gemm(g, dc_ws, workspace_bytes, st), st);
     }
     if (dc) {
         // dc(r, c) = sum_e dy[r][e] wo[e][c]: A = dy (K-contiguous), B = wo stored [k][n]; out
@@ -527,6 +533,7 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
     hipStream_t st = as_stream(stream);
     const bool v4 = linear_vec4(dtype, M, N, K, {x, w, dy, dx, dw});
     float *ws = static_cast<float *>(workspace);
+    void *const dx_ws = dx_workspace(workspace, dw || db);
     hipError_t e = hipSuccess;
     const int64_t split_bytes = linear_split_bytes(dtype, M, N, K);
     if (dw && lin_policy(dtype)) {
@@ -560,7 +567,7 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
     if (dx && lin_policy(dtype)) {
         const ctattn::LinGemm g = lin_dx(dtype, dy, w, dx, M, N, K);
         if (ctattn::lin_gemm_supported(g))
-            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, st), st);
+            return finish(fn, ctattn::launch_lin_gemm(g, dx_ws, workspace_bytes, st), st);
     }
     if (dx) {
         // dx[m][k] = sum_n dy[m][n] w[n][k]: A = dy [M][N] (K-contiguous), B = w stored [k'][n'].
@@ -612,7 +619,8 @@ int ctattn_linear_act_bwd(int dtype, int act, const void *x, const void *w, cons
         g.act_kind = act;
         g.aux[0] = const_cast<void *>(pre);
         if (ctattn::lin_gemm_supported(g))
-            return finish(fn, ctattn::launch_lin_gemm(g, workspace, workspace_bytes, as_stream(stream)), as_stream(stream));
+            return finish(fn, ctattn::launch_lin_gemm(g, dx_workspace(workspace, dw || db), workspace_bytes,
+                                                      as_stream(stream)), as_stream(stream));
     }
     if (int rc = ctattn_linear_bwd(dtype, x, w, dy, dpre, nullptr, nullptr, workspace, workspace_bytes, M, N, K, stream))
         return rc;

@@ -220,7 +220,15 @@ CTATTN_API int ctattn_qkv_proj_fwd(int dtype, const void *x, const void *wq, con
                                    void *q, void *k, void *v, int64_t B, int64_t T, int64_t E,
                                    int64_t H, int64_t d, void *stream);
 
-/* Workspace bytes ctattn_qkv_proj_bwd needs (>= 0), or -1 on invalid arguments. */
+/*
+ * Workspace bytes for ctattn_qkv_proj_bwd (>= 0), or -1 on invalid arguments.  This query and those
+ * of ctattn_out_proj_bwd and ctattn_linear_bwd return the size at which every product of the
+ * backward runs its fastest plan; the entry points accept less, down to the size their error
+ * message names.  The workspace is needed, read and written only where a weight or bias gradient
+ * is asked for: then the products of that call may all split their contraction into it, dX too,
+ * so the size given can change the summation order (the last bits) of a gradient and of dX.  A call
+ * for dX alone leaves it untouched, so it may overlap a call that uses it.
+ */
 CTATTN_API int64_t ctattn_qkv_proj_bwd_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t E,
                                                        int64_t H, int64_t d);
 
@@ -231,7 +239,7 @@ CTATTN_API int64_t ctattn_qkv_proj_bwd_workspace_bytes(int dtype, int64_t B, int
  *   dbq/dbk/dbv += column sums of dq/dk/dv over all B*T rows
  *   dx = dq wq + dk wk + dv wv     (overwritten)
  * Pass NULL for all three dw (or all three db, or dx) to skip that part; the workspace is
- * only needed for dw / db.  Replaces the qkvBackwardWB and qkvBackward launches of
+ * only used where dw / db are asked for.  Replaces the qkvBackwardWB and qkvBackward launches of
  * QKVProjectionLayer::computeBackward (QKVProjectionLayer.cu:124-137; kernels
  * attention_qkv_kernels.cu:171-364).  Unlike the reference's bias gradient, which sums only
  * the first row of each 32-row tile (attention_qkv_kernels.cu:233-237), every row counts.
@@ -252,15 +260,15 @@ CTATTN_API int ctattn_out_proj_fwd(int dtype, const void *c, const void *wo, con
                                    int64_t B, int64_t T, int64_t E, int64_t H, int64_t d,
                                    void *stream);
 
-/* Workspace bytes ctattn_out_proj_bwd needs (>= 0), or -1 on invalid arguments. */
+/* Workspace bytes for ctattn_out_proj_bwd, as ctattn_qkv_proj_bwd_workspace_bytes. */
 CTATTN_API int64_t ctattn_out_proj_bwd_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t E,
                                                        int64_t H, int64_t d);
 
 /*
  * Backward of the output projection:
  *   dwo += dy^T c,  dbo += column sums of dy,  dc = dy wo  (dc in [B, H, T, d], overwritten).
- * dwo, dbo or dc may be NULL to skip; the workspace is only needed for dwo / dbo.  Replaces
- * the projBackwardWB and projBackward launches of OutputProjectionLayer::backward
+ * dwo, dbo or dc may be NULL to skip; the workspace is only used where dwo / dbo are asked for.
+ * Replaces the projBackwardWB and projBackward launches of OutputProjectionLayer::backward
  * (OutputProjectionLayer.cu:83-94; kernels attention_proj_kernels.cu:142-288), with every
  * row in the bias gradient (the reference's sums one row per 32-row tile,
  * attention_proj_kernels.cu:188,194-196).  Deterministic.
@@ -294,13 +302,13 @@ CTATTN_API int ctattn_sgd_update(int dtype, void *params, const void *grads, dou
 CTATTN_API int ctattn_linear_fwd(int dtype, const void *x, const void *w, const void *b, void *y,
                                  int64_t M, int64_t N, int64_t K, void *stream);
 
-/* Workspace bytes ctattn_linear_bwd needs (>= 0), or -1 on invalid arguments. */
+/* Workspace bytes for ctattn_linear_bwd, as ctattn_qkv_proj_bwd_workspace_bytes. */
 CTATTN_API int64_t ctattn_linear_bwd_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
 
 /*
  * Backward of the linear layer: dw += dy^T x, db += column sums of dy, dx = dy w
- * (overwritten).  dw, db or dx may be NULL to skip; the workspace is only needed for dw / db.
- * Replaces the linearBackwardWB and linearBackward launches of LinearLayer::backward
+ * (overwritten).  dw, db or dx may be NULL to skip; the workspace is only used where dw / db are asked
+ * for.  Replaces the linearBackwardWB and linearBackward launches of LinearLayer::backward
  * (LinearLayer.cu:83,95; kernels linear_kernels.cu:115,199) and UnEmbedding::backward
  * (Embedding.cu:378,390).  Deterministic.
  */
@@ -323,8 +331,9 @@ CTATTN_API int ctattn_linear_act_fwd(int dtype, int act, const void *x, const vo
  * (= act(pre)), dw += dy^T x and db += column sums of dy as ctattn_linear_bwd, and
  * dpre[m][k] = act'(pre[m][k]) * sum_n dy[m][n] w[n][k] -- the linear layer's dX and the
  * activation's backward in one GEMM epilogue where the MFMA GEMMs take the shape.  Results equal
- * ctattn_linear_bwd followed by ctattn_activation_bwd; dw / db may be NULL; the workspace is
- * only needed for dw / db (ctattn_linear_bwd_workspace_bytes).  No counterpart in the
+ * ctattn_linear_bwd (with the same gradients asked for and workspace) followed by
+ * ctattn_activation_bwd; dw / db may be NULL; the workspace is only used where dw / db are asked for
+ * (ctattn_linear_bwd_workspace_bytes).  No counterpart in the
  * reference (LinearLayer.cu:83,95 then ActivationLayer.cu:83-92).
  */
 CTATTN_API int ctattn_linear_act_bwd(int dtype, int act, const void *x, const void *w, const void *dy,

@@ -134,3 +134,44 @@ def test_ragged_linear_whole_stages(name, mnk):
 @pytest.mark.parametrize("name", sorted(DT))
 def test_ragged_projections_whole_stages(name, dims):
     test_ragged_projections(name, dims)
+
+
+@pytest.mark.parametrize("name", sorted(DT))
+def test_dx_alone_leaves_the_workspace_alone(name):
+    """A backward for dX alone may overlap, on another stream, a call that works in the same workspace:
+    it writes none of it, in shapes whose dX splits K into the workspace of a call that also asks for
+    the weight gradient, and gives the same dX as with no workspace at all."""
+    print(f"dx alone {name}", flush=True)
+    lib, code, dt = _capi.load(), _capi._DTYPE_CODE[DT[name]], DT[name]
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(dt)
+
+    st = torch.cuda.current_stream().cuda_stream
+    ws = torch.full((64 << 20,), 0xA5, dtype=torch.uint8, device="cuda")
+
+    def check(call, out):
+        assert call(None, 0) == 0, _capi.last_error()
+        torch.cuda.synchronize()
+        plain = out.clone()
+        out.zero_()
+        assert call(ws.data_ptr(), ws.numel()) == 0, _capi.last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(plain, out)
+        assert bool((ws == 0xA5).all())
+
+    m, n, k = 100, 5003, 256  # 8 tiles of 64 x 64, 79 or 157 stages of K
+    dy, w, pre, dx = rnd(m, n), rnd(n, k), rnd(m, k), rnd(m, k)
+    check(lambda p, b: lib.ctattn_linear_bwd(code, None, w.data_ptr(), dy.data_ptr(), dx.data_ptr(), None, None, p, b,
+                                             m, n, k, st), dx)
+    check(lambda p, b: lib.ctattn_linear_act_bwd(code, _capi.ACT_GELU, None, w.data_ptr(), dy.data_ptr(),
+                                                 pre.data_ptr(), dx.data_ptr(), None, None, p, b, m, n, k, st), dx)
+    b_, t, e, h, d = 1, 101, 1003, 8, 40
+    x, gr, wq = rnd(b_, t, e), [rnd(b_, h, t, d) for _ in range(3)], [rnd(h * d, e) for _ in range(3)]
+    dxp = torch.empty_like(x)
+    args = [a.data_ptr() for a in (x, *gr, *wq)]
+    check(lambda p, b: lib.ctattn_qkv_proj_bwd(code, *args, *[None] * 6, dxp.data_ptr(), p, b, b_, t, e, h, d, st), dxp)
+    wo, dc = rnd(e, h * d), torch.empty_like(gr[0])
+    check(lambda p, b: lib.ctattn_out_proj_bwd(code, None, x.data_ptr(), wo.data_ptr(), None, None, dc.data_ptr(), p, b,
+                                               b_, t, e, h, d, st), dc)
