@@ -247,7 +247,9 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
             for (int j = 0; j < CPT; ++j)
 #pragma unroll
                 for (int e = 0; e < G::EPC; ++e) {
-                    const float d = G::get(dv[i][j], e), xh = (G::get(xv[i][j], e) - mu[i]) * rs[i];
+                    // Past D (0 - mean) rstd may overflow, and 0 times an infinity would reach the sums.
+                    const bool in = (lane + kWave * GW * j) * G::EPC + e < D;
+                    const float d = G::get(dv[i][j], e), xh = in ? (G::get(xv[i][j], e) - mu[i]) * rs[i] : 0.f;
                     sg[j * G::EPC + e] += d * xh;
                     sb[j * G::EPC + e] += d;
                     const float dxh = d * G::get(gv[j], e);

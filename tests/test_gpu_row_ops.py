@@ -64,6 +64,23 @@ def test_layernorm_edges(name, d):
         close(db, dy64.sum(0), TOL[name], "dbeta")
 
 
+@pytest.mark.parametrize("d", [96, 101, 200])
+def test_layernorm_bwd_large_constant_rows(d):
+    """Rows of one value 2^120: the statistics are exact (variance 0), but -mean rstd overflows, which
+    must stay out of the sums over the columns (lanes past the row's end hold zeros)."""
+    print(f"layernorm large rows D={d}", flush=True)
+    for name in ("f32", "bf16"):
+        dt = DT[name]
+        x = torch.full((5, d), 2.0 ** 120, device="cuda").to(dt)
+        g, dy = rnd((d,), dt, 3, 0.1, 1.0), rnd((5, d), dt, 2)
+        _, mean, rstd = _capi.layernorm_fwd(x, g, torch.zeros_like(g))
+        dx = _capi.layernorm_bwd(x, g, dy, mean, rstd)
+        torch.cuda.synchronize()
+        assert bool((mean == 2.0 ** 120).all())
+        dxh = dy.double() * g.double()
+        close(dx, rstd.double()[:, None] * (dxh - dxh.mean(-1, keepdim=True)), TOL[name], "dx")
+
+
 @pytest.mark.parametrize("v", [1, 3, 65, 256, 257, 512, 1025, 2048, 4097, 8193, 16385, 32769, 65536, 65537])
 @pytest.mark.parametrize("name", sorted(DT))
 def test_softmax_and_gradient_edges(name, v):
