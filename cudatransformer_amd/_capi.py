@@ -146,14 +146,19 @@ def set_policy(policy: int) -> int:
     return prev
 
 
+# Raw handle of a device's current stream: not a documented part of torch, so it may be missing.
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(stream) -> int:
-    """hipStream_t of `stream`, or of the current stream.  The current one is read as a raw handle:
-    torch.cuda.current_stream() builds a Stream object for it, 2.7 us of a small call's 12."""
+    """hipStream_t of `stream`, or of the current stream.  The current one is read as a raw handle
+    where torch has one: torch.cuda.current_stream() builds a Stream object for it, 2.7 us of a small
+    call's 12."""
     if stream is not None:
         return int(stream.cuda_stream)
-    if not torch.cuda.is_initialized():
-        torch.cuda.init()
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _current_raw_stream is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return _current_raw_stream(torch.cuda.current_device())
 
 
 def _check_qkv(name, *ts):

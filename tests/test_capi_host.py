@@ -305,3 +305,15 @@ def test_fwd_workspace_bytes(lib):
         assert lib.ctattn_fwd_workspace_bytes(0, b, h, t, 48) == 0
     finally:
         _capi.set_policy(prev)
+
+def test_stream_handle_without_torchs_raw_stream(monkeypatch):
+    """A torch without the raw stream getter: the handle comes from torch.cuda.current_stream()."""
+    class Stream:
+        cuda_stream = 0x1234
+
+    monkeypatch.setattr(_capi, "_current_raw_stream", None)
+    monkeypatch.setattr(_capi.torch.cuda, "current_stream", lambda: Stream)
+    assert _capi._stream_handle(None) == 0x1234
+    other = Stream()
+    other.cuda_stream = 7
+    assert _capi._stream_handle(other) == 7
