@@ -286,10 +286,9 @@ def test_layernorm_bwd_is_deterministic():
 @pytest.mark.parametrize("dtype", DTYPES, ids=DT_IDS)
 @pytest.mark.parametrize("nd", [(4096, 384), (77, 96), (300, 1000), (65, 1024), (40, 1100)])
 def test_layernorm_bwd_one_pass_equals_two(dtype, nd):
-    """dx with dgamma / dbeta in one pass (D <= 1024: one workgroup per 32-row chunk, the
-    partial sums kept per lane) against dx alone and dgamma / dbeta alone (the dx kernel and
-    the two-stage column sums): bitwise equal, ragged chunks included; D = 1100 takes the
-    separate kernels either way."""
+    """dx with dgamma / dbeta against dx alone and dgamma / dbeta alone: outputs that are not asked
+    for change nothing in the others, bit for bit, ragged chunks included (fp64: the separate
+    kernels' rows and column sums; their values are checked against float64 elsewhere)."""
     n, d = nd
     print(f"layernorm one pass {dtype} N={n} D={d}", flush=True)
     x = _dev(_randn((n, d), 60, 2.0) + 0.5, dtype)

@@ -114,3 +114,28 @@ def test_softmax_temperatures_past_fp32(v, temperature):
     for name, dt in DT.items():
         p = _capi.softmax_fwd(rnd((3, v), dt, 7), temperature)
         assert ((p.double() * v - 1).abs() <= TOL[name] + (2.0 ** -25 * v if name == "f16" else 0)).all()
+
+
+# The first length past each number of waves per row, and several past the row kernels.
+@pytest.mark.parametrize("d", [1025, 2049, 4097, 8193, 9001, 16390])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_layernorm_past_the_edges(name, d):
+    test_layernorm_edges(name, d)
+
+
+def test_softmax_exponential_ulps():
+    """The softmax's exponential through rows (0, x) in fp32, in units in the last place of the result.
+    Below -18 the probability of x is e^x itself: 1 ulp of the hardware's exp2 and 2 x 2^-26 of its
+    argument's fraction (0.7 ulp), results in the subnormals rounded once more (half a step).  Above,
+    the sum, its reciprocal and the product add 0.5, 1 and 0.5 ulp, and e^x enters twice: 6."""
+    print("softmax exponential", flush=True)
+    x = torch.cat([torch.linspace(-110, -18, 200001), torch.linspace(-18, 0, 200001)]).cuda()
+    p = _capi.softmax_fwd(torch.stack([torch.zeros_like(x), x], 1))[:, 1]
+    torch.cuda.synchronize()
+    want = torch.softmax(torch.stack([torch.zeros_like(x), x], 1).double(), 1)[:, 1]
+    ulp = torch.exp2(torch.floor(torch.log2(want)).clamp_min(-126) - 23)
+    err = (p.double() - want).abs() / ulp
+    print(f"largest {float(err[x < -18].max()):.2f} and {float(err[x >= -18].max()):.2f} ulp", flush=True)
+    assert float(err[x < -18].max()) <= 2.2
+    assert float(err.max()) <= 6
+    assert bool((p[x < -104] == 0).all())  # e^x below half of 2^-149

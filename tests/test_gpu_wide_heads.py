@@ -143,6 +143,9 @@ def test_wide_rounds_as_often_right_as_generic(name, causal):
         assert wide[key] <= 4 / 3 * generic[key], (key, wide[key], generic[key])
 
 
+UNIT = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}  # most that one rounding to storage changes a value
+
+
 def rel(got, want):
     return float((got.double() - want).norm() / want.norm())
 
@@ -165,8 +168,44 @@ def test_wide_rows_past_the_end_do_not_reach_dk(name, shape, a):
     assert float(lse.max()) < 0
     q, k, v, do = x
     got = dict(zip(("dq", "dk", "dv"), ct.flash_attn_bwd(q, k, v, o_in, do, lse_in, False)))
-    tol = {"f32": 0.0, "bf16": 2.0 ** -9, "f16": 2.0 ** -11}[name] + 1e-4
+    tol = UNIT[name] + 1e-4
     tail = shape[2] // 32 * 32
     assert rel(got["dk"][:, :, tail:], grads["dk"][:, :, tail:]) <= tol
     for key in grads:
         assert rel(got[key], grads[key]) <= tol, key
+
+
+def check64(x, causal, name):
+    """All outputs against float64: one rounding to storage and the fp32 error of scores of up to
+    1000 (1e-4)."""
+    o, lse, o_in, lse_in, grads = reference(x, causal, DT[name])
+    q, k, v, do = x
+    got_o, got_lse = ct.flash_attn_fwd(q, k, v, causal)
+    got = dict(zip(("dq", "dk", "dv"), ct.flash_attn_bwd(q, k, v, o_in, do, lse_in, causal)))
+    assert rel(got_lse, lse) <= 1e-5
+    for key, want in {"o": o, **grads}.items():
+        assert rel({"o": got_o, **got}[key], want) <= UNIT[name] + 1e-4, key
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_running_max_grows(name, causal):
+    """Scores that rise by 6 with every 32 keys (9 in log2 units): the running max passes its
+    first block's by more than 2^8 again and again."""
+    print(f"wide heads growing scores {name} causal={causal}", flush=True)
+    x = inputs((1, 2, 333, 256), name, seed=17)
+    x[0] = (x[0].float() + 1).to(DT[name])
+    x[1] = (x[1].float() + torch.linspace(0, 4, 333, device="cuda")[:, None]).to(DT[name])
+    check64(x, causal, name)
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_gradients_grow_along_the_sequence(name, causal):
+    """dO and V grow by 2^14 and 2^12 along the sequence, so the running scale of the fp16 dS has to
+    come down several times in the dK and dQ passes."""
+    print(f"wide heads growing gradients {name} causal={causal}", flush=True)
+    x = inputs((1, 2, 333, 256), name, seed=19)
+    x[2] = (x[2].float() * torch.logspace(-8, 4, 333, 2.0, device="cuda")[:, None]).to(DT[name])
+    x[3] = (x[3].float() * torch.logspace(-12, 2, 333, 2.0, device="cuda")[:, None]).to(DT[name])
+    check64(x, causal, name)
