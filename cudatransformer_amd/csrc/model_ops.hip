@@ -191,12 +191,19 @@ __global__ __launch_bounds__(256) void layernorm_bwd_part_kernel(const T *__rest
     }
 }
 
-// dx and the stage-1 gamma / beta partial sums of one 32-row chunk in one pass over x and dy (fp32
-// and 16-bit storage, D <= 64 GW CPT EPC; either output may be null).  8 waves: 8 / GW groups of GW
-// waves, group k taking rows k, k + 8 / GW, ... of the chunk, four (two) at a time (their 16-byte
-// loads issued together), with the columns' sums in registers and the groups' sums added in LDS in
-// group order.  Bound by HBM; bf16 8192 x 2048 (dx 30 + partial sums 17 us as two kernels) -> 26 us.
-template <typename T, int GW, int CPT>
+// The backward with rows in registers (fp32 and 16-bit storage, D <= 64 GW CPT EPC).  8 waves: 8 / GW
+// groups of GW waves, a row each, RB rows at a time (their 16-byte loads issued together).
+//   PART   dx (may be null) and the stage-1 gamma / beta partial sums of one 32-row chunk in one pass
+//          over x and dy: group k takes rows k, k + 8 / GW, ..., with the columns' sums in registers and
+//          the groups' sums added in LDS in group order.  Bound by HBM at many chunks; bf16 8192 x 2048
+//          (dx 30 + partial sums 17 us as two kernels) -> 26 us.  A workgroup per 32 rows, one of them
+//          on a CU (154 to 256 registers), leaves the chip idle at few chunks.
+//   !PART  dx alone, RB rows a group: 57 to 114 registers, 2 to 4 workgroups on a CU.  The same
+//          arithmetic, so the same dx.  Against one wave per row (layernorm_bwd_dx_kernel), us: bf16
+//          256 x 3072 12.5 -> 5.1, 8192 x 2048 24.1 -> 12.7, 65536 x 384 37.8 -> 23.6; fp32 256 x 3072
+//          14.6 -> 5.0, 65536 x 128 20.3 -> 17.4; PART's kernel for dx alone took 27.8, 17.0, 39.8,
+//          35.4 and 43.6.
+template <typename T, int GW, int CPT, bool PART>
 __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__restrict__ x, const T *__restrict__ g,
                                                                 const T *__restrict__ dy,
                                                                 const float *__restrict__ mean,
@@ -204,14 +211,15 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
                                                                 float *__restrict__ part, int64_t N, int D) {
     using G = Gran<T>;
     constexpr int EPT = CPT * G::EPC;
-    constexpr int NG = 8 / GW, RB = EPT > 8 ? 2 : 4, RPG = kLnRowsPerChunk / NG;
-    constexpr int COLS = kWave * GW * EPT;  // >= D
-    __shared__ float xch[2][8][RB][2];      // row sums of each wave, by batch parity
+    constexpr int NG = 8 / GW, RB = !PART ? 2 : EPT > 8 ? 2 : 4;
+    constexpr int RPG = PART ? kLnRowsPerChunk / NG : RB;  // rows per group
+    constexpr int COLS = PART ? kWave * GW * EPT : 1;  // >= D
+    __shared__ float xch[2][8][RB][2];                 // row sums of each wave, by batch parity
     __shared__ float red[NG][COLS];
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
     const int grp = wave / GW;
     const int lane = (wave % GW) * kWave + int(threadIdx.x) % kWave;  // within the group
-    const int64_t r0 = int64_t(blockIdx.x) * kLnRowsPerChunk;
+    const int64_t r0 = int64_t(blockIdx.x) * (NG * RPG);
     gran_raw gv[CPT];
     float sg[EPT], sb[EPT];
 #pragma unroll
@@ -250,8 +258,10 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
                     // Past D (0 - mean) rstd may overflow, and 0 times an infinity would reach the sums.
                     const bool in = (lane + kWave * GW * j) * G::EPC + e < D;
                     const float d = G::get(dv[i][j], e), xh = in ? (G::get(xv[i][j], e) - mu[i]) * rs[i] : 0.f;
-                    sg[j * G::EPC + e] += d * xh;
-                    sb[j * G::EPC + e] += d;
+                    if constexpr (PART) {
+                        sg[j * G::EPC + e] += d * xh;
+                        sb[j * G::EPC + e] += d;
+                    }
                     const float dxh = d * G::get(gv[j], e);
                     s1[i] += dxh;
                     s2[i] += dxh * xh;
@@ -300,7 +310,7 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
             }
         }
     }
-    if (part == nullptr) return;
+    if constexpr (!PART) return;
     float *pc = part + int64_t(blockIdx.x) * 2 * D;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -910,31 +920,40 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
         const A *mu = static_cast<const A *>(mean);
         const A *rs = static_cast<const A *>(rstd);
         A *part = static_cast<A *>(workspace);
-        // dx and the partial sums from one kernel while the columns fit the registers of 8 waves.
+        // Rows in registers: dx and the partial sums in one pass, or dx by itself and the partial sums
+        // from their own kernel.  The line depends on N and D alone, so an output has the same bits
+        // whichever others are asked for.  Measured, us, one pass / two kernels, both outputs:
+        //   D > 1024    few chunks leave CUs idle: bf16 256 x 3072 31.3 / 11.5, 4096 x 3072 33.9 / 28.5,
+        //               4096 x 2048 19.2 / 19.5, 8192 x 2048 21.7 / 31.5; fp32 256 x 8192 55.9 / 14.4,
+        //               2048 x 2048 19.0 / 16.6, 4096 x 2048 21.1 / 26.7
+        //   D <= 1024   one pass; in 16 bits not for many rows that leave lanes idle: 65536 x 128 51.1 /
+        //               36.2, 65536 x 768 96.8 / 91.3, 8192 x 768 15.2 / 18.4, 65536 x 512 40.8 / 57.0
+        // dx by itself: one wave per row past D 8192, in fp64 and for many 16-bit rows of at most 16 granules
+        // (65536 x 128: bf16 20.5 in registers / 18.9, fp16 25.5 / 20.3).
         bool one_pass = false;
+        const bool wave_dx = std::is_same_v<T, double> || D > 8192 || (sizeof(T) == 2 && D <= 128 && N > 8192);
         if constexpr (!std::is_same_v<T, double>) {
             constexpr int CU = sizeof(T) == 4 ? 2 : 1;  // granules per 8 elements
+            one_pass = D > 1024 ? D <= 8192 && N * int64_t(sizeof(T)) > 8192
+                                : CU == 2 || N <= 8192 || 8 * D >= 7 * (D <= 512 ? 512 : 1024);
             auto rows = [&](auto gw, auto cpt) {
                 constexpr int GW = decltype(gw)::value, CPT = decltype(cpt)::value;
-                hipLaunchKernelGGL((ctattn::layernorm_bwd_rows_kernel<T, GW, CPT>), dim3(unsigned(chunks)), dim3(512),
-                                   0, st, xt, static_cast<const T *>(gamma), dyt, mu, rs, static_cast<T *>(dx),
-                                   dgamma || dbeta ? part : nullptr, N, int(D));
+                auto launch = [&](auto kernel, int64_t wgs) {
+                    hipLaunchKernelGGL(kernel, dim3(unsigned(wgs)), dim3(512), 0, st, xt,
+                                       static_cast<const T *>(gamma), dyt, mu, rs, static_cast<T *>(dx), part, N, int(D));
+                };
+                constexpr int dx_rows = 8 / GW * 2;  // per workgroup
+                if (one_pass && (dgamma || dbeta)) launch(ctattn::layernorm_bwd_rows_kernel<T, GW, CPT, true>, chunks);
+                else if (dx && !wave_dx) launch(ctattn::layernorm_bwd_rows_kernel<T, GW, CPT, false>, (N + dx_rows - 1) / dx_rows);
             };
-            one_pass = D <= 8192;
-            if (!one_pass) {
-            } else if (D <= 512) {
-                rows(ctattn::Int<1>{}, ctattn::Int<CU>{});
-            } else if (D <= 1024) {
-                rows(ctattn::Int<2>{}, ctattn::Int<CU>{});
-            } else if (D <= 2048) {
-                rows(ctattn::Int<4>{}, ctattn::Int<CU>{});
-            } else if (D <= 4096) {
-                rows(ctattn::Int<8>{}, ctattn::Int<CU>{});
-            } else {
-                rows(ctattn::Int<8>{}, ctattn::Int<2 * CU>{});
-            }
+            if (D <= 256) rows(ctattn::Int<1>{}, ctattn::Int<1>{});
+            else if (D <= 512) rows(ctattn::Int<1>{}, ctattn::Int<CU>{});
+            else if (D <= 1024) rows(ctattn::Int<2>{}, ctattn::Int<CU>{});
+            else if (D <= 2048) rows(ctattn::Int<4>{}, ctattn::Int<CU>{});
+            else if (D <= 4096) rows(ctattn::Int<8>{}, ctattn::Int<CU>{});
+            else if (D <= 8192) rows(ctattn::Int<8>{}, ctattn::Int<2 * CU>{});
         }
-        if (dx && !one_pass)
+        if (dx && wave_dx)
             hipLaunchKernelGGL(ctattn::layernorm_bwd_dx_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st, xt,
                                static_cast<const T *>(gamma), dyt, mu, rs, static_cast<T *>(dx), N, int(D));
         if (dgamma || dbeta) {

@@ -139,3 +139,38 @@ def test_softmax_exponential_ulps():
     assert float(err[x < -18].max()) <= 2.2
     assert float(err.max()) <= 6
     assert bool((p[x < -104] == 0).all())  # e^x below half of 2^-149
+
+
+@pytest.mark.parametrize("nd", [(8192, 65), (8193, 65), (8193, 250), (8193, 384), (8193, 448), (8193, 513), (8193, 896),
+                                (2048, 1032), (2049, 1032), (4096, 1032), (4097, 1032), (4096, 2052), (4097, 2052),
+                                (2049, 4100), (4097, 4100)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", sorted(DT))
+def test_layernorm_bwd_one_pass_or_two(name, nd):
+    """Both sides of the lines in N and D between dx with the partial sums in one pass and dx by itself,
+    against float64, and each output alone: the same bits."""
+    n, d = nd
+    dt, code, lib = DT[name], _capi._DTYPE_CODE[DT[name]], _capi.load()
+    print(f"layernorm backward {name} {n} x {d}", flush=True)
+    x, dy = rnd((n, d), dt, 1, 2.0, 0.5), rnd((n, d), dt, 2)
+    g = rnd((d,), dt, 3, 0.1, 1.0)
+    _, mean, rstd = _capi.layernorm_fwd(x, g, torch.zeros_like(g))
+    ws = torch.empty(lib.ctattn_layernorm_bwd_workspace_bytes(code, n, d), dtype=torch.uint8, device="cuda")
+
+    def bwd(want_dx, want_g):
+        dx, dg, db = torch.zeros_like(x), torch.zeros_like(g), torch.zeros_like(g)
+        rc = lib.ctattn_layernorm_bwd(code, x.data_ptr(), g.data_ptr(), dy.data_ptr(), mean.data_ptr(), rstd.data_ptr(),
+                                      dx.data_ptr() if want_dx else None, dg.data_ptr() if want_g else None,
+                                      db.data_ptr() if want_g else None, ws.data_ptr() if want_g else None,
+                                      ws.numel() if want_g else 0, n, d, None)
+        assert rc == 0, _capi.last_error()
+        torch.cuda.synchronize()
+        return dx, dg, db
+
+    dx, dg, db = bwd(True, True)
+    assert torch.equal(bwd(True, False)[0], dx)
+    assert all(torch.equal(a, b) for a, b in zip(bwd(False, True)[1:], (dg, db)))
+    x64, dy64, mu, rs = x.double(), dy.double(), mean.double()[:, None], rstd.double()[:, None]
+    xh, dxh = (x64 - mu) * rs, dy64 * g.double()
+    close(dx, rs * (dxh - dxh.mean(-1, keepdim=True) - xh * (dxh * xh).mean(-1, keepdim=True)), TOL[name], "dx")
+    close(dg, (dy64 * xh).sum(0), TOL[name], "dgamma")
+    close(db, dy64.sum(0), TOL[name], "dbeta")
