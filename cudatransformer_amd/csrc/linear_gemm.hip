@@ -492,12 +492,16 @@ __device__ __forceinline__ void store_cols4(const Args &p, char *cz, const char 
 // The same where N is not a multiple of 4 or a group crosses heads (vec_out 0), kept out of the
 // common path.  GROUPS: whole groups at once where vec_out is 1, from their element-aligned
 // addresses -- faster for the wide rows of the shared tiles (bf16 256 x 50257 x 256 forward 50 ->
-// 36 us, 2048 x 5461 x 2048 95 -> 79), slower for the 64-wide ones (990 x 5003 x 256 25 -> 28).
+// 36 us, 2048 x 5461 x 2048 95 -> 79), slower for the 64-wide ones (990 x 5003 x 256 25 -> 28) and with
+// a fused activation's two outputs (1024 x 5003 x 768 with GELU bf16 45 -> 54, fp16 42 -> 53).
 template <typename F, bool GROUPS>
 __device__ __forceinline__ void store_cols_edge(const Args &p, const DView &view_c, char *cz, const char *bz, int z,
                                                 int gm, int gn, floatx4 x) {
-    if (GROUPS && p.vec_out == 1 && gn + 4 <= p.N) {
-        store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
+    if (GROUPS && p.vec_out == 1 && p.act_mode == 0 && gn + 4 <= p.N) {
+        char *dst = cz + rowoff(view_c, gm) + coloff(view_c, gn);
+        if (bz != nullptr) x += F::load4(bz + int64_t(gn) * F::EB);
+        if (p.beta) x += F::load4(dst);
+        F::store4(dst, x);
         return;
     }
 #pragma unroll
@@ -717,7 +721,8 @@ __global__ __launch_bounds__(NW * 64) void lin_kernel(Args p) {
             }
             continue;
         }
-        if (p.vec_out == 2)
+        // The hint keeps the common path in line (fp32 dX 8192 x 512, K 1024, head-split out: 80 -> 76 us).
+        if (__builtin_expect(p.vec_out == 2, 1))
             store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
         else
             store_cols_edge<F, false>(p, view_c, cz, bz, z, gm, gn, x);
@@ -951,7 +956,7 @@ __device__ __forceinline__ void shared_store(const floatx16 (&acc)[TM][TN], cons
                 }
                 continue;
             }
-            if (p.vec_out == 2)
+            if (__builtin_expect(p.vec_out == 2, 1))
                 store_cols4<F>(p, cz, bz, z, rowoff(view_c, gm) + coloff(view_c, gn), gn, x);
             else
                 store_cols_edge<F, true>(p, view_c, cz, bz, z, gm, gn, x);
@@ -972,7 +977,6 @@ __global__ __launch_bounds__(WM * WN * 64) void lin_shared_kernel(Args p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     const int wm = wave / WN, wn = wave - (wave / WN) * WN;
-    const int h = lane >> 5, col = lane & 31;
 
     // XCD-aware order, as lin_kernel: XCD x runs the contiguous work items [x q, x q + q).
     const int nblk = int(gridDim.x), blk = int(blockIdx.x);
