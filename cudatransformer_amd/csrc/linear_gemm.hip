@@ -1548,16 +1548,19 @@ struct Tables16 {
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Forward / dX products whose larger tiles would leave CUs without a workgroup: 32 x 32 tiles.
-// Up to `any_k` of them (fp32 256, one per CU, of 8 waves; 16-bit 384, of 4 waves) at any
-// contraction, up to 768 at a contraction of at most 512, where the shorter chain of each wave
+// Up to `any_k` of them (fp32 256, one per CU, of 8 waves, at any contraction; 16-bit 384, of 4 waves,
+// while tiles x contraction stay at 384 x 1536: past it the operands' second reading costs more than
+// the idle CUs), up to 768 at a contraction of at most 512, where the shorter chain of each wave
 // outweighs the operands read twice as often.  Measured, us, larger tiles -> these:
 //   fp32    256 x 384, K 384   7.1 -> 5.3     512 x 512, K 2048   21.1 -> 13.1
 //           2048 x 384, K 384 (768 tiles, of 4 waves) 10.3 -> 9.1; 1024 x 384, K 1536 (384) 17.6 / 18.7
-//   16-bit  256 x 384, K 384   6.0 -> 3.7     1024 x 384, K 1536   10.1 -> 7.5
-//           2048 x 384, K 384  6.2 -> 5.4     2048 x 512, K 2048 (1024 tiles) 12.1 / 18.0
+//   16-bit  256 x 384, K 384   6.0 -> 3.7     1024 x 384, K 1536 (384) 10.1 -> 7.5
+//           192 x 2048, K 2048 (384) 9.9 / 11.9, dX 10.3 / 14.9; 33 x 5461, K 2048 (342) 10.5 / 11.9;
+//           128 x 1024, K 6144 (128) dX 19.3 / 21.0; 2048 x 384, K 384 (768) 6.2 -> 5.4; 2048 x 512,
+//           K 2048 (1024) 12.1 / 18.0
 bool small_grid(const LinGemm &g, int64_t any_k) {
-    const int64_t t32 = cdiv(g.M, 32) * cdiv(g.N, 32) * g.nbatch;
-    return t32 <= any_k || (t32 <= 768 && g.K * g.nseg <= 512);
+    const int64_t t32 = cdiv(g.M, 32) * cdiv(g.N, 32) * g.nbatch, k = g.K * g.nseg;
+    return (t32 <= any_k && (g.dtype == 0 || t32 * k <= 384 * 1536)) || (t32 <= 768 && k <= 512);
 }
 
 // Chooses a configuration (index into the layout's table) and a K split count.

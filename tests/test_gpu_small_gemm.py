@@ -1,6 +1,7 @@
 """The 32 x 32-tile plans of linear_gemm.hip for small grids, at the edges of their rule: forward,
 forward with its activation and dX against float64 products of the same rounded inputs, with NaN
-around every operand and output.
+around every operand and output; and both sides of the lines between the ragged kernels' tiles and
+between them and the projection family.
 
 Tolerance: sums of K products in fp32, relative to the largest value, 1e-5; 16-bit outputs round
 once, half a unit in the last place of a value up to that largest: 2^-8 bf16, 2^-11 fp16.
@@ -56,3 +57,40 @@ def test_small_grid_linear(name, mnk):
     assert torch.equal(pre, y) and torch.equal(post, y.relu())
     for buf, t in ops + outs:
         assert torch.isnan(buf[:PAD]).all() and torch.isnan(buf[PAD + t.numel():]).all()
+
+
+def close(got, want, name):
+    err = (got.double() - want).abs().max() / want.abs().max()
+    assert err <= TOL[name], float(err)
+
+
+def against_float64(name, m, n, k, grads):
+    """Forward, dX (and with `grads` dW, db) of one linear layer on aligned tensors against float64, and
+    the fused activation's results against the two calls' it stands for, bit for bit."""
+    dt = DT[name]
+    print(f"route {name} {m} {n} {k} grads={grads}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w, dy, b = ((std * torch.randn(shape, generator=g, device="cuda")).to(dt)
+                   for shape, std in (((m, k), 1.0), ((n, k), k ** -0.5), ((m, n), 1.0), ((n,), 0.1)))
+    dw, db = (torch.zeros_like(w), torch.zeros(n, dtype=dt, device="cuda")) if grads else (None, None)
+    y = _capi.linear_fwd(x, w, b)
+    dx = _capi.linear_bwd(x, w, dy, dw, db)
+    pre, h = _capi.linear_act_fwd(x, w, b, _capi.ACT_GELU)
+    dwa, dba = (torch.zeros_like(w), torch.zeros_like(db)) if grads else (None, None)
+    dpre = _capi.linear_act_bwd(x, w, dy, x, _capi.ACT_GELU, dw=dwa, db=dba)
+    torch.cuda.synchronize()
+    x64, w64, dy64 = x.double(), w.double(), dy.double()
+    close(y, x64 @ w64.T + b.double(), name)
+    close(dx, dy64 @ w64, name)
+    if grads:
+        close(dw, dy64.T @ x64, name)
+        close(db, dy64.sum(0), name)
+    assert torch.equal(pre, y) and torch.equal(h, _capi.activation_fwd(y, _capi.ACT_GELU))
+    assert torch.equal(dpre, _capi.activation_bwd(x, dx, _capi.ACT_GELU))
+
+
+# 384 tiles of 32 x 32 at a contraction of 1536 and past it.
+@pytest.mark.parametrize("mnk", [(192, 2048, 1536), (192, 2048, 1568), (192, 1536, 2048)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", ["bf16", "f16"])
+def test_small_grid_contractions(name, mnk):
+    against_float64(name, *mnk, True)
