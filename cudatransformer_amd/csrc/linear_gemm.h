@@ -67,6 +67,11 @@ LinGemm lin_plain(int dtype, bool a_kc, bool b_kc, int64_t M, int64_t N, int64_t
 //     a multiple of 4 (fp32) or 8 (16-bit).
 bool lin_gemm_supported(const LinGemm &g);
 
+// Whether the projection family (proj_launch.h), given that it may use its vector loads, is faster at a
+// product that these kernels take on the ragged path: fp32, a dX of few tiles that runs unsplit in this
+// workspace, or a forward of few rows and a long contraction.
+bool lin_gemm_projection_faster(const LinGemm &g, const void *ws, int64_t ws_bytes);
+
 // Bytes of split-K partials the product's launch plan uses when workspace is allowed (0: the
 // plan does not split K across workgroups, or the shape is not supported).  Depends on the
 // dtype, layout, views and sizes only: the pointers may be null.  _min: of the direct-load

@@ -1413,8 +1413,17 @@ hipError_t run_ragged(const LinGemm &g, int splits, void *ws, int64_t ws_bytes, 
 }
 
 // The ragged plan: 128 x 128 tiles where they, with their K splits, give at least 192 workgroups
-// (three quarters of the CUs), else 64 x 64 tiles; K split (with workspace) up to 512 workgroups,
-// each keeping at least 4 stages.
+// (three quarters of the CUs), in fp32 only where the last round of one workgroup per CU is also at
+// least 7/8 full over all rounds, else 64 x 64 tiles; K split (with workspace) up to 512 workgroups,
+// each keeping at least 4 stages.  Measured, us, 128 / 64 tiles, unsplit (tiles of 128):
+//   fp32 forward  1001 x 1001, K 1001 (64) 89.8 / 37.9; 6000 x 576, K 1000 (235) 90 / 89; 2001 x 2001,
+//                 K 4001 (256) 333 / 336; 4097 x 1025, K 4097 (297) 567 / 444; 8192 x 576, K 1000 (320)
+//                 147 / 114; 3001 x 2001, K 1001 (384) 150 / 134; 8192 x 1000, K 1000 (512) 150 / 173
+//   bf16 forward  1501 x 1501, K 1001 (144) 28.0 / 21.1; 1733 x 1733 (196) 30.1 / 26.6; 4097 x 1025, K
+//                 4097 (297) 98 / 126; 3001 x 2001 (384) 35 / 44; 8192 x 1000 (512) 31 / 39
+//   bf16 dX       3001 x 1001, K 2001 (192) 90 / 48; 4001 x 1001 (256) 43 / 29; 8192 x 1000 (512) 33 / 40
+// and of K splits, 64 x 64 tiles of dW 257 x 257 (25 tiles), K 4001, bf16: 1 / 4 / 8 / 16 / 32 splits 89 /
+// 28.8 / 19.3 / 16.7 / 20.3 us; K 32001: 16 / 32 splits 62 / 44.5.
 struct RaggedPlan {
     bool big;
     int splits;
@@ -1427,8 +1436,9 @@ inline RaggedPlan ragged_plan(const LinGemm &g, bool allow_split) {
         if (!allow_split) return int64_t(1);
         return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(512 / t, stages / 4), 16));
     };
-    const int64_t big = tiles(128), sb = splits(big);
-    if (big * sb >= 192) return RaggedPlan{true, int(sb)};
+    const int64_t big = tiles(128), sb = splits(big), wgs = big * sb;
+    const bool full = g.dtype != 0 || 8 * wgs >= 7 * ((wgs + 255) / 256 * 256);
+    if (wgs >= 192 && full) return RaggedPlan{true, int(sb)};
     return RaggedPlan{false, int(splits(tiles(64)))};
 }
 template <typename F, bool A_KC, bool B_KC>
@@ -1725,12 +1735,31 @@ int64_t lin_gemm_workspace_bytes(const LinGemm &g) {
     return ragged_ok(g) ? lin::splits_bytes(g, lin::ragged_plan(g, true).splits) : 0;
 }
 
+namespace {
+
+// The ragged plan with this workspace.
+lin::RaggedPlan ragged_plan_in(const LinGemm &g, const void *ws, int64_t ws_bytes) {
+    const lin::RaggedPlan pl = lin::ragged_plan(g, true);
+    if (pl.splits == 1 || (ws != nullptr && uintptr_t(ws) % 16 == 0 && ws_bytes >= lin::splits_bytes(g, pl.splits))) return pl;
+    return lin::ragged_plan(g, false);
+}
+
+}  // namespace
+
+// Measured, us, ragged / projection family with vector loads: dX 1000 x 1000, K 1000 (256 tiles of 64 x
+// 64) 46.9 / 40.7, 1200 x 1000 (304) 59.4 / 68.1, 24 x 1000 46.1 / 35.4, 2000 x 260, K 500 25.6 / 23.0, with K
+// split 24 x 1000 13.1; forward 4 x 1000, K 1000 34.5 / 30.6, 28 x 1000 34.4 / 33.8, 64 x 1000 34.7 / 36.6,
+// 16 x 4000, K 200 10.5 / 11.3.
+bool lin_gemm_projection_faster(const LinGemm &g, const void *ws, int64_t ws_bytes) {
+    if (g.dtype != 0 || !g.a_kc || direct_ok(g) || !ragged_ok(g)) return false;
+    if (g.b_kc) return g.M <= 32 && g.K * g.nseg >= 512;
+    return cdiv(g.M, 64) * cdiv(g.N, 64) * g.nbatch <= 256 && ragged_plan_in(g, ws, ws_bytes).splits == 1;
+}
+
 hipError_t launch_lin_gemm(const LinGemm &g, void *ws, int64_t ws_bytes, hipStream_t stream) {
     if (!lin_gemm_supported(g)) return hipErrorInvalidValue;
     if (!direct_ok(g)) {
-        lin::RaggedPlan pl = lin::ragged_plan(g, true);
-        if (pl.splits > 1 && (ws == nullptr || uintptr_t(ws) % 16 != 0 || ws_bytes < lin::splits_bytes(g, pl.splits)))
-            pl = lin::ragged_plan(g, false);
+        const lin::RaggedPlan pl = ragged_plan_in(g, ws, ws_bytes);
         return g.dtype == 0   ? lin::run_ragged_plan<F32Fmt>(g, pl, ws, ws_bytes, stream)
                : g.dtype == 1 ? lin::run_ragged_plan<BF16Fmt>(g, pl, ws, ws_bytes, stream)
                               : lin::run_ragged_plan<F16Fmt>(g, pl, ws, ws_bytes, stream);

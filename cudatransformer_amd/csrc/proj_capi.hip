@@ -151,6 +151,11 @@ ctattn::LinGemm lin_out_dx(int dtype, const ProjShape &s) {
                     ctattn::lin_linear(s.hd()), ctattn::lin_heads(s.T, s.H, s.d), false);
 }
 
+// Whether a product runs on linear_gemm.hip: v4, the projection family may use vector loads.
+bool use_lin(const ctattn::LinGemm &g, bool v4, const void *ws = nullptr, int64_t ws_bytes = 0) {
+    return ctattn::lin_gemm_supported(g) && !(v4 && ctattn::lin_gemm_projection_faster(g, ws, ws_bytes));
+}
+
 // What dX may split K in: the caller's workspace where a weight or bias gradient is asked for too.  A
 // call for dX alone needs none and leaves it alone (another stream may hold it).
 void *dx_workspace(void *workspace, bool with_gradients) { return with_gradients ? workspace : nullptr; }
@@ -188,6 +193,7 @@ int ctattn_qkv_proj_fwd(int dtype, const void *x, const void *wq, const void *wk
         p.batch[z].out = o[z];
         p.batch[z].bias = b[z];
     }
+    const bool v4 = vec4_ok(dtype, s, {x, wq, wk, wv, q, k, v});
     if (lin_policy(dtype)) {
         ctattn::LinGemm g = lin_qkv_fwd(dtype, s);
         for (int z = 0; z < 3; ++z) {
@@ -196,10 +202,9 @@ int ctattn_qkv_proj_fwd(int dtype, const void *x, const void *wq, const void *wk
             g.c[z] = o[z];
             g.bias[z] = b[z];
         }
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, v4))
             return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, as_stream(stream)), as_stream(stream));
     }
-    const bool v4 = vec4_ok(dtype, s, {x, wq, wk, wv, q, k, v});
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 3, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
@@ -271,7 +276,7 @@ int ctattn_qkv_proj_bwd(int dtype, const void *x, const void *dq, const void *dk
             lg.b[0][z] = w[z];
         }
         lg.c[0] = dx;
-        if (ctattn::lin_gemm_supported(lg)) {
+        if (use_lin(lg, v4, dx_ws, workspace_bytes)) {
             e = ctattn::launch_lin_gemm(lg, dx_ws, workspace_bytes, st);
             if (e != hipSuccess) return finish(fn, e, st);
             dx_done = true;
@@ -332,16 +337,16 @@ int ctattn_out_proj_fwd(int dtype, const void *c, const void *wo, const void *bo
     p.batch[0].b[0] = linear_view(wo, s.hd());
     p.batch[0].out = y;
     p.batch[0].bias = bo;
+    const bool v4 = vec4_ok(dtype, s, {c, wo, y});
     if (lin_policy(dtype)) {
         ctattn::LinGemm g = lin_out_fwd(dtype, s);
         g.a[0][0] = c;
         g.b[0][0] = wo;
         g.c[0] = y;
         g.bias[0] = bo;
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, v4))
             return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, as_stream(stream)), as_stream(stream));
     }
-    const bool v4 = vec4_ok(dtype, s, {c, wo, y});
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 1, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
@@ -418,7 +423,7 @@ int ctattn_out_proj_bwd(int dtype, const void *c, const void *dy, const void *wo
         g.a[0][0] = dy;
         g.b[0][0] = wo;
         g.c[0] = dc;
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, v4, dc_ws, workspace_bytes))
             return finish(fn, ctattn::launch_lin_gemm(g, dc_ws, workspace_bytes, st), st);
     }
     if (dc) {
@@ -487,9 +492,10 @@ int ctattn_linear_fwd(int dtype, const void *x, const void *w, const void *b, vo
     if (int rc = validate_linear(fn, dtype, M, N, K)) return rc;
     if (M == 0) return ok();
     if (!x || !w || !y) return fail(hipErrorInvalidValue, "%s: null x/w/y pointer", fn);
+    const bool v4 = linear_vec4(dtype, M, N, K, {x, w, y});
     if (lin_policy(dtype)) {
         const ctattn::LinGemm g = lin_fwd(dtype, x, w, b, y, M, N, K);
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, v4))
             return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, as_stream(stream)), as_stream(stream));
     }
     // y[m][n] = sum_k x[m][k] w[n][k] + b[n]: A = x [M][K], B = w [N][K], both K-contiguous.
@@ -499,7 +505,6 @@ int ctattn_linear_fwd(int dtype, const void *x, const void *w, const void *b, vo
     p.batch[0].b[0] = linear_view(w, K);
     p.batch[0].out = y;
     p.batch[0].bias = b;
-    const bool v4 = linear_vec4(dtype, M, N, K, {x, w, y});
     return finish(fn, ctattn::launch_proj_gemm(dtype, p, 1, true, true, v4, as_stream(stream)), as_stream(stream));
 }
 
@@ -566,7 +571,7 @@ int ctattn_linear_bwd(int dtype, const void *x, const void *w, const void *dy, v
     }
     if (dx && lin_policy(dtype)) {
         const ctattn::LinGemm g = lin_dx(dtype, dy, w, dx, M, N, K);
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, v4, dx_ws, workspace_bytes))
             return finish(fn, ctattn::launch_lin_gemm(g, dx_ws, workspace_bytes, st), st);
     }
     if (dx) {
@@ -594,7 +599,7 @@ int ctattn_linear_act_fwd(int dtype, int act, const void *x, const void *w, cons
         g.act_mode = 1;
         g.act_kind = act;
         g.aux[0] = y;
-        if (ctattn::lin_gemm_supported(g))
+        if (use_lin(g, linear_vec4(dtype, M, N, K, {x, w, pre})))
             return finish(fn, ctattn::launch_lin_gemm(g, nullptr, 0, as_stream(stream)), as_stream(stream));
     }
     if (int rc = ctattn_linear_fwd(dtype, x, w, b, pre, M, N, K, stream)) return rc;
@@ -618,9 +623,9 @@ int ctattn_linear_act_bwd(int dtype, int act, const void *x, const void *w, cons
         g.act_mode = 2;
         g.act_kind = act;
         g.aux[0] = const_cast<void *>(pre);
-        if (ctattn::lin_gemm_supported(g))
-            return finish(fn, ctattn::launch_lin_gemm(g, dx_workspace(workspace, dw || db), workspace_bytes,
-                                                      as_stream(stream)), as_stream(stream));
+        void *const dx_ws = dx_workspace(workspace, dw || db);
+        if (use_lin(g, linear_vec4(dtype, M, N, K, {x, w, dy, dpre, dw}), dx_ws, workspace_bytes))
+            return finish(fn, ctattn::launch_lin_gemm(g, dx_ws, workspace_bytes, as_stream(stream)), as_stream(stream));
     }
     if (int rc = ctattn_linear_bwd(dtype, x, w, dy, dpre, nullptr, nullptr, workspace, workspace_bytes, M, N, K, stream))
         return rc;

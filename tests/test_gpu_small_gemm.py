@@ -89,6 +89,21 @@ def against_float64(name, m, n, k, grads):
     assert torch.equal(dpre, _capi.activation_bwd(x, dx, _capi.ACT_GELU))
 
 
+# fp32 sizes that are multiples of 4 and not of the K chunk: forwards of 32 rows and more (contraction 516 and
+# 508), a dX of 256 tiles of 64 x 64 and of more, contractions of 2 and of more K splits.
+@pytest.mark.parametrize("mnk", [(32, 100, 516), (36, 100, 516), (32, 100, 508), (4, 1000, 1000), (1024, 500, 1000),
+                                 (1028, 500, 1000), (64, 132, 64), (64, 300, 64)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("grads", [False, True], ids=["dx", "all"])
+def test_f32_products_off_the_chunk(mnk, grads):
+    against_float64("f32", *mnk, grads)
+
+
+# 210 and 225 tiles of 128 x 128 (rounds of CUs 82 and 88 % full).
+@pytest.mark.parametrize("mnk", [(1700, 1900, 70), (1900, 1900, 70)], ids=lambda s: "x".join(map(str, s)))
+def test_f32_ragged_tile_choice(mnk):
+    against_float64("f32", *mnk, True)
+
+
 # 384 tiles of 32 x 32 at a contraction of 1536 and past it.
 @pytest.mark.parametrize("mnk", [(192, 2048, 1536), (192, 2048, 1568), (192, 1536, 2048)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("name", ["bf16", "f16"])
