@@ -893,24 +893,30 @@ int ctattn_tensor_matmul(int dtype, const void *a, const void *b, void *c, int64
     // fp32 / bf16 / fp16 on the plain GEMMs of linear_gemm.hip (A [M][K] K-contiguous, B stored
     // [K][N]): one launch when the batches stack (one B), one per three for up to 16 batches.
     const int64_t rows = batch_b == 1 ? batch * M : M;
+    const int64_t es = elem_size(dtype);
+    const bool v4 = rows % 4 == 0 && N % 4 == 0 && K % 4 == 0 &&
+                    uintptr_t(a) % uintptr_t(4 * es) == 0 && uintptr_t(b) % uintptr_t(4 * es) == 0 &&
+                    uintptr_t(c) % uintptr_t(4 * es) == 0;
     if ((dtype == CTATTN_F32 || dtype == CTATTN_BF16 || dtype == CTATTN_F16) &&
         ctattn_get_policy() != CTATTN_POLICY_GENERIC && (batch_b == 1 || batch <= 16)) {
         const int ld = dtype == CTATTN_F32 ? 0 : dtype == CTATTN_BF16 ? 1 : 2;
-        const int64_t es1 = elem_size(dtype);
         const int64_t calls = batch_b == 1 ? 1 : batch;
         auto product = [&](int64_t z0) {  // batches z0 .. of one launch
             ctattn::LinGemm g = ctattn::lin_plain(ld, true, false, rows, N, K, nullptr, K, nullptr, N, nullptr, N,
                                                   nullptr, false);
             g.nbatch = int(std::min<int64_t>(ctattn::kLinMaxBatch, calls - z0));
             for (int j = 0; j < g.nbatch; ++j) {
-                g.a[j][0] = static_cast<const char *>(a) + (z0 + j) * M * K * es1;
-                g.b[j][0] = static_cast<const char *>(b) + (z0 + j) * K * N * es1;
-                g.c[j] = static_cast<char *>(c) + (z0 + j) * M * N * es1;
+                g.a[j][0] = static_cast<const char *>(a) + (z0 + j) * M * K * es;
+                g.b[j][0] = static_cast<const char *>(b) + (z0 + j) * K * N * es;
+                g.c[j] = static_cast<char *>(c) + (z0 + j) * M * N * es;
             }
             return g;
         };
         bool all = true;
-        for (int64_t z = 0; z < calls && all; z += ctattn::kLinMaxBatch) all = ctattn::lin_gemm_supported(product(z));
+        for (int64_t z = 0; z < calls && all; z += ctattn::kLinMaxBatch) {
+            const ctattn::LinGemm g = product(z);
+            all = ctattn::lin_gemm_supported(g) && !(v4 && ctattn::lin_gemm_projection_faster(g, nullptr, 0));
+        }
         for (int64_t z = 0; z < calls && all; z += ctattn::kLinMaxBatch) {
             const hipError_t e = ctattn::launch_lin_gemm(product(z), nullptr, 0, st);
             if (e != hipSuccess) return finish(fn, e, st);
@@ -921,10 +927,6 @@ int ctattn_tensor_matmul(int dtype, const void *a, const void *b, void *c, int64
     // stack into one product of batch * M rows.
     if (rows > 2147483647 || N > 2147483647 || K > 2147483647)
         return fail(hipErrorInvalidValue, "%s: sizes must be below 2^31", fn);
-    const int64_t es = elem_size(dtype);
-    const bool v4 = rows % 4 == 0 && N % 4 == 0 && K % 4 == 0 &&
-                    uintptr_t(a) % uintptr_t(4 * es) == 0 && uintptr_t(b) % uintptr_t(4 * es) == 0 &&
-                    uintptr_t(c) % uintptr_t(4 * es) == 0;
     const int64_t launches = batch_b == 1 ? 1 : batch;
     for (int64_t z0 = 0; z0 < launches; z0 += ctattn::kMaxBatch) {
         ctattn::GemmParams p{};

@@ -571,7 +571,7 @@ CTATTN_API int ctattn_tensor_kron(int dtype, const void *a, const void *b, int n
                                   const int64_t *b_shape, void *out, void *stream);
 
 /* c[z] = a[z] (M x K) times b[z] (K x N), z < batch, with one b for every z when batch_b == 1.
- * Floating types run on the projection GEMMs, integer and bool types on a per-output kernel.
+ * Floating types run on the GEMMs of the linear layers, integer and bool types on a per-output kernel.
  * Replaces Tensor::matmul (Tensor.cu:912-950; matmulKernel). */
 CTATTN_API int ctattn_tensor_matmul(int dtype, const void *a, const void *b, void *c, int64_t batch,
                                     int64_t batch_b, int64_t M, int64_t K, int64_t N, void *stream);

@@ -109,3 +109,20 @@ def test_f32_ragged_tile_choice(mnk):
 @pytest.mark.parametrize("name", ["bf16", "f16"])
 def test_small_grid_contractions(name, mnk):
     against_float64(name, *mnk, True)
+
+
+# Up to and past 256 tiles of 64 x 64, stacked batches and not, the last launch of three with fewer.
+@pytest.mark.parametrize("shape", [(1, 1, 1024, 1000, 1000), (1, 1, 1028, 1000, 1000), (4, 1, 28, 1000, 100),
+                                   (4, 4, 28, 1000, 100), (4, 4, 512, 132, 1024), (2, 2, 1024, 68, 516)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_f32_matmul_off_the_chunk(shape):
+    batch, batch_b, m, k, n = shape
+    print(f"matmul f32 {shape}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn((batch, m, k), generator=g, device="cuda")
+    b = torch.randn((batch_b, k, n), generator=g, device="cuda")
+    c = torch.empty((batch, m, n), device="cuda")
+    assert _capi.load().ctattn_tensor_matmul(0, a.data_ptr(), b.data_ptr(), c.data_ptr(), batch, batch_b, m, k, n,
+                                             torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    close(c, a.double() @ b.double(), "f32")
