@@ -3,8 +3,9 @@
 // in the storage type's accumulation type (fp64 for fp64 storage, the reference's
 // ComputeType; fp32 otherwise), with LSE and delta in that type.
 //
-// These serve head dims and dtypes the MFMA kernels do not cover (fp16, fp64) and are the
-// GPU-side cross-check of those kernels.  The math is the reference's
+// These serve the calls that the MFMA kernels do not take (head dims above 128 that are no multiple
+// of 8 or in fp64, tensors off 16 bytes, the shortest sequences of wide heads) and every call under
+// the GENERIC policy, the GPU-side cross-check of those kernels.  The math is the reference's
 // (flash_attention.cu:97-161 forward online softmax; :269-299 delta, P and dS), with the
 // causal mask, no padded keys, and the correct dK/dV.  Deterministic: no atomics.
 #include "attn_common.h"

@@ -37,7 +37,8 @@
 // 512 registers.  Bound: MFMA issue of one wave per SIMD, which its own exponentials and
 // conversions interrupt; per 32 x 32 tile of the mask the passes execute, for the convention's
 // 2 + 5 units, bf16 4 + 5 + 5 + 4, fp16 3 + 4 + 4 + 3 and fp32 2 + 3 + 3 + 2.  Measured, B2 H8
-// T1024 d256 bf16 unmasked, forward and backward: generic kernels 60 700 us, this 237.
+// T1024 d256 bf16 unmasked, forward and backward: generic kernels 60 700 us, this 237 (forward 49,
+// preprocess 6, dQ 59, dK 66, dV 57; matrix cores busy 15 to 25 % of the launches).
 #include "attn_bf16_tiles.h"
 #include "attn_launch.h"
 
@@ -573,7 +574,8 @@ hipError_t launch_wide(const WideArgs &p, int64_t bh, hipStream_t stream) {
     const int64_t blocks = (int64_t(p.T) + C::OB - 1) / C::OB * bh;
     if (!grid_fits(blocks, 256)) return hipErrorInvalidValue;
     const dim3 grid{unsigned(blocks)}, block{256};
-    // 32-column head-dim tiles: 5 or 6 of them for d = 160 and 192, else all 8.
+    // 32-column head-dim tiles: 5 or 6 of them for d = 160 and 192, else all 8 (136 and 224 too: every
+    // count is another four kernels a type to build).
     if (p.d == 160)
         hipLaunchKernelGGL((wide_attn_kernel<E, 5, MODE, false>), grid, block, 0, stream, p);
     else if (p.d == 192)
@@ -641,8 +643,8 @@ hipError_t wide_bwd(const void *q, const void *k, const void *v, const void *dou
 // Shortest sequences worth a 32 x 32 tile: below them one wave per row (the generic kernels) is
 // faster.  Measured, us, wide / generic, B H T at d = 256 causal: bf16 backward 1 1 1 47.5 / 42.3,
 // 4 8 16 52.6 / 63.1, 32 32 8 188 / 281; fp32 forward 1 1 16 20.3 / 26.5, 32 32 8 85 / 69,
-// backward 1 2 64 142 / 123, 1 4 128 249 / 273 (the fp32 dQ and dK passes at d = 256 spill 200
-// registers: two sets of own rows are 256 of them).
+// backward 1 2 64 142 / 123, 1 4 128 249 / 273 (on eight tiles the fp32 dQ, dK and forward spill 201,
+// 221 and 40 registers: two sets of own rows are 256 of them; fp16 dK spills 26, the other passes none).
 bool wide_supported(int dtype, const AttnShape &s, bool backward) {
     const int64_t min_t = dtype != 0 ? 8 : backward ? 96 : 32;
     return (dtype == 0 || dtype == 1 || dtype == 2) && s.d > 128 && s.d <= 256 && s.d % 8 == 0 && s.T >= min_t &&
