@@ -142,8 +142,17 @@ ctattn::AttnShape padded_shape(const ctattn::AttnShape &s, int64_t dp) {
 // of whole 16-byte chunks.  Then no copies are made (their workspace stays part of what the queries
 // ask for, unused), and d in (64, 96] computes 96 of the 128 columns.  Measured, bf16 B2 H16 T2000
 // d80 causal fwd+bwd: 244 us with the copies (50 us of them) at width 128, 160 us in place.
-bool padded_in_place(int dtype, int64_t d, std::initializer_list<const void *> ps) {
-    return (dtype == CTATTN_BF16 || dtype == CTATTN_F16) && d % 8 == 0 && aligned16(ps);
+// An output on an input's memory keeps the copies, which let the kernels read the inputs as given.
+bool padded_in_place(int dtype, const ctattn::AttnShape &s, std::initializer_list<const void *> in,
+                     std::initializer_list<const void *> out, const void *lse) {
+    if ((dtype != CTATTN_BF16 && dtype != CTATTN_F16) || s.d % 8 != 0 || !aligned16(in) || !aligned16(out) ||
+        !aligned16({lse}))
+        return false;
+    const uintptr_t bytes = uintptr_t(s.rows() * s.d) * 2;
+    for (const void *a : in)
+        for (const void *b : out)
+            if (uintptr_t(a) < uintptr_t(b) + bytes && uintptr_t(b) < uintptr_t(a) + bytes) return false;
+    return true;
 }
 ctattn::AttnShape in_place_shape(const ctattn::AttnShape &s, int64_t dp) {
     ctattn::AttnShape sp = padded_shape(s, dp);
@@ -311,7 +320,7 @@ int ctattn_fwd(int dtype, const void *q, const void *k, const void *v, void *o, 
         return fail(hipErrorInvalidValue, "ctattn_fwd: null q/k/v/o pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (const int64_t dp = padded_width(dtype, d)) {
-        if (padded_in_place(dtype, d, {q, k, v, o, lse}))
+        if (padded_in_place(dtype, s, {q, k, v}, {o}, lse))
             return finish("ctattn_fwd", ctattn::launch_mfma_fwd(dtype, q, k, v, o, static_cast<float *>(lse),
                                                                 in_place_shape(s, dp), st), st);
         return fwd_padded_pool(dtype, dp, q, k, v, o, lse, s, st);
@@ -347,7 +356,7 @@ int ctattn_fwd_ws(int dtype, const void *q, const void *k, const void *v, void *
                     "(ctattn_fwd_workspace_bytes), %lld given",
                     (long long)need, (long long)workspace_bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (padded_in_place(dtype, d, {q, k, v, o, lse}))
+    if (padded_in_place(dtype, s, {q, k, v}, {o}, lse))
         return finish("ctattn_fwd_ws", ctattn::launch_mfma_fwd(dtype, q, k, v, o, static_cast<float *>(lse),
                                                                in_place_shape(s, dp), st), st);
     return finish("ctattn_fwd_ws", fwd_padded_in(dtype, dp, q, k, v, o, lse, s, st, workspace), st);
@@ -406,7 +415,7 @@ int ctattn_bwd(int dtype, const void *q, const void *k, const void *v, const voi
             dtype != CTATTN_F64 ? align_up(ctattn::mfma_bwd_workspace_bytes(dtype, sp, deterministic_policy(), with_ds))
                                 : 0;
         w += extra_bytes;
-        if (padded_in_place(dtype, d, {q, k, v, o, dout, lse, dq, dk, dv})) {
+        if (padded_in_place(dtype, s, {q, k, v, o, dout}, {dq, dk, dv}, lse)) {
             e = ctattn::launch_mfma_bwd(dtype, q, k, v, o, dout, static_cast<const float *>(lse),
                                         static_cast<float *>(delta), dq, dk, dv, extra, extra_bytes,
                                         deterministic_policy(), in_place_shape(s, dp), st);
