@@ -118,6 +118,15 @@ bool deterministic_policy() { return g_policy.load() == CTATTN_POLICY_DETERMINIS
 
 // Bytes of one storage element.
 int64_t elem_bytes(int dtype) { return dtype == CTATTN_F64 ? 8 : dtype == CTATTN_F32 ? 4 : 2; }
+// Whether one of the [B, H, T, d] tensors `out` shares memory with one of `in`.
+bool overlap(int dtype, const ctattn::AttnShape &s, std::initializer_list<const void *> in,
+             std::initializer_list<const void *> out) {
+    const uintptr_t bytes = uintptr_t(s.rows() * s.d * elem_bytes(dtype));
+    for (const void *a : in)
+        for (const void *b : out)
+            if (uintptr_t(a) < uintptr_t(b) + bytes && uintptr_t(b) < uintptr_t(a) + bytes) return true;
+    return false;
+}
 
 // Head dims up to 128 without an MFMA kernel of their own (not 32, 64 or 128) run the MFMA
 // kernels of the next width on zero-padded copies of the tensors (attn_pad.hip), with the
@@ -148,11 +157,7 @@ bool padded_in_place(int dtype, const ctattn::AttnShape &s, std::initializer_lis
     if ((dtype != CTATTN_BF16 && dtype != CTATTN_F16) || s.d % 8 != 0 || !aligned16(in) || !aligned16(out) ||
         !aligned16({lse}))
         return false;
-    const uintptr_t bytes = uintptr_t(s.rows() * s.d) * 2;
-    for (const void *a : in)
-        for (const void *b : out)
-            if (uintptr_t(a) < uintptr_t(b) + bytes && uintptr_t(b) < uintptr_t(a) + bytes) return false;
-    return true;
+    return !overlap(dtype, s, in, out);
 }
 ctattn::AttnShape in_place_shape(const ctattn::AttnShape &s, int64_t dp) {
     ctattn::AttnShape sp = padded_shape(s, dp);
@@ -443,7 +448,8 @@ int ctattn_bwd(int dtype, const void *q, const void *k, const void *v, const voi
                                     deterministic_policy(), s, st);
     } else if (use_f64_mfma(dtype, d) && al) {
         e = ctattn::launch_f64_bwd(q, k, v, o, dout, lse, workspace, dq, dk, dv, s, st);
-    } else if (use_wide(dtype, s, true) && al) {
+    } else if (use_wide(dtype, s, true) && al && !overlap(dtype, s, {q, k, v, dout}, {dq, dk, dv})) {
+        // (dK and dV are passes of their own, and each reads K; the generic kernel writes both from one read.)
         e = ctattn::launch_wide_bwd(dtype, q, k, v, o, dout, static_cast<const float *>(lse),
                                     static_cast<float *>(workspace), dq, dk, dv, s, st);
     } else {

@@ -209,3 +209,20 @@ def test_wide_gradients_grow_along_the_sequence(name, causal):
     x[2] = (x[2].float() * torch.logspace(-8, 4, 333, 2.0, device="cuda")[:, None]).to(DT[name])
     x[3] = (x[3].float() * torch.logspace(-12, 2, 333, 2.0, device="cuda")[:, None]).to(DT[name])
     check64(x, causal, name)
+
+
+@pytest.mark.parametrize("name", sorted(DT))
+def test_wide_gradients_on_their_inputs(name):
+    """dK and dV written onto K and V: the generic kernels' results, which such calls run on."""
+    print(f"wide heads gradients on inputs {name}", flush=True)
+    q, k, v, do = inputs((2, 2, 150, 160), name, seed=23)
+    o, lse = ct.flash_attn_fwd(q, k, v, True)
+    prev = ct.set_policy(ct.POLICY_GENERIC)
+    try:
+        want = ct.flash_attn_bwd(q, k, v, o, do, lse, True)
+    finally:
+        ct.set_policy(prev)
+    k2, v2 = k.clone(), v.clone()
+    got = ct.flash_attn_bwd(q, k2, v2, o, do, lse, True, dk=k2, dv=v2)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
