@@ -938,10 +938,15 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
         // (65536 x 128: bf16 20.5 in registers / 18.9, fp16 25.5 / 20.3).
         bool one_pass = false;
         const bool wave_dx = std::is_same_v<T, double> || D > 8192 || (sizeof(T) == 2 && D <= 128 && N > 8192);
+        if constexpr (!std::is_same_v<T, double>)
+            one_pass = D > 1024 ? D <= 8192 && N * int64_t(sizeof(T)) > 8192
+                                : sizeof(T) == 4 || N <= 8192 || 8 * D >= 7 * (D <= 512 ? 512 : 1024);
+        // Before dx, which may lie on x or dy.
+        if ((dgamma || dbeta) && !one_pass)
+            hipLaunchKernelGGL(ctattn::layernorm_bwd_part_kernel<T>, dim3(unsigned((D + 63) / 64), unsigned(chunks)),
+                               dim3(256), 0, st, xt, dyt, mu, rs, part, N, int(D));
         if constexpr (!std::is_same_v<T, double>) {
             constexpr int CU = sizeof(T) == 4 ? 2 : 1;  // granules per 8 elements
-            one_pass = D > 1024 ? D <= 8192 && N * int64_t(sizeof(T)) > 8192
-                                : CU == 2 || N <= 8192 || 8 * D >= 7 * (D <= 512 ? 512 : 1024);
             auto rows = [&](auto gw, auto cpt) {
                 constexpr int GW = decltype(gw)::value, CPT = decltype(cpt)::value;
                 auto launch = [&](auto kernel, int64_t wgs) {
@@ -963,9 +968,6 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
             hipLaunchKernelGGL(ctattn::layernorm_bwd_dx_kernel<T>, dim3(ctattn::rows_grid(N)), dim3(256), 0, st, xt,
                                static_cast<const T *>(gamma), dyt, mu, rs, static_cast<T *>(dx), N, int(D));
         if (dgamma || dbeta) {
-            if (!one_pass)
-                hipLaunchKernelGGL(ctattn::layernorm_bwd_part_kernel<T>, dim3(unsigned((D + 63) / 64), unsigned(chunks)),
-                                   dim3(256), 0, st, xt, dyt, mu, rs, part, N, int(D));
             const int64_t groups = std::min<int64_t>((2 * D + 31) / 32, 65536);  // of columns; the kernel loops
             hipLaunchKernelGGL(ctattn::layernorm_bwd_reduce_kernel<T>, dim3(unsigned(groups)), dim3(1024), 0, st,
                                static_cast<const A *>(part), static_cast<T *>(dgamma), static_cast<T *>(dbeta),

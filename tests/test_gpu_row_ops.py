@@ -147,7 +147,7 @@ def test_softmax_exponential_ulps():
 @pytest.mark.parametrize("name", sorted(DT))
 def test_layernorm_bwd_one_pass_or_two(name, nd):
     """Both sides of the lines in N and D between dx with the partial sums in one pass and dx by itself,
-    against float64, and each output alone: the same bits."""
+    against float64; each output alone and dx written onto dy: the same bits."""
     n, d = nd
     dt, code, lib = DT[name], _capi._DTYPE_CODE[DT[name]], _capi.load()
     print(f"layernorm backward {name} {n} x {d}", flush=True)
@@ -169,6 +169,12 @@ def test_layernorm_bwd_one_pass_or_two(name, nd):
     dx, dg, db = bwd(True, True)
     assert torch.equal(bwd(True, False)[0], dx)
     assert all(torch.equal(a, b) for a, b in zip(bwd(False, True)[1:], (dg, db)))
+    dy2, dg2, db2 = dy.clone(), torch.zeros_like(g), torch.zeros_like(g)  # dx onto dy
+    assert lib.ctattn_layernorm_bwd(code, x.data_ptr(), g.data_ptr(), dy2.data_ptr(), mean.data_ptr(), rstd.data_ptr(),
+                                    dy2.data_ptr(), dg2.data_ptr(), db2.data_ptr(), ws.data_ptr(), ws.numel(), n, d,
+                                    None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(dy2, dx) and torch.equal(dg2, dg) and torch.equal(db2, db)
     x64, dy64, mu, rs = x.double(), dy.double(), mean.double()[:, None], rstd.double()[:, None]
     xh, dxh = (x64 - mu) * rs, dy64 * g.double()
     close(dx, rs * (dxh - dxh.mean(-1, keepdim=True) - xh * (dxh * xh).mean(-1, keepdim=True)), TOL[name], "dx")
