@@ -196,22 +196,24 @@ __global__ __launch_bounds__(256) void layernorm_bwd_part_kernel(const T *__rest
 //   PART   dx (may be null) and the stage-1 gamma / beta partial sums of one 32-row chunk in one pass
 //          over x and dy: group k takes rows k, k + 8 / GW, ..., with the columns' sums in registers and
 //          the groups' sums added in LDS in group order.  Bound by HBM at many chunks; bf16 8192 x 2048
-//          (dx 30 + partial sums 17 us as two kernels) -> 26 us.  A workgroup per 32 rows, one of them
-//          on a CU (154 to 256 registers), leaves the chip idle at few chunks.
-//   !PART  dx alone, RB rows a group: 57 to 114 registers, 2 to 4 workgroups on a CU.  The same
+//          (dx 30 + partial sums 17 us as two kernels) -> 26 us.  A workgroup per 32 rows; rows of one
+//          wave take 103 to 113 registers, two workgroups on a CU (past 128 bf16 65536 x 256 took 56 us
+//          for 37, so fp32 takes 2 rows at a time there), the others 169 to 220, one, which leaves the
+//          chip idle at few chunks.
+//   !PART  dx alone, RB rows a group: 39 to 120 registers, 2 to 4 workgroups on a CU.  The same
 //          arithmetic, so the same dx.  Against one wave per row (layernorm_bwd_dx_kernel), us: bf16
-//          256 x 3072 12.5 -> 5.1, 8192 x 2048 24.1 -> 12.7, 65536 x 384 37.8 -> 23.6; fp32 256 x 3072
-//          14.6 -> 5.0, 65536 x 128 20.3 -> 17.4; PART's kernel for dx alone took 27.8, 17.0, 39.8,
-//          35.4 and 43.6.
+//          256 x 3072 13 -> 5, 8192 x 2048 27 -> 17, 65536 x 384 38 -> 28; fp32 256 x 3072 14 -> 4,
+//          65536 x 384 71 -> 52.
 template <typename T, int GW, int CPT, bool PART>
 __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__restrict__ x, const T *__restrict__ g,
                                                                 const T *__restrict__ dy,
                                                                 const float *__restrict__ mean,
                                                                 const float *__restrict__ rstd, T *__restrict__ dx,
                                                                 float *__restrict__ part, int64_t N, int D) {
+#pragma clang fp contract(off)  // written out: PART and !PART have to round alike
     using G = Gran<T>;
     constexpr int EPT = CPT * G::EPC;
-    constexpr int NG = 8 / GW, RB = !PART ? 2 : EPT > 8 ? 2 : 4;
+    constexpr int NG = 8 / GW, RB = !PART || EPT > 8 || (GW == 1 && CPT > 1) ? 2 : 4;
     constexpr int RPG = PART ? kLnRowsPerChunk / NG : RB;  // rows per group
     constexpr int COLS = PART ? kWave * GW * EPT : 1;  // >= D
     __shared__ float xch[2][8][RB][2];                 // row sums of each wave, by batch parity
@@ -255,24 +257,41 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
             for (int j = 0; j < CPT; ++j)
 #pragma unroll
                 for (int e = 0; e < G::EPC; ++e) {
-                    // Past D (0 - mean) rstd may overflow, and 0 times an infinity would reach the sums.
-                    const bool in = (lane + kWave * GW * j) * G::EPC + e < D;
-                    const float d = G::get(dv[i][j], e), xh = in ? (G::get(xv[i][j], e) - mu[i]) * rs[i] : 0.f;
+                    const float d = G::get(dv[i][j], e), xh = (G::get(xv[i][j], e) - mu[i]) * rs[i];
                     if constexpr (PART) {
-                        sg[j * G::EPC + e] += d * xh;
+                        sg[j * G::EPC + e] = fmaf(d, xh, sg[j * G::EPC + e]);
                         sb[j * G::EPC + e] += d;
                     }
                     const float dxh = d * G::get(gv[j], e);
                     s1[i] += dxh;
-                    s2[i] += dxh * xh;
+                    s2[i] = fmaf(dxh, xh, s2[i]);
                 }
         }
         if (dx == nullptr) continue;
+        if constexpr (GW == 1) {  // x^ again below: kept, it takes the second workgroup's registers
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CPT; ++j) asm("" : "+v"(xv[i][j]));
+        }
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             s1[i] = wave_sum_dpp(s1[i]);
             s2[i] = wave_sum_dpp(s2[i]);
         }
+        // Past D x and dy are 0, but (0 - mean) rstd may overflow, and 0 times an infinity made s2 NaN: again
+        // from memory, so that it holds no registers (a mask per element above took 30 %: bf16 65536 x 384
+        // 42 -> 55 us).  Uniform over the wave, and before this row's dx, which may lie on x or dy.
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+            if (__builtin_expect(s2[i] != s2[i], 0)) {
+                const int64_t r = r0 + grp + NG * (i0 + i);
+                float s = 0.f;
+#pragma unroll 1
+                for (int c = lane; c < D; c += kWave * GW)
+                    s = fmaf(to_f32(dy[r * D + c]) * to_f32(g[c]), (to_f32(x[r * D + c]) - mu[i]) * rs[i], s);
+                s2[i] = wave_sum_dpp(s);
+            }
         if constexpr (GW > 1) {
             float (*xb)[RB][2] = xch[(i0 / RB) & 1];
             if (threadIdx.x % kWave == 0) {
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(512) void layernorm_bwd_rows_kernel(const T *__rest
 #pragma unroll
                 for (int e = 0; e < G::EPC; ++e) {
                     const float xh = (G::get(xv[i][j], e) - mu[i]) * rs[i];
-                    o[e] = rs[i] * (G::get(dv[i][j], e) * G::get(gv[j], e) - m1 - xh * m2);
+                    o[e] = rs[i] * fmaf(-xh, m2, fmaf(G::get(dv[i][j], e), G::get(gv[j], e), -m1));
                 }
                 G::store(dx + r * D, (lane + kWave * GW * j) * G::EPC, D, o);
             }
@@ -929,18 +948,16 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
         // Rows in registers: dx and the partial sums in one pass, or dx by itself and the partial sums
         // from their own kernel.  The line depends on N and D alone, so an output has the same bits
         // whichever others are asked for.  Measured, us, one pass / two kernels, both outputs:
-        //   D > 1024    few chunks leave CUs idle: bf16 256 x 3072 31.3 / 11.5, 4096 x 3072 33.9 / 28.5,
-        //               4096 x 2048 19.2 / 19.5, 8192 x 2048 21.7 / 31.5; fp32 256 x 8192 55.9 / 14.4,
-        //               2048 x 2048 19.0 / 16.6, 4096 x 2048 21.1 / 26.7
-        //   D <= 1024   one pass; in 16 bits not for many rows that leave lanes idle: 65536 x 128 51.1 /
-        //               36.2, 65536 x 768 96.8 / 91.3, 8192 x 768 15.2 / 18.4, 65536 x 512 40.8 / 57.0
+        //   D > 1024    few chunks leave CUs idle: bf16 256 x 3072 34 / 11, 4096 x 3072 37 / 31,
+        //               4096 x 2048 21 / 22, 8192 x 2048 26 / 36; fp32 256 x 8192 48 / 16,
+        //               2048 x 2048 21 / 20, 4096 x 2048 26 / 33
+        //   D <= 1024   bf16 256 x 384 10 / 11, 2048 x 768 14 / 11, 8192 x 768 18 / 20, 65536 x 384 40 / 58,
+        //               65536 x 768 138 / 118, 65536 x 1024 103 / 166; fp32 256 x 768 12 / 11,
+        //               65536 x 128 36 / 38, 65536 x 768 148 / 232
         // dx by itself: one wave per row past D 8192, in fp64 and for many 16-bit rows of at most 16 granules
-        // (65536 x 128: bf16 20.5 in registers / 18.9, fp16 25.5 / 20.3).
-        bool one_pass = false;
-        const bool wave_dx = std::is_same_v<T, double> || D > 8192 || (sizeof(T) == 2 && D <= 128 && N > 8192);
-        if constexpr (!std::is_same_v<T, double>)
-            one_pass = D > 1024 ? D <= 8192 && N * int64_t(sizeof(T)) > 8192
-                                : sizeof(T) == 4 || N <= 8192 || 8 * D >= 7 * (D <= 512 ? 512 : 1024);
+        // (bf16 65536 x 128 21 in registers / 19; both outputs 36 in one pass, 34 as two kernels).
+        const bool wave_dx = std::is_same_v<T, double> || D > 8192 || (sizeof(T) == 2 && D <= 128 && N > 16384);
+        const bool one_pass = !wave_dx && (D <= 1024 || N * int64_t(sizeof(T)) > 8192);
         // Before dx, which may lie on x or dy.
         if ((dgamma || dbeta) && !one_pass)
             hipLaunchKernelGGL(ctattn::layernorm_bwd_part_kernel<T>, dim3(unsigned((D + 63) / 64), unsigned(chunks)),

@@ -81,6 +81,36 @@ def test_layernorm_bwd_large_constant_rows(d):
         close(dx, rstd.double()[:, None] * (dxh - dxh.mean(-1, keepdim=True)), TOL[name], "dx")
 
 
+@pytest.mark.parametrize("nd", [(5, 65), (37, 300), (5, 600), (2100, 1100), (4100, 1100), (4100, 3000), (4100, 5000)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("name", ["f32", "bf16"])
+def test_layernorm_bwd_given_large_statistics(name, nd):
+    """The same with given statistics, for rows of one and of several waves, dx with the partial sums and by
+    itself, and written onto x; a NaN in a row stays in that row's dx."""
+    n, d = nd
+    dt = DT[name]
+    print(f"layernorm given statistics {name} {n} x {d}", flush=True)
+    x = torch.full((n, d), 2.0 ** 120, device="cuda").to(dt)
+    g, dy = rnd((d,), dt, 3, 0.1, 1.0), rnd((n, d), dt, 2)
+    dy[1, d - 1] = float("nan")
+    mean, rstd = torch.full((n,), 2.0 ** 120, device="cuda"), torch.full((n,), 2.0 ** 9, device="cuda")
+    dg, db = torch.zeros_like(g), torch.zeros_like(g)
+    dx = _capi.layernorm_bwd(x, g, dy, mean, rstd, dg, db)
+    alone = _capi.layernorm_bwd(x, g, dy, mean, rstd)
+    torch.cuda.synchronize()
+    ok = [i for i in range(n) if i != 1]
+    assert bool(dx[1].isnan().all()) and torch.equal(alone[ok], dx[ok])
+    dxh = dy.double() * g.double()
+    close(dx[ok], (2.0 ** 9 * (dxh - dxh.mean(-1, keepdim=True)))[ok], TOL[name], "dx")
+    assert bool((dg[:-1] == 0).all()) and bool(dg[-1].isnan()) and bool(db[-1].isnan())
+    close(db[:-1], dy.double().sum(0)[:-1], TOL[name], "dbeta")
+    code, lib = _capi._DTYPE_CODE[dt], _capi.load()
+    assert lib.ctattn_layernorm_bwd(code, x.data_ptr(), g.data_ptr(), dy.data_ptr(), mean.data_ptr(), rstd.data_ptr(),
+                                    x.data_ptr(), None, None, None, 0, n, d, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(x[ok], dx[ok])
+
+
 @pytest.mark.parametrize("v", [1, 3, 65, 256, 257, 512, 1025, 2048, 4097, 8193, 16385, 32769, 65536, 65537])
 @pytest.mark.parametrize("name", sorted(DT))
 def test_softmax_and_gradient_edges(name, v):
@@ -141,7 +171,8 @@ def test_softmax_exponential_ulps():
     assert bool((p[x < -104] == 0).all())  # e^x below half of 2^-149
 
 
-@pytest.mark.parametrize("nd", [(8192, 65), (8193, 65), (8193, 250), (8193, 384), (8193, 448), (8193, 513), (8193, 896),
+@pytest.mark.parametrize("nd", [(8192, 65), (8193, 65), (16384, 128), (16385, 128), (16385, 129),
+                                (8193, 250), (8193, 384), (8193, 448), (8193, 513), (8193, 896),
                                 (2048, 1032), (2049, 1032), (4096, 1032), (4097, 1032), (4096, 2052), (4097, 2052),
                                 (2049, 4100), (4097, 4100)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("name", sorted(DT))
