@@ -952,8 +952,8 @@ int ctattn_layernorm_bwd(int dtype, const void *x, const void *gamma, const void
         //               4096 x 2048 21 / 22, 8192 x 2048 26 / 36; fp32 256 x 8192 48 / 16,
         //               2048 x 2048 21 / 20, 4096 x 2048 26 / 33
         //   D <= 1024   bf16 256 x 384 10 / 11, 2048 x 768 14 / 11, 8192 x 768 18 / 20, 65536 x 384 40 / 58,
-        //               65536 x 768 138 / 118, 65536 x 1024 103 / 166; fp32 256 x 768 12 / 11,
-        //               65536 x 128 36 / 38, 65536 x 768 148 / 232
+        //               65536 x 768 138 / 118 (131072 rows 275 / 271, 32768 57 / 57), 65536 x 1024 103 / 166;
+        //               fp32 256 x 768 12 / 11, 65536 x 128 36 / 38, 65536 x 768 148 / 232
         // dx by itself: one wave per row past D 8192, in fp64 and for many 16-bit rows of at most 16 granules
         // (bf16 65536 x 128 21 in registers / 19; both outputs 36 in one pass, 34 as two kernels).
         const bool wave_dx = std::is_same_v<T, double> || D > 8192 || (sizeof(T) == 2 && D <= 128 && N > 16384);
